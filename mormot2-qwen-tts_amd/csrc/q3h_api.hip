@@ -609,6 +609,14 @@ void upload_rows(Mat &m, int dtype, const void *src, int src_dtype, int rows, in
   check_hip(hipStreamSynchronize(st), "upload sync");
 }
 
+// m's quants rewritten in the operand order of the int8 products (act_q8
+// stacks), through tmp (N * K bytes)
+void tile_mat(Mat &m, void *tmp, hipStream_t st) {
+  check_hip(hipMemcpyAsync(tmp, m.q, (size_t)m.N * m.K, hipMemcpyDeviceToDevice, st), "tile");
+  launch_tile_q8((const int8_t *)tmp, m.N, m.K, m.q, st);
+  check_hip(hipGetLastError(), "tile kernel");
+}
+
 float *upload_vec(const float *src, int n, const char *what) {
   require(src != nullptr, Q3H_E_ARG, std::string("a norm vector is NULL: ") + what);
   float *d = (float *)dev_alloc(sizeof(float) * n);
@@ -688,7 +696,11 @@ extern "C" int q3h_stack_create(q3h_device *dev, const q3h_stack_config *cfg,
     const int H = c.hidden, hd = c.head_dim, NQ = c.heads * hd, NKV = c.kv_heads * hd;
     const int I = c.intermediate;
     const int maxK = std::max(std::max(H, NQ), I), maxN = std::max(std::max(NQ, I), H);
-    void *staging = dev_alloc(src_row_bytes(w->src_dtype, maxK) * maxN);
+    // (an act_q8 stack also passes each matrix through it: tile_mat)
+    const size_t tile_bytes =
+        c.act_q8 ? std::max((size_t)(NQ + 2 * NKV) * H, std::max((size_t)2 * I * H, (size_t)H * NQ))
+                 : 0;
+    void *staging = dev_alloc(std::max(src_row_bytes(w->src_dtype, maxK) * maxN, tile_bytes));
     try {
       s->layers.resize(c.layers);
       for (int l = 0; l < c.layers; l++) {
@@ -706,6 +718,8 @@ extern "C" int q3h_stack_create(q3h_device *dev, const q3h_stack_config *cfg,
         upload_rows(L.gu, c.dtype, lw.wgate, w->src_dtype, I, H, 2, 0, staging, s->stream);
         upload_rows(L.gu, c.dtype, lw.wup, w->src_dtype, I, H, 2, 1, staging, s->stream);
         upload_rows(L.down, c.dtype, lw.wdown, w->src_dtype, H, I, 1, 0, staging, s->stream);
+        if (c.act_q8)
+          for (Mat *m : {&L.qkv, &L.o, &L.gu, &L.down}) tile_mat(*m, staging, s->stream);
         if (c.dtype == Q3H_F32 && c.max_positions > 64)
           for (Mat *m : {&L.qkv, &L.o, &L.gu, &L.down}) make_x3(*m, s->aux_bytes, s->stream);
         L.in_norm = upload_vec(lw.input_norm, H, "input_layernorm");
@@ -745,6 +759,7 @@ extern "C" int q3h_stack_create(q3h_device *dev, const q3h_stack_config *cfg,
       check_hip(hipMemcpy(s->rope_cs, cs.data(), sizeof(float) * cs.size(),
                           hipMemcpyHostToDevice),
                 "upload rope");
+      if (c.act_q8) check_hip(hipStreamSynchronize(s->stream), "tile sync");
     } catch (...) {
       dev_free(staging);
       throw;
@@ -776,9 +791,13 @@ extern "C" int q3h_stack_add_head(q3h_stack *s, const void *w, int rows, int src
     const int H = s->cfg.hidden;
     int64_t bytes = 0;
     Mat m = alloc_mat(rows, H, s->cfg.dtype, bytes);
-    void *staging = dev_alloc(src_row_bytes(src_dtype, H) * rows);
+    void *staging = dev_alloc(std::max(src_row_bytes(src_dtype, H), (size_t)H) * rows);
     try {
       upload_rows(m, s->cfg.dtype, w, src_dtype, rows, H, 1, 0, staging, s->stream);
+      if (s->cfg.act_q8) {
+        tile_mat(m, staging, s->stream);
+        check_hip(hipStreamSynchronize(s->stream), "tile sync");
+      }
     } catch (...) {
       dev_free(staging);
       free_mat(m);

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(NT) void k_attn_x(const RowDesc *rd, const float *q
     for (int i = t; i < GRP * HD; i += NT) {
       const int h = g * GRP + i / HD, k = i % HD;
       xq[qoff(h, k)] = 0;
-      if ((k & 31) == 0) dx[(size_t)m * nbq + 4 * h + (k >> 5)] = 0.f;
+      if ((k & 31) == 0) dx[qscale_offset(m, 4 * h + (k >> 5), nbq)] = 0.f;
     }
     return;
   }
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(NT) void k_attn_x(const RowDesc *rd, const float *q
     const float dq = __fdiv_rn(amax, 127.0f);
     const float id = dq != 0.f ? __fdiv_rn(1.0f, dq) : 0.f;
     xq[qoff(h, k)] = (int8_t)(int)roundf(__fmul_rn(o, id));
-    if ((k & 31) == 0) dx[(size_t)m * nbq + 4 * h + (k >> 5)] = (float)(_Float16)dq;
+    if ((k & 31) == 0) dx[qscale_offset(m, 4 * h + (k >> 5), nbq)] = (float)(_Float16)dq;
   }
 }
 

@@ -14,13 +14,16 @@
 // Operand layouts (v_mfma_i32_16x16x32_i8, wave64): lane l holds 8 int8 of
 // row l % 16 of A and of column l % 16 of B, k = 8 * (l / 16) .. + 7; the
 // result C[4 * (l / 16) + r][l % 16], r < 4, lands in lane l. A is 16 weight
-// rows of the row-major Q8_0 matrix; B is 16 activation rows, which the
-// quantizers write already in operand order (qtile_offset), so one coalesced
-// 1 KB load gives the B operands of two blocks.
+// rows, B 16 activation rows, both stored in operand order (wtile_offset: the
+// matrices of an act_q8 stack are rewritten so at load; qtile_offset: written
+// so by the quantizers), so one coalesced 1 KB load gives the operands of two
+// blocks.
 //
-// Two schedules of the same chains:
+// Three schedules of the same chains:
 //  - k_gemm_i8: a workgroup per 16 weight rows, its waves taking the chunks
 //    and adding them through LDS; any number of rows (prefill);
+//  - k_gemm_i8r: a wave per 64 weight rows and activation tile over the whole
+//    K, where these fill the chip (long or several prompts);
 //  - k_gemm_i8p (up to 64 rows, the batched decode step): one wave per (16
 //    weight rows, chunk) over the whole chip, the chunk sums written out as
 //    partials that the consumer adds in chunk order (k_quant_act with a
@@ -41,6 +44,11 @@ constexpr int kMaxChunks = 6;     // chunks of a product: K <= 3072
 
 __device__ __forceinline__ float *scales_of(int8_t *xq, int M, int K) {
   return reinterpret_cast<float *>(xq + (size_t)((M + 15) & ~15) * K);
+}
+
+// block h (0, 1) of a lane's 16 operand bytes of a pair of blocks
+__device__ __forceinline__ long half_pair(const int4 &v, int h) {
+  return h ? ((long)(unsigned)v.w << 32) | (unsigned)v.z : ((long)(unsigned)v.y << 32) | (unsigned)v.x;
 }
 
 // The quantizer. One workgroup per activation row m < Mp and slice of its
@@ -80,7 +88,7 @@ __global__ __launch_bounds__(kQuantThreads) void k_quant_act(float *x, const flo
     if (xq)
       for (int j = j0; j < nch; j += js) {
         *reinterpret_cast<long *>(xq + qtile_offset(m, 8 * j, mt16)) = 0;
-        if ((j & 3) == 0) dx[(size_t)m * nb + (j >> 2)] = 0.f;
+        if ((j & 3) == 0) dx[qscale_offset(m, j >> 2, nb)] = 0.f;
       }
     return;
   }
@@ -220,7 +228,7 @@ __global__ __launch_bounds__(kQuantThreads) void k_quant_act(float *x, const flo
       packed |= (unsigned long long)(uint8_t)(int8_t)q << (8 * e);
     }
     *reinterpret_cast<long *>(xq + qtile_offset(m, 8 * j, mt16)) = (long)packed;
-    if ((j & 3) == 0) dx[(size_t)m * nb + (j >> 2)] = (float)(_Float16)d;
+    if ((j & 3) == 0) dx[qscale_offset(m, j >> 2, nb)] = (float)(_Float16)d;
   }
 }
 
@@ -251,40 +259,31 @@ __device__ __forceinline__ void chains(const long (&av)[NB], const long (&bv)[TM
 // acc[t][r] = output (n0 + 4 (lane / 16) + r, 16 (mt0 + t) + lane % 16); a
 // tile past the last (mt16) repeats the last one and its outputs are not
 // stored. All loads are unconditional and issued before the first MFMA (a
-// guarded load would make the compiler wait for each one). LDSA: the weight
-// tile is read with 16-byte loads (4 rows x 256 bytes per instruction instead
-// of 16 rows x 32 bytes) and rearranged through the wave's own 16 x (4 NB + 1)
-// longs of LDS (at).
-template <int TM, bool LDSA, int NB>
+// guarded load would make the compiler wait for each one).
+template <int TM, int NB>
 __device__ __forceinline__ void chunk_chains(const int8_t *wq, const int8_t *xq, const float *dx,
                                              int N, int K, int n0, int mt0, int mt16, int b0,
-                                             long (*at)[4 * NB + 1], float (&acc)[TM][4]) {
+                                             float (&acc)[TM][4]) {
   static_assert(NB % 8 == 0, "whole 8-block groups");
-  constexpr int NH = NB / 8;  // 256-byte pieces of a weight row
+  constexpr int NH = NB / 8;  // 8-block groups of the weight scales
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int nb = K >> 5;
   const _Float16 *wd = reinterpret_cast<const _Float16 *>(wq + (size_t)N * K);
   const int4 *xq16 = reinterpret_cast<const int4 *>(xq);
+  const int4 *wq16 = reinterpret_cast<const int4 *>(wq) + (size_t)(n0 >> 4) * K + lane;
   long av[NB], bv[TM][NB];
   float dwv[4][NB], dxv[TM][NB];
-  int4 araw[4 * NH];
-  if (LDSA) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)  // rows 4i + lane / 16, bytes 256 h + 16 (lane % 16) of the chunk
-#pragma unroll
-      for (int h = 0; h < NH; h++)
-        araw[i * NH + h] = *reinterpret_cast<const int4 *>(
-            wq + (size_t)(n0 + 4 * i + (lane >> 4)) * K + b0 * 32 + 256 * h + 16 * (lane & 15));
-  } else {
-    const int8_t *wr = wq + (size_t)(n0 + c) * K + 8 * g;
-#pragma unroll
-    for (int i = 0; i < NB; i++) av[i] = *reinterpret_cast<const long *>(wr + 32 * (b0 + i));
+  for (int q = 0; q < NB / 2; q++) {  // blocks b0 + 2q, b0 + 2q + 1
+    const int4 v = wq16[((b0 >> 1) + q) * 64];
+    av[2 * q] = ((long)(unsigned)v.y << 32) | (unsigned)v.x;
+    av[2 * q + 1] = ((long)(unsigned)v.w << 32) | (unsigned)v.z;
   }
 #pragma unroll
   for (int t = 0; t < TM; t++) {
     const int tt = min(mt0 + t, mt16 - 1);
 #pragma unroll
-    for (int q = 0; q < NB / 2; q++) {  // blocks b0 + 2q, b0 + 2q + 1
+    for (int q = 0; q < NB / 2; q++) {
       const int4 v = xq16[((size_t)((b0 >> 1) + q) * mt16 + tt) * 64 + lane];
       bv[t][2 * q] = ((long)(unsigned)v.y << 32) | (unsigned)v.x;
       bv[t][2 * q + 1] = ((long)(unsigned)v.w << 32) | (unsigned)v.z;
@@ -306,26 +305,12 @@ __device__ __forceinline__ void chunk_chains(const int8_t *wq, const int8_t *xq,
 #pragma unroll
   for (int t = 0; t < TM; t++) {
     const int tt = min(mt0 + t, mt16 - 1);
-    const float4 *dp = reinterpret_cast<const float4 *>(dx + (size_t)(tt * 16 + c) * nb + b0);
+    const float4 *dp = reinterpret_cast<const float4 *>(dx + qscale_offset(tt * 16 + c, b0, nb));
 #pragma unroll
     for (int q = 0; q < NB / 4; q++) {
-      const float4 p = dp[q];
+      const float4 p = dp[16 * q];
       dxv[t][4 * q] = p.x, dxv[t][4 * q + 1] = p.y, dxv[t][4 * q + 2] = p.z, dxv[t][4 * q + 3] = p.w;
     }
-  }
-  if (LDSA) {
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int h = 0; h < NH; h++) {
-        const int row = 4 * i + (lane >> 4), l2 = 32 * h + 2 * (lane & 15);
-        at[row][l2] = ((long)(unsigned)araw[i * NH + h].y << 32) | (unsigned)araw[i * NH + h].x;
-        at[row][l2 + 1] = ((long)(unsigned)araw[i * NH + h].w << 32) | (unsigned)araw[i * NH + h].z;
-      }
-    // the wave reads back only what it wrote itself (LDS keeps a wave's order)
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int i = 0; i < NB; i++) av[i] = at[c][4 * i + g];  // row c, bytes 32 i + 8 g
   }
   __builtin_amdgcn_sched_barrier(0);
   chains<TM, NB>(av, bv, dwv, dxv, acc);
@@ -355,9 +340,8 @@ __global__ __launch_bounds__(KW * 64) void k_gemm_i8(const int8_t *wq, const int
     for (int t = 0; t < TM; t++)
 #pragma unroll
       for (int r = 0; r < 4; r++) acc[t][r] = 0.f;
-    chunk_chains<TM, false, 8>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks, nullptr, acc);
-    chunk_chains<TM, false, 8>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks + 8, nullptr,
-                               acc);
+    chunk_chains<TM, 8>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks, acc);
+    chunk_chains<TM, 8>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks + 8, acc);
 #pragma unroll
     for (int t = 0; t < TM; t++)
 #pragma unroll
@@ -390,6 +374,124 @@ __global__ __launch_bounds__(KW * 64) void k_gemm_i8(const int8_t *wq, const int
   }
 }
 
+// Many rows (a prompt's, or several prompts' together): a wave owns 64 weight
+// rows x one activation tile and walks the whole K, the chain of each
+// 512-column chunk in acc and the chunk sums added in chunk order in sum, so
+// nothing meets in LDS. Per pair of 32-blocks the operands of both sides
+// (coalesced 16-byte loads) are issued one pair ahead of the arithmetic, the
+// activation scales two pairs ahead; the weight scales of a chunk go through
+// the wave's own LDS as f32 (a lane needs those of four rows per block: one
+// 16-byte read), loaded a chunk ahead. The four waves of a workgroup take
+// consecutive weight rows of one activation tile (shared through the
+// CU's L1). What bounds it is the scale chain: 12 VALU instructions (convert,
+// multiply, fused multiply-add) per lane and MFMA, about three times the
+// MFMA's own cycles.
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void k_gemm_i8r(const int8_t *wq, const int8_t *xq, float *y,
+                                                     int N, int K, int M, int ldy) {
+  constexpr int NT = 4;
+  __shared__ float dws[4][2][kChunkBlocks][16 * NT];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  const int nb = K >> 5, np = K >> 6, nch = nb / kChunkBlocks, mt16 = (M + 15) >> 4;
+  const int n0 = (blockIdx.x * 4 + wave) * 16 * NT, mt = blockIdx.y;
+  const float *dx = scales_of(const_cast<int8_t *>(xq), M, K);
+  const int4 *wt = reinterpret_cast<const int4 *>(wq) + (size_t)(n0 >> 4) * K + lane;
+  // lane l loads (and writes to LDS) the scales of weight row n0 + l
+  const uint4 *dwr = reinterpret_cast<const uint4 *>(
+      reinterpret_cast<const _Float16 *>(wq + (size_t)N * K) + (size_t)(n0 + lane) * nb);
+  const int4 *xt = reinterpret_cast<const int4 *>(xq) + (size_t)mt * 64 + lane;
+  const float4 *dxr = reinterpret_cast<const float4 *>(dx + qscale_offset(16 * mt + c, 0, nb));
+  int4 a[2][NT], b[2];
+  float4 d4[2];
+  uint4 dw[2];
+  auto load = [&](int p, int s) {
+    b[s] = xt[(size_t)p * mt16 * 64];
+#pragma unroll
+    for (int i = 0; i < NT; i++) a[s][i] = wt[(size_t)i * K + 64 * p];
+  };
+  auto load_dx = [&](int p, int s) { d4[s] = dxr[(p >> 1) * 16]; };  // blocks 2p .. 2p + 3, p even
+  auto load_dw = [&](int ch) {
+    dw[0] = dwr[2 * ch];
+    dw[1] = dwr[2 * ch + 1];
+  };
+  auto store_dw = [&](int s) {
+    const unsigned u[8] = {dw[0].x, dw[0].y, dw[0].z, dw[0].w, dw[1].x, dw[1].y, dw[1].z, dw[1].w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      dws[wave][s][2 * i][lane] = (float)__builtin_bit_cast(_Float16, (unsigned short)(u[i] & 0xffff));
+      dws[wave][s][2 * i + 1][lane] = (float)__builtin_bit_cast(_Float16, (unsigned short)(u[i] >> 16));
+    }
+  };
+  float acc[NT][4], sum[NT][4];
+#pragma unroll
+  for (int i = 0; i < NT; i++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) sum[i][r] = 0.f;
+  load_dw(0);
+  load(0, 0);
+  load_dx(0, 0);
+  store_dw(0);
+  for (int ch = 0; ch < nch; ch++) {
+    const int p0 = ch * (kChunkBlocks / 2);
+    load_dw(min(ch + 1, nch - 1));
+#pragma unroll
+    for (int i = 0; i < NT; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[i][r] = 0.f;
+    // the wave reads back only what it wrote itself (LDS keeps a wave's order)
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < kChunkBlocks / 2; q++) {
+      load(min(p0 + q + 1, np - 1), (q + 1) & 1);
+      if ((q & 1) == 0) load_dx(min(p0 + q + 2, np - 2), ((q >> 1) + 1) & 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        float4 dv[NT];
+#pragma unroll
+        for (int i = 0; i < NT; i++)
+          dv[i] = *reinterpret_cast<const float4 *>(&dws[wave][ch & 1][2 * q + h][16 * i + 4 * g]);
+        const float4 &dq = d4[(q >> 1) & 1];
+        const float dxv = (q & 1) ? (h ? dq.w : dq.z) : (h ? dq.y : dq.x);
+#pragma unroll
+        for (int i = 0; i < NT; i++) {
+          const v4i ci = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+              half_pair(a[q & 1][i], h), half_pair(b[q & 1], h), v4i{0, 0, 0, 0}, 0, 0, 0);
+          const float dwv[4] = {dv[i].x, dv[i].y, dv[i].z, dv[i].w};
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            acc[i][r] = fmaf((float)ci[r], __fmul_rn(dwv[r], dxv), acc[i][r]);
+        }
+      }
+    }
+    store_dw((ch + 1) & 1);
+#pragma unroll
+    for (int i = 0; i < NT; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) sum[i][r] = __fadd_rn(sum[i][r], acc[i][r]);
+  }
+  const int m = mt * 16 + c;
+  if (m >= M) return;
+#pragma unroll
+  for (int i = 0; i < NT; i++) {
+    const int n = n0 + 16 * i + 4 * g;
+    const float(&s)[4] = sum[i];
+    if (EPI == EPI_SWIGLU) {  // gate, up of outputs n / 2, n / 2 + 1
+      *reinterpret_cast<float2 *>(y + (size_t)m * ldy + (n >> 1)) =
+          make_float2(silu_mul_ieee(s[0], s[1]), silu_mul_ieee(s[2], s[3]));
+    } else {
+      float4 *yp = reinterpret_cast<float4 *>(y + (size_t)m * ldy + n);
+      float4 v = make_float4(s[0], s[1], s[2], s[3]);
+      if (EPI == EPI_ADD) {
+        const float4 o = *yp;
+        v = make_float4(__fadd_rn(o.x, s[0]), __fadd_rn(o.y, s[1]), __fadd_rn(o.z, s[2]),
+                        __fadd_rn(o.w, s[3]));
+      }
+      *yp = v;
+    }
+  }
+}
+
 // One wave per (16 weight rows, chunk, TM activation tiles from TM z):
 // part[chunk][m][n] = the chunk's chains. The waves of one (weight rows,
 // chunk) over the row tiles are gridDim.x * gridDim.y workgroups apart (a
@@ -402,14 +504,12 @@ __global__ __launch_bounds__(64) void k_gemm_i8p(const int8_t *wq, const int8_t 
   const int n0 = blockIdx.x * 16, ch = blockIdx.y, mt0 = blockIdx.z * TM;
   const int mt16 = (M + 15) >> 4;
   const float *dx = scales_of(const_cast<int8_t *>(xq), M, K);
-  __shared__ long at[16][4 * kChunkBlocks + 1];
   float acc[TM][4];
 #pragma unroll
   for (int t = 0; t < TM; t++)
 #pragma unroll
     for (int r = 0; r < 4; r++) acc[t][r] = 0.f;
-  chunk_chains<TM, true, kChunkBlocks>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks, at,
-                                       acc);
+  chunk_chains<TM, kChunkBlocks>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks, acc);
 #pragma unroll
   for (int t = 0; t < TM; t++) {
     const int m = (mt0 + t) * 16 + c;
@@ -433,7 +533,6 @@ __global__ __launch_bounds__(512) void k_gemm_i8_swq(const int8_t *wq, const int
                                                      int8_t *yq, int N, int M) {
   constexpr int K = 1024, LD = TM * 16 + 4, NCH = K / (32 * kChunkBlocks);
   __shared__ float red[NCH][64][LD];
-  __shared__ long at[4 * NCH][16][4 * kChunkBlocks + 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int mt16 = (M + 15) >> 4, mt0 = blockIdx.y * TM;
@@ -445,8 +544,7 @@ __global__ __launch_bounds__(512) void k_gemm_i8_swq(const int8_t *wq, const int
   for (int t = 0; t < TM; t++)
 #pragma unroll
     for (int r = 0; r < 4; r++) acc[t][r] = 0.f;
-  chunk_chains<TM, true, kChunkBlocks>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks, at[w],
-                                       acc);
+  chunk_chains<TM, kChunkBlocks>(wq, xq, dx, N, K, n0, mt0, mt16, ch * kChunkBlocks, acc);
 #pragma unroll
   for (int t = 0; t < TM; t++)
 #pragma unroll
@@ -473,7 +571,7 @@ __global__ __launch_bounds__(512) void k_gemm_i8_swq(const int8_t *wq, const int
     const float d = __fdiv_rn(amax, 127.0f);
     const float id = d != 0.f ? __fdiv_rn(1.0f, d) : 0.f;
     yq[qtile_offset(m, 32 * b + j, mt16)] = (int8_t)(int)roundf(__fmul_rn(o, id));
-    if (j == 0) dy[(size_t)m * nbo + b] = (float)(_Float16)d;
+    if (j == 0) dy[qscale_offset(m, b, nbo)] = (float)(_Float16)d;
   }
 }
 
@@ -504,6 +602,34 @@ void gemm_by_k(const Mat &W, const QAct &xa, int M, int epi, float *y, int ldy, 
     gemm_launch<TM, 4>(W, xa, M, epi, y, ldy, st);
   else
     gemm_launch<TM, 2>(W, xa, M, epi, y, ldy, st);
+}
+
+// Q8_0 quants [N][K] row-major to operand order (wtile_offset), 16 bytes (a
+// lane's operands of a pair of blocks) per thread
+__global__ __launch_bounds__(256) void k_tile_q8(const int8_t *__restrict__ src, int N, int K,
+                                                 int8_t *__restrict__ dst) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (size_t)N * K / 16) return;
+  const int lane = i & 63;
+  const size_t tile = i >> 6;
+  const int np = K >> 6, p = (int)(tile % np), n = (int)(tile / np) * 16 + (lane & 15);
+  const int8_t *s = src + (size_t)n * K + 64 * p + 8 * (lane >> 4);
+  const uint2 a = *reinterpret_cast<const uint2 *>(s), b = *reinterpret_cast<const uint2 *>(s + 32);
+  reinterpret_cast<uint4 *>(dst)[i] = make_uint4(a.x, a.y, b.x, b.y);
+}
+
+void gemm_rows_launch(const Mat &W, const QAct &xa, int M, int epi, float *y, int ldy,
+                      hipStream_t st) {
+  const dim3 grid(W.N / 256, (M + 15) >> 4);
+#define Q3H_GEMM(E)                                                                            \
+  hipLaunchKernelGGL((k_gemm_i8r<E>), grid, dim3(256), 0, st, W.q, xa.q, y, W.N, W.K, M, ldy)
+  if (epi == EPI_STORE)
+    Q3H_GEMM(EPI_STORE);
+  else if (epi == EPI_ADD)
+    Q3H_GEMM(EPI_ADD);
+  else
+    Q3H_GEMM(EPI_SWIGLU);
+#undef Q3H_GEMM
 }
 
 // slices > 1 only without a norm (each slice a whole number of 32-blocks)
@@ -545,6 +671,12 @@ bool gemm_i8_supported(int N, int K) {
          K <= kQuantThreads * kQuantChunks * 8;
 }
 
+void launch_tile_q8(const int8_t *src, int N, int K, int8_t *dst, hipStream_t st) {
+  const size_t n = (size_t)N * K / 16;
+  hipLaunchKernelGGL(k_tile_q8, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, src, N, K,
+                     dst);
+}
+
 int gemm_i8_chunks(int K) { return K / (32 * kChunkBlocks); }
 
 size_t qact_bytes(int M, int K) {
@@ -571,14 +703,26 @@ void launch_swiglu_quantize(const float *part, int chunks, int M, int K, QAct ou
                            slices);
 }
 
+// The waves of k_gemm_i8r are 64 weight rows x one activation tile over the
+// whole K: taken from 768 of them (three quarters of the chip's SIMDs), with
+// fewer the chunk-parallel k_gemm_i8 ends first. Measured, both after the
+// operand-order weights: gate/up (96 waves a tile) 100 rows 8.5 / 7.5 us, 136
+// rows 8.6 / 9.7; q/k/v (64) 136 rows 7.9 / 6.9, 203 rows 8.2 / 8.8; o_proj
+// (16) 512 rows 13.6 / 11.1, 1024 rows 15.0 / 18.6, 4350 rows 48 / 68; gate/up
+// at 4350 rows 126 / 170 us (275 before, 215 -> 435 TOPS). Two tiles a wave
+// (weights loaded once for both) gave 120 there but 87 / 80 us on q/k/v.
+// k_gemm_i8 takes one tile per workgroup up to 160 rows (70 rows: q/k/v 4.6
+// against 5.3 us with two and 7.8 with four, 9.2 with row-major weights),
+// two above (o_proj, 512 rows: 11.1 / 11.8).
 void launch_gemm_i8(const Mat &W, const QAct &xa, int M, int epi, float *y, int ldy,
                     hipStream_t st) {
-  if (M <= 16)
+  const int mt16 = (M + 15) >> 4;
+  if (W.N % 256 == 0 && (W.N / 64) * mt16 >= 768)
+    gemm_rows_launch(W, xa, M, epi, y, ldy, st);
+  else if (M <= 160)
     gemm_by_k<1>(W, xa, M, epi, y, ldy, st);
-  else if (M <= 32)
-    gemm_by_k<2>(W, xa, M, epi, y, ldy, st);
   else
-    gemm_by_k<4>(W, xa, M, epi, y, ldy, st);
+    gemm_by_k<2>(W, xa, M, epi, y, ldy, st);
 }
 
 // Both products below take one 16-row activation tile per workgroup, the

@@ -10,7 +10,9 @@ namespace q3h {
 
 // A matrix [N][K] on the device: Q8_0 as int8 quants [N][K] followed, in the
 // same allocation, by the fp16 scales [N][K/32] (d == q + N*K; structure of
-// arrays, so a wave reads 1 KB of quants per instruction), or f32 [N][K].
+// arrays, so a wave reads 1 KB of quants per instruction), or f32 [N][K]. The
+// quants of act_q8 stacks are in the operand order of the int8 products
+// instead (wtile_offset).
 struct Mat {
   int N = 0, K = 0;
   int8_t *q = nullptr;
@@ -82,8 +84,9 @@ struct GemvArgs {
 
 // Activations quantized per 32-block for the int8 products, M rows padded to
 // Mp = M rounded up to 16, one buffer: the int8 values at q in MFMA operand
-// order (qtile_offset), then the fp16-rounded block scales [Mp][K/32] as f32
-// at q + Mp * K (qact_bytes(M, K) in all).
+// order (qtile_offset), then the fp16-rounded block scales as f32 at
+// q + Mp * K, in groups of 4 blocks of 16 rows (qscale_offset; qact_bytes(M, K)
+// in all).
 struct QAct {
   int8_t *q = nullptr;
 };
@@ -96,7 +99,25 @@ __host__ __device__ inline size_t qtile_offset(int m, int k, int mt16) {
   return ((((size_t)(b >> 1) * mt16 + (m >> 4)) * 64 + g * 16 + (m & 15)) * 16) + (b & 1) * 8 +
          (k & 7);
 }
+// scale of block b of row m (nb = K / 32 blocks a row): 16 rows x 4 blocks
+// contiguous, so that the 16 lanes of a product that hold a tile's rows read
+// 4 blocks' scales as 256 contiguous bytes (16 rows of nb scales each apart
+// cost the products a cache line per row and load: 4350 rows x gate/up 182 ->
+// 144 us with half as many tiles of them)
+__host__ __device__ inline size_t qscale_offset(int m, int b, int nb) {
+  return ((size_t)(m >> 4) * (nb >> 2) + (b >> 2)) * 64 + (m & 15) * 4 + (b & 3);
+}
 size_t qact_bytes(int M, int K);
+// The quants of a matrix of an act_q8 stack, in the same operand order: the
+// tile of rows 16 i .. + 15 and block pair p is the 1 KB at (i K / 64 + p) KB,
+// lane g * 16 + n % 16 its bytes 8g .. + 7 of both blocks (K % 64 == 0,
+// N % 16 == 0; the scales stay row-major at q + N K)
+__host__ __device__ inline size_t wtile_offset(int n, int k, int K) {
+  return (((size_t)(n >> 4) * (K >> 6) + (k >> 6)) * 64 + ((k & 31) >> 3) * 16 + (n & 15)) * 16 +
+         ((k >> 5) & 1) * 8 + (k & 7);
+}
+// row-major quants [N][K] at src to that order at dst
+void launch_tile_q8(const int8_t *src, int N, int K, int8_t *dst, hipStream_t st);
 
 void launch_gemv(const GemvArgs &a, int epi, bool q8, hipStream_t st);
 // the wide Q8_0 kernel (K in {1024, 2048, 3072}, N % 256 == 0, M <= 4);

@@ -65,7 +65,7 @@ __device__ inline void quant_row_regs(float (&v)[8], const float (&w8)[8], bool 
   }
   *reinterpret_cast<unsigned long long *>(xq + qtile_offset(m, 8 * t, mt16)) = packed;
   if ((t & 3) == 0)
-    reinterpret_cast<float *>(xq + (size_t)mt16 * 16 * K)[(size_t)m * nb + (t >> 2)] =
+    reinterpret_cast<float *>(xq + (size_t)mt16 * 16 * K)[qscale_offset(m, t >> 2, nb)] =
         (float)(_Float16)d;
 }
 

@@ -50,6 +50,34 @@ def test_int8_prefill_then_decode(small8, q3h, q3o, synth):
         octx.destroy()
 
 
+@pytest.fixture(scope="module")
+def long8(device):
+    m = Model(device, seed=19, talker_layers=2, cp_layers=1, act_q8=1, norm_std=0.1,
+              max_positions=800)
+    yield m
+    m.destroy()
+
+
+@pytest.mark.parametrize("rows", [65, 113, 160, 161, 177, 193, 753])
+def test_int8_prefill_many_rows(long8, q3h, q3o, synth, rows):
+    """Prompts around the row counts where a product changes its schedule
+    (launch_gemm_i8): one or two 16-row tiles per workgroup at 160 / 161, a
+    wave per 64 weight rows from 8 tiles on gate/up, 12 on q/k/v, 48 on o_proj
+    and down, with a last tile of one row (65, 113, 161, 177, 193, 753)."""
+    m = long8
+    print(f"case rows={rows}", flush=True)
+    ctx, octx = q3h.Context(m.ts, rows), q3o.Ctx(m.ot, rows)
+    try:
+        x = synth.prompt(50 + rows, rows)
+        lg, st = ctx.forward(x, head=0)
+        ost = octx.forward(x)
+        olg = m.ot.head(m.th, ost)
+        assert np.array_equal(lg, olg) and np.array_equal(st, ost), (rel(lg, olg), rel(st, ost))
+    finally:
+        ctx.destroy()
+        octx.destroy()
+
+
 @pytest.mark.parametrize("n", [3, 20, 32])
 def test_int8_batch_rows(small8, q3h, q3o, synth, n):
     """forward_embeds_batch over n contexts of ragged lengths (products over
