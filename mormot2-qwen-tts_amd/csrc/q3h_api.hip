@@ -277,7 +277,9 @@ static void run_layers_f32(const q3h_stack *s, Work &w, int M, int positions, bo
     at.rope_cs = reinterpret_cast<const float2 *>(s->rope_cs);
     at.out = w.att;
     at.part = w.part;
-    if (!fused && single_context && M >= kPrefillRows)
+    at.tiles = io.tiles;
+    at.n_tiles = io.n_tiles;
+    if (!fused && (io.tiles || (single_context && M >= kPrefillRows)))
       launch_attn_prefill(at, M, kv16, st);
     else
       launch_attn(at, M, positions, fused, kv16, st);

@@ -165,6 +165,8 @@ struct LayerIO {
   const float *final_norm = nullptr;  // after the last layer: RMSNorm with it, quantized into w.xa
   float *final_normed = nullptr;      // [M][hidden] device: those normed rows (int8 path, few rows)
   bool single_context = false;        // the rows are consecutive positions of one context
+  const int2 *tiles = nullptr;        // rows of several prompts: AttnArgs::tiles of their attention
+  int n_tiles = 0;
   float *layer_out = nullptr;         // [layers][M][hidden] device: w.h after each layer
   // the rows come in pairs, row 2i + 1 at the position after row 2i's in the
   // same context (the int8 path over few rows then runs the fused attention)
@@ -172,6 +174,9 @@ struct LayerIO {
 };
 // whether run_layers takes the int8 partial-product path for M rows of stack s
 bool partial_path(const struct ::q3h_stack *s, int M);
+
+// whether run_layers takes the sliced f32-activation path for M rows of stack s
+bool f32_slice_path(const struct ::q3h_stack *s, int M);
 
 // fused: every row is the single new position of its own context; positions:
 // the most positions any row attends to (its own included), Work sized for

@@ -955,8 +955,9 @@ __device__ __forceinline__ v4f mfma_x3(const u32x4 (&a)[3], const u32x4 (&b)[3],
   return acc;
 }
 
-// Prefill attention (rows m = 0 .. M-1 of one context at positions pos0 + m,
-// their keys and values already in the cache, q already normed and rotated):
+// Prefill attention (rows m = 0 .. M-1 of one context at positions
+// rd[0].pos + m, or the query tiles of several contexts' rows, their keys and
+// values already in the cache, q already normed and rotated):
 // causal softmax(q K^T / sqrt(128)) V on the bf16 matrix cores
 // (v_mfma_f32_16x16x32_bf16, lane l holding A[l % 16][8 (l / 16) .. + 7] and
 // B[8 (l / 16) .. + 7][l % 16], receiving D[4 (l / 16) + r][l % 16]) with
@@ -981,26 +982,27 @@ template <typename KV, int GRP>
 __global__ __launch_bounds__(256) void k_attn_prefill_x3(const RowDesc *__restrict__ rd,
                                                          const float *__restrict__ qkv, int ldq,
                                                          int layer, int kvh, int M,
-                                                         float *__restrict__ outp) {
+                                                         float *__restrict__ outp,
+                                                         const int2 *__restrict__ tiles) {
   __shared__ float ms[4][16], ls[4][16];
   __shared__ float os[4][8][4][64];
   // the tiles with the most keys first; a kv head's query heads on one XCD
   const int g = blockIdx.x % kvh, h = g * GRP + blockIdx.x / kvh;
-  const int q0 = (gridDim.y - 1 - blockIdx.y) * 16;
+  const int2 tile = tiles ? tiles[blockIdx.y] : make_int2((gridDim.y - 1 - blockIdx.y) * 16, 16);
+  const int q0 = tile.x, nq = tiles ? tile.y : min(16, M - q0);
   const int heads = GRP * kvh;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r16 = lane & 15, gq = lane >> 4;
-  const RowDesc d = rd[0];
-  const int pos0 = d.pos;
-  const int p_hi = pos0 + min(q0 + 15, M - 1);  // the tile's last position
-  const int pq = pos0 + q0 + r16;              // this lane's query position
+  const RowDesc d = rd[q0];
+  const int p_hi = d.pos + nq - 1;  // the tile's last position
+  const int pq = d.pos + r16;       // this lane's query position
   const size_t head_off = ((size_t)layer * kvh + g) * d.max_pos * HD;
   const KV *kc = global_ptr(reinterpret_cast<const KV *>(d.k)) + head_off;
   const KV *vc = global_ptr(reinterpret_cast<const KV *>(d.v)) + head_off;
-  // this lane's query: row min(q0 + r16, M - 1), dims 32 c + 8 gq .. + 7
+  // this lane's query: row q0 + min(r16, nq - 1), dims 32 c + 8 gq .. + 7
   u32x4 qp[4][3];
   {
-    const float *qr = qkv + (size_t)min(q0 + r16, M - 1) * ldq + h * HD + 8 * gq;
+    const float *qr = qkv + (size_t)(q0 + min(r16, nq - 1)) * ldq + h * HD + 8 * gq;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       const float4 a = *reinterpret_cast<const float4 *>(qr + 32 * c);
@@ -1101,7 +1103,7 @@ __global__ __launch_bounds__(256) void k_attn_prefill_x3(const RowDesc *__restri
   // output (query q, dim k): tile i = k / 16, lane 16 (q / 4) + k % 16, r = q % 4
   for (int e = t; e < 16 * HD; e += 256) {
     const int q = e / HD, k = e % HD;
-    if (q0 + q >= M) break;
+    if (q >= nq) break;
     const int i = k >> 4, l = 16 * (q >> 2) + (k & 15), r = q & 3;
     float mx = ms[0][q];
 #pragma unroll
@@ -1294,11 +1296,11 @@ void launch_attn_merge_o(const AttnArgs &a, const Mat &wo, float *y, int positio
 
 namespace q3h {
 void launch_attn_prefill(const AttnArgs &a, int M, bool kv16, hipStream_t st) {
-  const dim3 grid(a.heads, (M + 15) / 16), block(256);
+  const dim3 grid(a.heads, a.tiles ? a.n_tiles : (M + kPrefillTile - 1) / kPrefillTile), block(256);
   const int grp = a.heads / a.kvh;
 #define Q3H_P(KV, G)                                                                         \
   hipLaunchKernelGGL((k_attn_prefill_x3<KV, G>), grid, block, 0, st, a.rd, a.qkv, a.ldq,      \
-                     a.layer, a.kvh, M, a.out)
+                     a.layer, a.kvh, M, a.out, a.tiles)
   if (kv16) {
     if (grp == 1) Q3H_P(_Float16, 1);
     else if (grp == 2) Q3H_P(_Float16, 2);

@@ -685,9 +685,9 @@ size_t qact_bytes(int M, int K) {
 }
 
 void launch_quantize_act(const float *x, int ldx, int M, int K, const float *norm_w, float eps,
-                         QAct out, float *xn_out, hipStream_t st) {
-  quant_launch<SRC_X>(const_cast<float *>(x), nullptr, ldx, M, K, norm_w, eps, out, xn_out, 1,
-                      st);
+                         QAct out, float *xn_out, hipStream_t st, int xn_rows) {
+  quant_launch<SRC_X>(const_cast<float *>(x), nullptr, ldx, M, K, norm_w, eps, out, xn_out,
+                      xn_rows, st);
 }
 
 void launch_residual_quantize(float *h, const float *part, int chunks, int M, int K,

@@ -175,8 +175,9 @@ void launch_resid_norm(float *h, const float *part, int M, int K, const float *n
 bool gemm_i8_supported(int N, int K);
 // rows x [M][ldx] (RMS-normed with norm_w when non-null) quantized into out;
 // xn_out, when non-null, receives the (normed) row M - 1
+// (xn_rows > 1: the rows M - xn_rows .. M - 1)
 void launch_quantize_act(const float *x, int ldx, int M, int K, const float *norm_w, float eps,
-                         QAct out, float *xn_out, hipStream_t st);
+                         QAct out, float *xn_out, hipStream_t st, int xn_rows = 1);
 // y [M][ldy] (+)= W . x over the quantized rows xa (Q8_0 W)
 void launch_gemm_i8(const Mat &W, const QAct &xa, int M, int epi, float *y, int ldy,
                     hipStream_t st);
@@ -235,7 +236,14 @@ struct AttnArgs {
   float *out;    // [M][heads * head_dim]
   float *part;   // [M][heads][attn_splits slots][head_dim + 2]
   int layers;    // > layer + 1: a decode launch also loads layer + 1's cache rows ahead
+  // launch_attn_prefill over several contexts' rows: its tiles of queries
+  // (x: first row, y: rows, consecutive positions of one context), n_tiles of
+  // them; null: M rows of one context
+  const int2 *tiles;
+  int n_tiles;
 };
+// rows per query tile of launch_attn_prefill
+constexpr int kPrefillTile = 16;
 // how the decode attention cuts contexts of up to `positions` positions: len
 // positions per split (a multiple of 16), threads per workgroup (0: one
 // workgroup per query head over at most 256 positions, no split); fold: the
