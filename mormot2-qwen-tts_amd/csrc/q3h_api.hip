@@ -171,13 +171,27 @@ static void probe_layer(const LayerIO &io, const Work &w, int l, int M, int H, h
               "probe copy");
 }
 
+// the int8 path's attention over whole q/k/v rows: prompts by the kernel that
+// shares the keys between rows, where it takes them
+static void prompt_attn_x(const q3h_stack *s, Work &w, AttnArgs &at, int M, int positions,
+                          bool fused, const LayerIO &io, hipStream_t st) {
+  const q3h_stack_config &c = s->cfg;
+  at.tiles = io.tiles;
+  at.n_tiles = io.n_tiles;
+  at.tile_rows = io.tile_rows;
+  if (!fused && (io.tiles || io.single_context) &&
+      launch_attn_x_prompt(at, M, positions, c.kv_f16 != 0, w.xa, st))
+    return;
+  launch_attn_x(at, M, fused, c.kv_f16 != 0, 0, w.xa, c.max_positions, st);
+}
+
 // The int8 path over M <= kPartialRows rows: every product leaves its chunk
 // partials (one wave per 16 rows and 512 columns over the whole chip), and
 // the consumer adds them in chunk order: the attention prologue (q/k/v, decode
 // rows), the residual add + RMSNorm + quantization of the next input (o_proj,
 // down), SiLU(gate) * up + quantization (gate/up). Results equal the
 // workgroup-reduced schedule of run_layers to the bit.
-static void run_layers_partial(const q3h_stack *s, Work &w, int M, bool fused,
+static void run_layers_partial(const q3h_stack *s, Work &w, int M, int positions, bool fused,
                                const LayerIO &io, hipStream_t st) {
   const q3h_stack_config &c = s->cfg;
   const int H = c.hidden, hd = c.head_dim, NQ = c.heads * hd, NKV = c.kv_heads * hd;
@@ -208,7 +222,7 @@ static void run_layers_partial(const q3h_stack *s, Work &w, int M, bool fused,
       launch_qk_rope_append(w.qkv, ldq, w.rd, M, l, c.heads, c.kv_heads, hd, L.q_norm,
                             L.k_norm, eps, s->rope_cs, kv16, st);
       at.qkv = w.qkv;
-      launch_attn_x(at, M, false, kv16, 0, w.xa, c.max_positions, st);
+      prompt_attn_x(s, w, at, M, positions, false, io, st);
     }
     launch_gemm_i8_partial(L.o, w.xa, M, w.gpart, st);
     launch_residual_quantize(w.h, w.gpart, gemm_i8_chunks(NQ), M, H, L.post_norm, eps, &w.xa,
@@ -306,7 +320,7 @@ void run_layers(const q3h_stack *s, Work &w, int M, int positions, bool fused, h
   const int I = c.intermediate, ldq = NQ + 2 * NKV;
   const bool kv16 = c.kv_f16 != 0;
   if (partial_path(s, M)) {
-    run_layers_partial(s, w, M, fused, io, st);
+    run_layers_partial(s, w, M, positions, fused, io, st);
     return;
   }
   if (f32_slice_path(s, M)) {
@@ -331,7 +345,7 @@ void run_layers(const q3h_stack *s, Work &w, int M, int positions, bool fused, h
       at.kvh = c.kv_heads;
       at.qkn = L.q_norm;
       at.rope_cs = reinterpret_cast<const float2 *>(s->rope_cs);
-      launch_attn_x(at, M, fused, kv16, 0, w.xa, c.max_positions, st);
+      prompt_attn_x(s, w, at, M, positions, fused, io, st);
       launch_gemm_i8(L.o, w.xa, M, EPI_ADD, w.h, H, st);
       linear(s, w, L.gu, w.h, H, M, L.post_norm, w.act, I, EPI_SWIGLU, nullptr, st);
       linear(s, w, L.down, w.act, I, M, nullptr, w.h, H, EPI_ADD, nullptr, st);

@@ -166,7 +166,7 @@ struct LayerIO {
   float *final_normed = nullptr;      // [M][hidden] device: those normed rows (int8 path, few rows)
   bool single_context = false;        // the rows are consecutive positions of one context
   const int2 *tiles = nullptr;        // rows of several prompts: AttnArgs::tiles of their attention
-  int n_tiles = 0;
+  int n_tiles = 0, tile_rows = 0;
   float *layer_out = nullptr;         // [layers][M][hidden] device: w.h after each layer
   // the rows come in pairs, row 2i + 1 at the position after row 2i's in the
   // same context (the int8 path over few rows then runs the fused attention)

@@ -448,6 +448,283 @@ __global__ __launch_bounds__(NT) void k_attn_x(const RowDesc *rd, const float *q
   }
 }
 
+// four cached values as floats
+template <typename KV>
+__device__ __forceinline__ float4 load4(const KV *p) {
+  if constexpr (sizeof(KV) == 4) {
+    return *reinterpret_cast<const float4 *>(p);
+  } else {
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    const h4 h = *reinterpret_cast<const h4 *>(p);
+    return make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
+  }
+}
+
+// Two chains of 8 fused multiply-adds (the first product rounded alone, as the
+// multiply-add onto zero does) of the 16 elements of q, held one per lane of
+// every 16-lane row, and the lane's own k: a0 over elements 0 .. 7, a1 over 8
+// .. 15. The element is taken from the row by the multiply-add itself (DPP
+// row_newbcast), an operand form the compiler does not build for fused
+// multiply-adds; the wait states let a q written just before be read by DPP.
+__device__ __forceinline__ void dot8x2(float q, const float4 &k0, const float4 &k1,
+                                       const float4 &k2, const float4 &k3, float &a0, float &a1) {
+#define Q3H_BC(n) " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n"
+  asm("s_nop 1\n"
+      "v_mul_f32_dpp %0, %2, %3" Q3H_BC(0) "v_mul_f32_dpp %1, %2, %11" Q3H_BC(8)
+      "v_fmac_f32_dpp %0, %2, %4" Q3H_BC(1) "v_fmac_f32_dpp %1, %2, %12" Q3H_BC(9)
+      "v_fmac_f32_dpp %0, %2, %5" Q3H_BC(2) "v_fmac_f32_dpp %1, %2, %13" Q3H_BC(10)
+      "v_fmac_f32_dpp %0, %2, %6" Q3H_BC(3) "v_fmac_f32_dpp %1, %2, %14" Q3H_BC(11)
+      "v_fmac_f32_dpp %0, %2, %7" Q3H_BC(4) "v_fmac_f32_dpp %1, %2, %15" Q3H_BC(12)
+      "v_fmac_f32_dpp %0, %2, %8" Q3H_BC(5) "v_fmac_f32_dpp %1, %2, %16" Q3H_BC(13)
+      "v_fmac_f32_dpp %0, %2, %9" Q3H_BC(6) "v_fmac_f32_dpp %1, %2, %17" Q3H_BC(14)
+      "v_fmac_f32_dpp %0, %2, %10" Q3H_BC(7) "v_fmac_f32_dpp %1, %2, %18" Q3H_BC(15)
+      : "=&v"(a0), "=&v"(a1)
+      : "v"(q), "v"(k0.x), "v"(k0.y), "v"(k0.z), "v"(k0.w), "v"(k1.x), "v"(k1.y), "v"(k1.z),
+        "v"(k1.w), "v"(k2.x), "v"(k2.y), "v"(k2.z), "v"(k2.w), "v"(k3.x), "v"(k3.y), "v"(k3.z),
+        "v"(k3.w));
+#undef Q3H_BC
+}
+
+// The same attention for prompt rows (q normed and rotated, every K/V row of
+// the tile's context already appended), several rows sharing one read of the
+// keys and values: a workgroup of 4 waves per (kv head, tile of R = PAIRS / GRP
+// consecutive positions of one context), PAIRS (row, query head) pairs, every
+// value by the operations of k_attn_x in the same order.
+//  - scores: 64 keys at a time through LDS, then a key per lane in 128
+//    registers; the wave's PAIRS / 4 pairs one after another, the query's
+//    elements broadcast by DPP: 16 chains of 8 fused multiply-adds and the 15
+//    adds of their tree in one lane, where k_attn_x's 16 lanes per key pay 4
+//    DPP adds each (146 instructions per 64 keys and pair against about 200)
+//    and re-read the key from L2 for every row;
+//  - softmax: the wave's pairs together, a position per lane; the weights e * inv left in place of the scores;
+//  - values: half-wave 2 wave + h runs chain 2 wave + h over positions = chain
+//    mod 8, 4 dims per lane, all pairs (the value row loaded once for them, the
+//    weights of a position as 16-byte LDS broadcasts); positions after a row's
+//    own are skipped by selects, in the tile's last rounds only;
+//  - the chains joined through LDS 8 pairs at a time and quantized.
+// Scores in LDS: [position][PAIRS + 4] (rows of 16-byte multiples whose lanes
+// start 4 banks apart). What bounds it is the VALU: about 4.3 instructions per
+// (row, head, position).
+template <typename KV, int GRP, int PAIRS>
+__global__ __launch_bounds__(256, 2) void k_attn_xp(const RowDesc *__restrict__ rd,
+                                                    const float *__restrict__ qkv,
+                                                    int8_t *__restrict__ xq, int layer, int kvh,
+                                                    int M, const int2 *__restrict__ tiles) {
+  constexpr int R = PAIRS / GRP, ST = PAIRS + 4, PW = PAIRS / 4, KS = HD + 4;
+  static_assert(PAIRS % 8 == 0 && PAIRS % GRP == 0, "8 pairs per join round");
+  extern __shared__ float sm[];
+  float *ks = sm;             // [64][KS] keys; then the joining sums [4][8][HD]
+  float *sc = sm + 64 * KS;   // [positions rounded up to 64][ST]
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int g = blockIdx.x, heads = kvh * GRP, ldq = (heads + 2 * kvh) * HD;
+  const int NQ = heads * HD, nbq = NQ >> 5, mt16 = (M + 15) >> 4;
+  const int tl = gridDim.y - 1 - blockIdx.y;
+  const int2 tile = tiles ? tiles[blockIdx.y] : make_int2(tl * R, min(R, M - tl * R));
+  const int q0 = tile.x, nq = tile.y;
+  const RowDesc d = rd[q0];
+  const int pos0 = d.pos, L = pos0 + nq;  // positions of the tile's last row
+  const size_t head_off = ((size_t)layer * kvh + g) * d.max_pos * HD;
+  const KV *kc = global_ptr(reinterpret_cast<const KV *>(d.k)) + head_off;
+  const KV *vc = global_ptr(reinterpret_cast<const KV *>(d.v)) + head_off;
+  const float scale = (float)(1.0 / __builtin_sqrt((double)HD));
+
+  // scores
+  float4 kn[8];
+  auto load_keys = [&](int kb) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int f = t + 256 * i;  // float4 f of the block's 64 x 32
+      kn[i] = load4(kc + (size_t)min(kb + (f >> 5), L - 1) * HD + 4 * (f & 31));
+    }
+  };
+  // element 16 k + lane % 16 of the query of the wave's pair i, k < 8
+  float qn[8];
+  auto load_q = [&](int i) {
+    const int pair = wave * PW + i, r = min(pair / GRP, nq - 1);
+    const float *q = qkv + (size_t)(q0 + r) * ldq + (g * GRP + pair % GRP) * HD + (lane & 15);
+#pragma unroll
+    for (int k = 0; k < 8; k++) qn[k] = q[16 * k];
+  };
+  load_keys(0);
+  load_q(0);
+  for (int kb = 0; kb < L; kb += 64) {
+    if (kb) __syncthreads();  // the waves have read the block before
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int f = t + 256 * i;
+      *reinterpret_cast<float4 *>(&ks[(f >> 5) * KS + 4 * (f & 31)]) = kn[i];
+    }
+    __syncthreads();
+    float4 kr[HD / 4];
+#pragma unroll
+    for (int i = 0; i < HD / 4; i++) kr[i] = *reinterpret_cast<const float4 *>(&ks[lane * KS + 4 * i]);
+    load_keys(kb + 64);
+    for (int i = 0; i < PW; i++) {
+      const int pair = wave * PW + i, r = min(pair / GRP, nq - 1);
+      float q[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) q[k] = qn[k];
+      load_q(i + 1 < PW ? i + 1 : 0);
+      if (kb > pos0 + r) continue;  // wholly after the row
+      float a[16];
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        dot8x2(q[k], kr[4 * k], kr[4 * k + 1], kr[4 * k + 2], kr[4 * k + 3], a[2 * k], a[2 * k + 1]);
+#pragma unroll
+      for (int n = 8; n >= 1; n >>= 1)
+#pragma unroll
+        for (int c = 0; c < n; c++) a[c] = __fadd_rn(a[2 * c], a[2 * c + 1]);
+      sc[(kb + lane) * ST + pair] = __fmul_rn(a[0], scale);
+    }
+  }
+  __syncthreads();
+
+  // softmax: the wave's PW pairs together, a position per lane and round
+  {
+    float mx[PW], inv[PW];
+    double sum[PW];
+    int Lr[PW];
+    float *sw = sc + wave * PW;
+#pragma unroll
+    for (int i = 0; i < PW; i++) {
+      Lr[i] = pos0 + min((wave * PW + i) / GRP, nq - 1) + 1;
+      mx[i] = -INFINITY;
+      sum[i] = 0.0;
+    }
+    auto get = [&](int p, float (&v)[PW]) {
+#pragma unroll
+      for (int i = 0; i < PW; i += 2) {
+        const float2 u = *reinterpret_cast<const float2 *>(&sw[p * ST + i]);
+        v[i] = u.x;
+        v[i + 1] = u.y;
+      }
+    };
+    auto put = [&](int p, const float (&v)[PW]) {
+#pragma unroll
+      for (int i = 0; i < PW; i += 2)
+        *reinterpret_cast<float2 *>(&sw[p * ST + i]) = make_float2(v[i], v[i + 1]);
+    };
+    float v[PW];
+    for (int p = lane; p < L; p += 64) {
+      get(p, v);
+#pragma unroll
+      for (int i = 0; i < PW; i++) mx[i] = p < Lr[i] ? fmaxf(mx[i], v[i]) : mx[i];
+    }
+#pragma unroll
+    for (int i = 0; i < PW; i++) mx[i] = wave_max_dpp(mx[i]);
+    for (int p = lane; p < L; p += 64) {
+      get(p, v);
+#pragma unroll
+      for (int i = 0; i < PW; i++) {
+        v[i] = exp_ieee(__fsub_rn(v[i], mx[i]));
+        sum[i] += p < Lr[i] ? (double)v[i] : 0.0;
+      }
+      put(p, v);
+    }
+#pragma unroll
+    for (int i = 0; i < PW; i++) inv[i] = (float)(1.0 / wave_sum_dpp_d(sum[i]));
+    for (int p = lane; p < L; p += 64) {
+      get(p, v);
+#pragma unroll
+      for (int i = 0; i < PW; i++) v[i] = __fmul_rn(v[i], inv[i]);
+      put(p, v);
+    }
+  }
+  __syncthreads();
+
+  // values
+  const int ch = 2 * wave + (lane >> 5), dim = 4 * (lane & 31);
+  float c[PAIRS][4];
+#pragma unroll
+  for (int j = 0; j < PAIRS; j++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) c[j][e] = 0.f;
+  auto load_v = [&](int p) { return load4(vc + (size_t)min(p, L - 1) * HD + dim); };
+  // position p of the chain, for every pair (MASK: those whose row is at p or after)
+  auto step = [&](int p, const float4 &v, auto masked) {
+    constexpr bool MASK = decltype(masked)::value;
+    const float *w = sc + (size_t)(MASK ? min(p, L - 1) : p) * ST;
+#pragma unroll
+    for (int j0 = 0; j0 < PAIRS; j0 += 4) {
+      const float4 w4 = *reinterpret_cast<const float4 *>(w + j0);
+      const float wj[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        float *cj = c[j0 + j];
+        const bool on = !MASK || p <= pos0 + (j0 + j) / GRP;
+        cj[0] = on ? fmaf(wj[j], v.x, cj[0]) : cj[0];
+        cj[1] = on ? fmaf(wj[j], v.y, cj[1]) : cj[1];
+        cj[2] = on ? fmaf(wj[j], v.z, cj[2]) : cj[2];
+        cj[3] = on ? fmaf(wj[j], v.w, cj[3]) : cj[3];
+      }
+    }
+  };
+  int p0 = 0;
+  float4 vb[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++) vb[u] = load_v(ch + 8 * u);
+  for (; p0 + 31 <= pos0; p0 += 32) {
+    float4 vn[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) vn[u] = load_v(p0 + 32 + ch + 8 * u);
+#pragma unroll
+    for (int u = 0; u < 4; u++) step(p0 + ch + 8 * u, vb[u], std::false_type{});
+#pragma unroll
+    for (int u = 0; u < 4; u++) vb[u] = vn[u];
+  }
+  for (; p0 < L; p0 += 8) {
+    const float4 v = load_v(p0 + ch);
+    step(p0 + ch, v, std::true_type{});
+  }
+  // the sums of chains 2 wave and 2 wave + 1 added across the halves, the
+  // waves' through LDS 8 pairs at a time, quantized per 32-block (8 lanes x 4
+  // dims): thread t takes pair t / 32 of the 8, dims 4 (t % 32) .. + 3
+  float *dx = reinterpret_cast<float *>(xq + (size_t)mt16 * 16 * NQ);
+#pragma unroll
+  for (int j0 = 0; j0 < PAIRS; j0 += 8) {
+    __syncthreads();  // the keys, or the sums of the round before, are read
+    // the lower half holds pair j0 + i, the upper one pair j0 + 4 + i
+    const int half = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float4 o;
+      o.x = swap32_add(c[j0 + i][0], c[j0 + 4 + i][0]);
+      o.y = swap32_add(c[j0 + i][1], c[j0 + 4 + i][1]);
+      o.z = swap32_add(c[j0 + i][2], c[j0 + 4 + i][2]);
+      o.w = swap32_add(c[j0 + i][3], c[j0 + 4 + i][3]);
+      *reinterpret_cast<float4 *>(&ks[(wave * 8 + 4 * half + i) * HD + dim]) = o;
+    }
+    __syncthreads();
+    const int jp = t >> 5, k = 4 * (t & 31), pair = j0 + jp, r = pair / GRP;
+    float o[4], amax = 0.f;
+    float4 s4[4];
+#pragma unroll
+    for (int w = 0; w < 4; w++) s4[w] = *reinterpret_cast<const float4 *>(&ks[(w * 8 + jp) * HD + k]);
+    const float sv[4][4] = {{s4[0].x, s4[0].y, s4[0].z, s4[0].w},
+                            {s4[1].x, s4[1].y, s4[1].z, s4[1].w},
+                            {s4[2].x, s4[2].y, s4[2].z, s4[2].w},
+                            {s4[3].x, s4[3].y, s4[3].z, s4[3].w}};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      o[e] = __fadd_rn(__fadd_rn(sv[0][e], sv[1][e]), __fadd_rn(sv[2][e], sv[3][e]));
+      amax = fmaxf(amax, fabsf(o[e]));
+    }
+    amax = quad_max_dpp(amax);
+    amax = fmaxf(amax, dpp_f_keep<kHalfMirror>(amax));
+    if (r < nq) {
+      const float dq = __fdiv_rn(amax, 127.0f);
+      const float id = dq != 0.f ? __fdiv_rn(1.0f, dq) : 0.f;
+      unsigned packed = 0;
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        packed |= (unsigned)(uint8_t)(int8_t)(int)roundf(__fmul_rn(o[e], id)) << (8 * e);
+      const int m = q0 + r, h = g * GRP + pair % GRP;
+      *reinterpret_cast<unsigned *>(xq + qtile_offset(m, h * HD + k, mt16)) = packed;
+      if ((t & 7) == 0) dx[qscale_offset(m, 4 * h + (k >> 5), nbq)] = (float)(_Float16)dq;
+    }
+  }
+}
+
 }  // namespace
 
 bool attn_x_supported(int heads, int kvh, int head_dim, int max_positions) {
@@ -496,6 +773,74 @@ void attn_x_len(const AttnArgs &a, int M, int nch, const QAct &xa, int max_posit
     attn_x_grp<KV, F, 4, 8, 512, true>(a, M, nch, xa, max_positions, st);
   else
     attn_x_grp<KV, F, 8, 16, 512, false>(a, M, nch, xa, max_positions, st);
+}
+
+// LDS of k_attn_xp: the keys, then a score row per position
+template <int PAIRS>
+constexpr size_t attn_xp_lds(int positions) {
+  return sizeof(float) * (64 * (HD + 4) + (size_t)((positions + 63) / 64 * 64) * (PAIRS + 4));
+}
+constexpr size_t kLdsBytes = 160 << 10;
+
+// The rows of k_attn_xp's tiles, 0 where k_attn_x takes the rows: 16 (row,
+// head) pairs per workgroup where that still makes 1024 workgroups, 8 below
+// (601 rows: 51 us against 71; 1201 rows: 224 with 16, 275 with 8), and where
+// 16 pairs' scores do not fit in LDS (above 1600 positions; 2300 rows: 870
+// against 1016 us by k_attn_x). k_attn_x takes contexts above 2688 positions
+// (8 pairs' scores do not fit), and few rows onto a long context, whose walk
+// over the keys it spreads over more workgroups. 3798 rows of 32 prompts: 110
+// us, 430 by k_attn_x; 203 rows 13.5 / 29; 70 rows 7.9 / 12.9; 17 rows 5.7 /
+// 6.7.
+int attn_x_tile_rows(int heads, int kvh, int M, int positions) {
+  const int grp = heads / kvh;
+  if (M < 8 || 4 * M < positions || attn_xp_lds<8>(positions) > kLdsBytes) return 0;
+  const int r16 = 16 / grp;
+  return (M + r16 - 1) / r16 * kvh >= 1024 && attn_xp_lds<16>(positions) <= kLdsBytes ? r16 : 8 / grp;
+}
+
+template <typename KV, int GRP, int PAIRS>
+void attn_xp_launch(const AttnArgs &a, int M, int positions, const QAct &xa, hipStream_t st) {
+  constexpr int R = PAIRS / GRP;
+  const dim3 grid(a.kvh, a.tiles ? a.n_tiles : (M + R - 1) / R);
+  const size_t lds = attn_xp_lds<PAIRS>(positions);
+  if (lds > (64 << 10))
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_attn_xp<KV, GRP, PAIRS>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes),
+              "attention LDS");
+  hipLaunchKernelGGL((k_attn_xp<KV, GRP, PAIRS>), grid, dim3(256), lds, st, a.rd, a.qkv, xa.q,
+                     a.layer, a.kvh, M, a.tiles);
+}
+
+template <typename KV, int GRP>
+void attn_xp_grp(const AttnArgs &a, int M, int rows, int positions, const QAct &xa,
+                 hipStream_t st) {
+  if (rows == 16 / GRP)
+    attn_xp_launch<KV, GRP, 16>(a, M, positions, xa, st);
+  else
+    attn_xp_launch<KV, GRP, 8>(a, M, positions, xa, st);
+}
+
+bool launch_attn_x_prompt(const AttnArgs &a, int M, int positions, bool kv16, const QAct &xa,
+                          hipStream_t st) {
+  const int rows = a.tiles ? a.tile_rows : attn_x_tile_rows(a.heads, a.kvh, M, positions);
+  if (rows == 0) return false;
+  require(a.ldq == (a.heads + 2 * a.kvh) * HD, Q3H_E_ARG, "attention: q/k/v rows not packed");
+  const int grp = a.heads / a.kvh;
+#define Q3H_XP(KV)                                             \
+  do {                                                         \
+    if (grp == 1)                                              \
+      attn_xp_grp<KV, 1>(a, M, rows, positions, xa, st);       \
+    else if (grp == 2)                                         \
+      attn_xp_grp<KV, 2>(a, M, rows, positions, xa, st);       \
+    else                                                       \
+      attn_xp_grp<KV, 4>(a, M, rows, positions, xa, st);       \
+  } while (0)
+  if (kv16)
+    Q3H_XP(_Float16);
+  else
+    Q3H_XP(float);
+#undef Q3H_XP
+  return true;
 }
 
 bool attn_x_pairs_supported(int max_positions) { return max_positions <= 32; }

@@ -1208,11 +1208,14 @@ void start_group(q3h_frame *f, const StartArg *args, int n, std::vector<StartPro
     longest = std::max(longest, a.rows);
   }
   // the query tiles, those with the most keys first
+  const int tr = s->cfg.act_q8 ? attn_x_tile_rows(s->cfg.heads, s->cfg.kv_heads, M, longest)
+                               : kPrefillTile;
   tiles.clear();
-  for (int q0 = (longest - 1) / kPrefillTile * kPrefillTile; q0 >= 0; q0 -= kPrefillTile)
-    for (int i = 0; i < n; i++)
-      if (q0 < args[i].rows)
-        tiles.push_back(make_int2(vals[i].row0 + q0, std::min(kPrefillTile, args[i].rows - q0)));
+  if (tr > 0)
+    for (int q0 = (longest - 1) / tr * tr; q0 >= 0; q0 -= tr)
+      for (int i = 0; i < n; i++)
+        if (q0 < args[i].rows)
+          tiles.push_back(make_int2(vals[i].row0 + q0, std::min(tr, args[i].rows - q0)));
   Work &w = f->sw;
   w.ensure(s, M, 0, 0);
   if (f->start_tiles_cap < (int)tiles.size()) {
@@ -1225,9 +1228,10 @@ void start_group(q3h_frame *f, const StartArg *args, int n, std::vector<StartPro
   check_hip(hipMemcpyAsync(f->start_prompts, vals.data(), sizeof(StartPrompt) * n,
                            hipMemcpyHostToDevice, st),
             "upload prompts");
-  check_hip(hipMemcpyAsync(f->start_tiles, tiles.data(), sizeof(int2) * tiles.size(),
-                           hipMemcpyHostToDevice, st),
-            "upload tiles");
+  if (!tiles.empty())
+    check_hip(hipMemcpyAsync(f->start_tiles, tiles.data(), sizeof(int2) * tiles.size(),
+                             hipMemcpyHostToDevice, st),
+              "upload tiles");
   for (int i = 0; i < n; i++) {
     const StartArg &a = args[i];
     check_hip(hipMemcpyAsync(w.h + (size_t)vals[i].row0 * H, a.prefill, sizeof(float) * a.rows * H,
@@ -1240,8 +1244,9 @@ void start_group(q3h_frame *f, const StartArg *args, int n, std::vector<StartPro
   }
   hipLaunchKernelGGL(k_start_prep, dim3(n), dim3(256), 0, st, f->start_prompts, w.rd);
   LayerIO io;
-  io.tiles = f->start_tiles;
+  io.tiles = tr > 0 ? f->start_tiles : nullptr;
   io.n_tiles = (int)tiles.size();
+  io.tile_rows = tr;
   run_layers(s, w, M, longest, false, st, io);
   const Mat &head = s->heads[c.talker_head];
   if (s->cfg.act_q8) {

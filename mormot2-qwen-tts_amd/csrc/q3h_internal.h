@@ -236,11 +236,11 @@ struct AttnArgs {
   float *out;    // [M][heads * head_dim]
   float *part;   // [M][heads][attn_splits slots][head_dim + 2]
   int layers;    // > layer + 1: a decode launch also loads layer + 1's cache rows ahead
-  // launch_attn_prefill over several contexts' rows: its tiles of queries
-  // (x: first row, y: rows, consecutive positions of one context), n_tiles of
-  // them; null: M rows of one context
+  // launch_attn_prefill and launch_attn_x_prompt over several contexts' rows:
+  // their tiles of up to tile_rows queries (x: first row, y: rows, consecutive
+  // positions of one context), n_tiles of them; null: M rows of one context
   const int2 *tiles;
-  int n_tiles;
+  int n_tiles, tile_rows;
 };
 // rows per query tile of launch_attn_prefill
 constexpr int kPrefillTile = 16;
@@ -296,6 +296,14 @@ bool attn_x_supported(int heads, int kvh, int head_dim, int max_positions);
 bool attn_x_pairs_supported(int max_positions);
 void launch_attn_x(const AttnArgs &a, int M, bool fused, bool kv16, int qkv_chunks,
                    const QAct &xa, int max_positions, hipStream_t st, bool pairs = false);
+// the rows of one context, or of the contexts of a.tiles (of attn_x_tile_rows
+// rows, for the M rows and the longest context), their K/V appended and q
+// normed and rotated, by the kernel that shares the keys and values between
+// rows; positions: the most any row attends to. false (nothing launched) where
+// attn_x_tile_rows is 0
+int attn_x_tile_rows(int heads, int kvh, int M, int positions);
+bool launch_attn_x_prompt(const AttnArgs &a, int M, int positions, bool kv16, const QAct &xa,
+                          hipStream_t st);
 
 // the code predictor's fused attention + o_proj (q3h_cp.hip): one context
 // of 16 positions, the new row at pos; k_layer: the layer's keys, values at

@@ -217,6 +217,31 @@ def test_int8_frame_32_streams_long_prompts(device, synth):
         m.destroy()
 
 
+@pytest.mark.parametrize("heads, kvh, kv16", [(4, 4, 0), (4, 2, 1), (4, 1, 0), (4, 1, 1)])
+def test_int8_prompt_attention_tiles(device, q3h, q3o, synth, heads, kvh, kv16):
+    """The prompt attention (k_attn_xp) at 1, 2 and 4 query heads per kv head
+    and both cache types: a first prompt of 21 rows (a last tile of one to five
+    rows), 8 rows and 64 rows onto it (positions past one 64-key block), then 9
+    rows onto 93 positions, which k_attn_x takes."""
+    print(f"case heads={heads} kvh={kvh} kv16={kv16}", flush=True)
+    dims = dict(synth.TALKER, layers=2, heads=heads, kv_heads=kvh, intermediate=1536)
+    layers, final = synth.stack_weights(37, "s.", dims, norm_std=0.1, quantize=q3o.quantize_q8_0)
+    s = q3h.Stack(device, dict(dims, dtype=q3h.Q8_0, kv_f16=kv16, act_q8=1, max_positions=128),
+                  layers, final, q3h.Q8_0)
+    o = q3o.Stack(dims, layers, final, q3o.Q8_0, kv_f16=kv16, act_q8=1)
+    ctx, octx = q3h.Context(s, 128), q3o.Ctx(o, 128)
+    try:
+        for i, rows in enumerate((21, 8, 64, 9)):
+            x = synth.prompt(60 + i, rows)
+            _, st = ctx.forward(x)
+            assert np.array_equal(st, octx.forward(x)), (rows, heads, kvh, kv16)
+    finally:
+        ctx.destroy()
+        octx.destroy()
+        s.destroy()
+        o.destroy()
+
+
 @pytest.fixture(scope="module")
 def small8h(device):
     """The int8 path with half-float K/V caches (the reference's KvF16,
