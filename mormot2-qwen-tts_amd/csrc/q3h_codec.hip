@@ -8,15 +8,18 @@
 //
 // Every convolution (transposed ones included, rewritten as causal
 // convolutions of taps K / stride whose stride x out output columns are the
-// stride output rows) is one f32 matrix-core product over an implicit
-// im2col: output row t reads input rows t + k dil, k < taps, of a sequence
-// buffer that holds the `past` history rows of the previous call on top of
-// the new rows (TQwenVkSeq, codec.vulkan.pas:33-40). A workgroup owns 64
-// output rows x 16 WN output columns and walks the whole K = taps x Cin in
-// 32-column chunks (activations through double-buffered LDS, weights in
-// registers one chunk ahead): the order of every sum depends only on the
-// layer, not on the rows of the call, so decoding 1 + 3 frames or 4 at once
-// gives the same samples (the reference's property, codec.vulkan.pas:12-13).
+// stride output rows) is one matrix-core product over an implicit im2col:
+// output row t reads input rows t + k dil, k < taps, of a sequence buffer that
+// holds the `past` history rows of the previous call on top of the new rows
+// (TQwenVkSeq, codec.vulkan.pas:33-40). The f32 operands are split exactly into
+// bf16 parts (q3h_x3.h). The columns of a product are walked in units of 32
+// channels x all taps, so a unit's rows are staged once for its taps, in slices
+// of a few units that are summed alone and then in order: the order of every
+// sum depends only on the layer, not on the rows of the call, so decoding 1 + 3
+// frames or 4 at once gives the same samples (the reference's property,
+// codec.vulkan.pas:12-13). Measured (156 frames in passes of 16; one frame per
+// call): 14.3 ms and 698 us with f32 MFMAs, partial sums of every 16 chunks
+// through memory and sinf epilogues, 9.3 ms and 398 us.
 //
 // The elementwise steps ride in the products' epilogues: bias, GELU (erf),
 // the residual add, the ConvNeXt layer scale, and SnakeBeta of the output
@@ -29,9 +32,11 @@
 #include <algorithm>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "q3h_api_internal.h"
+#include "q3h_x3.h"
 
 namespace q3h {
 namespace {
@@ -42,236 +47,204 @@ constexpr int kDils[3] = {1, 3, 9};
 
 enum ConvEpi { CE_BIAS = 0, CE_GELU = 1, CE_RES = 2, CE_SCALED_RES = 3 };
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
-
 struct ConvArgs {
   const float *x;  // sequence buffer [past + T][cin] (history rows first)
-  const float *w;  // [n][taps cin], column k cin + c
+  const void *w;   // operand tiles (x3, or f32) of [n][taps cin], column 32 (u taps + k) + c % 32
+                   // for channel c of unit u = c / 32 at tap k
   const float *b;  // [n]
   float *y;        // [T][n] or null
   const float *r;  // residual [T][n] (CE_RES, CE_SCALED_RES)
   const float *g;  // layer scale [n] (CE_SCALED_RES)
   float *z;        // SnakeBeta of the output [T][n] or null
   const float *sa, *sib;  // e^alpha, 1 / (e^beta + 1e-9), indexed by column % sc
-  float *part;            // K-slice sums [gridDim.z][T][n] when the K walk is split
-  int cin, taps, dil, T, n, sc;
+  float *part;            // slice sums [slices][T][n] when the walk is split over workgroups
+  int sc;
 };
 
-// chunks of 32 K columns per K slice: a product whose K walk is longer runs
-// as ceil(chunks / kSliceChunks) slices, summed in slice order by
-// k_conv_reduce (a fixed split per layer: the sums do not depend on T)
-constexpr int kSliceChunks = 16;
-constexpr int kRingWorkgroups = 512;  // launches up to this size take k_conv_gemm_ring
-
-// the epilogue of one output: bias, GELU / residual / layer scale, then the
-// stores (y, and SnakeBeta of the value to z)
-template <int EPI>
-__device__ __forceinline__ void conv_out(const ConvArgs &a, int m, int n, float acc) {
-  const size_t o = (size_t)m * a.n + n;
-  float v = acc + a.b[n];
-  if (EPI == CE_GELU) v = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
-  if (EPI == CE_RES) v = a.r[o] + v;
-  if (EPI == CE_SCALED_RES) v = a.r[o] + a.g[n] * v;
-  if (a.y) a.y[o] = v;
-  if (a.z) {
-    const int sc = n % a.sc;
-    const float s = sinf(v * a.sa[sc]);
-    a.z[o] = v + a.sib[sc] * (s * s);
-  }
+__device__ __forceinline__ float gelu(float v) {
+  return 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
 }
 
-// one workgroup: output rows m0 .. m0 + 16 TM - 1, columns n0 .. n0 + 16 WN
-// - 1 (the row tile follows T; every output's sum has the same order in any
-// tile: a sum of the same MFMAs over the same chunks)
-template <int WN, int TM, int EPI>
-__global__ __launch_bounds__(64 * WN) void k_conv_gemm(ConvArgs a) {
-  constexpr int NT = 64 * WN, XS = 36, MR = 16 * TM;
-  constexpr int NF4 = MR * 32 / 4;                  // float4 of an activation chunk
-  constexpr int XF4 = NF4 >= NT ? NF4 / NT : 1;     // per thread
-  __shared__ float xs[2][MR * XS];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+// SnakeBeta of v: v + sin(v e^alpha)^2 / (e^beta + 1e-9)
+__device__ __forceinline__ float snake(float v, float sa, float sib) {
+  return fmaf(sib, sin_squared(__fmul_rn(v, sa)), v);
+}
+
+// One workgroup: output rows m0 .. m0 + 16 MT - 1, columns n0 .. n0 + 16 NT WN
+// - 1 (NT 16-column tiles per wave), on the bf16 matrix cores with both
+// operands split exactly (X3Walk). The units of a layer are summed in fixed
+// slices of su units, each alone and then in slice order, by
+//  - CM_WALK: one set of waves, slice after slice;
+//  - CM_GROUP: a set of waves per slice, their sums met in LDS;
+//  - CM_PART: a workgroup per slice (blockIdx.z), its sums to a.part for
+//    k_conv_reduce.
+// Every output's sum has the same order in any tile and mode.
+enum ConvMode { CM_WALK = 0, CM_GROUP = 1, CM_PART = 2 };
+
+// SU > 0: one slice of at most SU units over one 16-row tile (X3Short), any mode.
+template <int MT, int NT, int WN, int SG, int TAPS, bool WF32, int MODE, int SU>
+struct ConvWalk {
+  static constexpr int kHalo = (TAPS - 1) * (TAPS == 7 ? 9 : 1);  // (the largest dilation)
+  using Walk = X3Walk<MT, NT, WN, TAPS, kHalo, WF32>;
+  using Short = X3Short<WN, TAPS, kHalo, SU ? SU : 1, WF32>;
+  static_assert(SU == 0 || (MT == 1 && NT == 1), "short slices: one tile per wave");
+  static constexpr int kLds = SU ? Short::kLds : Walk::kLds;
+  static constexpr int kWords = Walk::kWords;
+};
+
+template <int MT, int NT, int WN, int SG, int TAPS, bool WF32, int MODE, int SU>
+__global__ __launch_bounds__(64 * WN * SG, SG > 2 ? 4 : 2) void k_conv_x3(
+    const float *__restrict__ x, const void *__restrict__ w, int cin, int dil, int T, int n, int su,
+    int epi, ConvArgs a) {
+  using W = ConvWalk<MT, NT, WN, SG, TAPS, WF32, MODE, SU>;
+  constexpr int kGroup = 64 * WN;
+  constexpr int kSum = MT * NT * WN * 256;  // floats of a group's sums
+  extern __shared__ uint16_t xs[];          // [SG][W::kLds]; then the groups' sums
+  const int grp = SG > 1 ? threadIdx.x / kGroup : 0, t = threadIdx.x - grp * kGroup;
+  const int lane = t & 63, wave = t >> 6;
+  const int n0 = (blockIdx.x * WN + wave) * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const int U = cin / 32;
+  const int sl = MODE == CM_PART ? blockIdx.z : grp;
+  const int u0 = MODE == CM_WALK ? 0 : sl * su, u1 = MODE == CM_WALK ? U : min(U, u0 + su);
+  const size_t ts = (size_t)U * TAPS * W::kWords;  // 16-byte words of a weight tile
+  const x3_u4 *wt = reinterpret_cast<const x3_u4 *>(w) + (size_t)(n0 >> 4) * ts + lane;
+  x3_v4f acc[NT][MT];
+  const float *xt = x + (size_t)m0 * cin;
+  const int rmax = T - 1 - m0 + (TAPS - 1) * dil;
+  if constexpr (SU > 0) {
+    acc[0][0] = W::Short::run(xt, cin, rmax, dil, wt, t, u0, u1, xs + grp * W::kLds);
+    if (MODE == CM_GROUP) __syncthreads();
+  } else {
+    x3_v4f tot[NT][MT];
+    W::Walk::template run<MODE == CM_WALK>(xt, cin, rmax, dil, wt, ts, t, u0, u1,
+                                           MODE == CM_WALK ? U : su, su, xs + grp * W::kLds, acc,
+                                           tot);
+  }
   const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * WN + 16 * wave, m0 = blockIdx.y * MR;
-  const int K = a.taps * a.cin, cpk = a.cin / 32;
-  const int q0 = blockIdx.z * kSliceChunks, q1 = min(a.taps * cpk, q0 + kSliceChunks);
-  const float *wr = a.w + (size_t)min(n0 + r, a.n - 1) * K + 4 * g;
-  int xrow[XF4], xcol[XF4], xo[XF4];
-  const bool xact = NF4 >= NT || t < NF4;  // threads that move activations
+  if constexpr (MODE == CM_PART) {
 #pragma unroll
-  for (int i = 0; i < XF4; i++) {
-    const int f = min(t + NT * i, NF4 - 1), row = f >> 3, c4 = f & 7;
-    xrow[i] = min(m0 + row, a.T - 1);
-    xcol[i] = 4 * c4;
-    xo[i] = row * XS + 4 * c4;
-  }
-  float4 xn[XF4], wn[2], wc[2];
-  auto load = [&](int q) {
-    const int k = q / cpk, c0 = (q - k * cpk) * 32;
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-    for (int i = 0; i < XF4; i++)
-      xn[i] = ld4(a.x + (size_t)(xrow[i] + k * a.dil) * a.cin + c0 + xcol[i]);
-    wn[0] = ld4(wr + 32 * q);
-    wn[1] = ld4(wr + 32 * q + 16);
-  };
-  v4f acc[TM];
+      for (int q = 0; q < 4; q++) {
+        const int m = m0 + 16 * i + 4 * g + q;
+        if (m >= T) continue;
 #pragma unroll
-  for (int i = 0; i < TM; i++) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
-  load(q0);
-  if (xact)
-#pragma unroll
-    for (int i = 0; i < XF4; i++) *reinterpret_cast<float4 *>(&xs[0][xo[i]]) = xn[i];
-  wc[0] = wn[0];
-  wc[1] = wn[1];
-  __syncthreads();
-  for (int q = q0; q < q1; q++) {
-    const int b = (q - q0) & 1;
-    if (q + 1 < q1) load(q + 1);
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-#pragma unroll
-      for (int tm = 0; tm < TM; tm++) {
-        const float4 xa = *reinterpret_cast<const float4 *>(&xs[b][(16 * tm + r) * XS + 16 * s + 4 * g]);
-        acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.x, wc[s].x, acc[tm], 0, 0, 0);
-        acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.y, wc[s].y, acc[tm], 0, 0, 0);
-        acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.z, wc[s].z, acc[tm], 0, 0, 0);
-        acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.w, wc[s].w, acc[tm], 0, 0, 0);
+        for (int j = 0; j < NT; j++)
+          a.part[((size_t)blockIdx.z * T + m) * n + n0 + 16 * j + r] = acc[j][i][q];
       }
-    }
-    if (q + 1 < q1) {
-      if (xact)
-#pragma unroll
-        for (int i = 0; i < XF4; i++) *reinterpret_cast<float4 *>(&xs[b ^ 1][xo[i]]) = xn[i];
-      wc[0] = wn[0];
-      wc[1] = wn[1];
-    }
-    __syncthreads();
+    return;
   }
-  // lane l holds (m = m0 + 16 tm + 4 g + q, n = n0 + r)
-  const int n = n0 + r;
-  if (n >= a.n) return;
+  if constexpr (MODE == CM_GROUP) {
+    // (the walk ended with a barrier: the staged rows are read)
+    x3_v4f *ps = reinterpret_cast<x3_v4f *>(xs);
+    if (grp > 0)
 #pragma unroll
-  for (int tm = 0; tm < TM; tm++)
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+          ps[(grp - 1) * (kSum / 4) + (j * MT + i) * kGroup + t] = acc[j][i];
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int s = 1; s < SG; s++)
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+          acc[j][i] = acc[j][i] + ps[(s - 1) * (kSum / 4) + (j * MT + i) * kGroup + t];
+  }
+  // the epilogue: the residuals of all outputs are loaded together, before
+  // anything is stored (a load behind a store to memory that could be the same
+  // waits for it: 16 us of an epilogue at one frame were such waits)
+  float rs[MT][4][NT], bias[NT], sa[NT], sib[NT], gs[NT];
+  const bool snk = a.z != nullptr;
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+    const int nc = n0 + 16 * j + r;
+    bias[j] = a.b[nc];
+    sa[j] = snk ? a.sa[nc % a.sc] : 0.f;
+    sib[j] = snk ? a.sib[nc % a.sc] : 0.f;
+    gs[j] = epi == CE_SCALED_RES ? a.g[nc] : 0.f;
+  }
+  if (epi >= CE_RES) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          rs[i][q][j] = a.r[(size_t)min(m0 + 16 * i + 4 * g + q, T - 1) * n + n0 + 16 * j + r];
+  }
+#pragma unroll
+  for (int i = 0; i < MT; i++)
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      const int m = m0 + 16 * tm + 4 * g + q;
-      if (m >= a.T) continue;
-      if (gridDim.z > 1)
-        a.part[((size_t)blockIdx.z * a.T + m) * a.n + n] = acc[tm][q];
-      else
-        conv_out<EPI>(a, m, n, acc[tm][q]);
-    }
-}
-
-// k_conv_gemm for launches of few workgroups (a frame per call), where the
-// serial K walk is the time: the same tile and sums, the chunks of the slice
-// walked with the loads of D chunks in flight (a register ring,
-// the loop unrolled over the kSliceChunks chunks a slice can hold, loads at
-// clamped chunk indices so that none sits behind a branch); chunk i's
-// activations go through LDS buffer i & 1. The operands the loads need come
-// as plain arguments (preloaded in SGPRs); the epilogue's in a.
-template <int WN, int TM, int EPI>
-__global__ __launch_bounds__(64 * WN) void k_conv_gemm_ring(const float *__restrict__ x,
-                                                       const float *__restrict__ w, int cin,
-                                                       int taps, int dil, int T, int n,
-                                                       ConvArgs a) {
-  constexpr int NT = 64 * WN, XS = 36, MR = 16 * TM, D = 4;
-  constexpr int NF4 = MR * 32 / 4;                  // float4 of an activation chunk
-  constexpr int XF4 = NF4 >= NT ? NF4 / NT : 1;     // per thread
-  __shared__ float xs[2][MR * XS];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * WN + 16 * wave, m0 = blockIdx.y * MR;
-  const int K = taps * cin, cpk = cin / 32;
-  const int q0 = blockIdx.z * kSliceChunks, nq = min(taps * cpk - q0, kSliceChunks);
-  const float *wr = w + (size_t)min(n0 + r, n - 1) * K + 4 * g;
-  int xrow[XF4], xcol[XF4], xo[XF4];
-  const bool xact = NF4 >= NT || t < NF4;  // threads that move activations
+      const int m = m0 + 16 * i + 4 * g + q;
+      float v[NT], z[NT];
 #pragma unroll
-  for (int i = 0; i < XF4; i++) {
-    const int f = min(t + NT * i, NF4 - 1), row = f >> 3, c4 = f & 7;
-    xrow[i] = min(m0 + row, T - 1);
-    xcol[i] = 4 * c4;
-    xo[i] = row * XS + 4 * c4;
-  }
-  float4 xn[D][XF4], wn[D][2];
-  // chunk q0 + i (clamped to the slice's last) into ring slot i % D
-  auto load = [&](int i) {
-    const int q = q0 + min(i, nq - 1), k = q / cpk, c0 = (q - k * cpk) * 32, sl = i % D;
+      for (int j = 0; j < NT; j++) {
+        v[j] = __fadd_rn(acc[j][i][q], bias[j]);
+        // GELU and the layer scale: ConvNeXt's layers, which are never walked
+        if (MODE != CM_WALK && epi == CE_GELU) v[j] = gelu(v[j]);
+        if (MODE != CM_WALK && epi == CE_SCALED_RES) v[j] = fmaf(gs[j], v[j], rs[i][q][j]);
+        if (epi == CE_RES) v[j] = __fadd_rn(rs[i][q][j], v[j]);
+        z[j] = snk ? snake(v[j], sa[j], sib[j]) : 0.f;
+      }
+      if (m < T) {
+        const size_t o = (size_t)m * n + n0 + r;
 #pragma unroll
-    for (int j = 0; j < XF4; j++)
-      xn[sl][j] = ld4(x + (size_t)(xrow[j] + k * dil) * cin + c0 + xcol[j]);
-    wn[sl][0] = ld4(wr + 32 * q);
-    wn[sl][1] = ld4(wr + 32 * q + 16);
-  };
-  v4f acc[TM];
-#pragma unroll
-  for (int i = 0; i < TM; i++) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < D; i++) load(i);
-  if (xact)
-#pragma unroll
-    for (int j = 0; j < XF4; j++) *reinterpret_cast<float4 *>(&xs[0][xo[j]]) = xn[0][j];
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kSliceChunks; i++) {
-    const int b = i & 1, sl = i % D, sn = (i + 1) % D;
-    const float4 wc[2] = {wn[sl][0], wn[sl][1]};
-    // chunk i + 1's activations to the other buffer, then chunk i + D's loads
-    // into the slot chunk i leaves
-    if (xact)
-#pragma unroll
-      for (int j = 0; j < XF4; j++) *reinterpret_cast<float4 *>(&xs[b ^ 1][xo[j]]) = xn[sn][j];
-    load(i + D);
-    if (i < nq) {
-      // the chunk's activation operands read from LDS before the MFMAs
-      float4 xa[2][TM];
-#pragma unroll
-      for (int s = 0; s < 2; s++)
-#pragma unroll
-        for (int tm = 0; tm < TM; tm++)
-          xa[s][tm] =
-              *reinterpret_cast<const float4 *>(&xs[b][(16 * tm + r) * XS + 16 * s + 4 * g]);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-#pragma unroll
-        for (int tm = 0; tm < TM; tm++) {
-          acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[s][tm].x, wc[s].x, acc[tm], 0, 0, 0);
-          acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[s][tm].y, wc[s].y, acc[tm], 0, 0, 0);
-          acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[s][tm].z, wc[s].z, acc[tm], 0, 0, 0);
-          acc[tm] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[s][tm].w, wc[s].w, acc[tm], 0, 0, 0);
+        for (int j = 0; j < NT; j++) {
+          if (a.y) a.y[o + 16 * j] = v[j];
+          if (snk) a.z[o + 16 * j] = z[j];
         }
       }
     }
-    __syncthreads();
-  }
-  // lane l holds (m = m0 + 16 tm + 4 g + q, n = n0 + r)
-  const int nc = n0 + r;
-  if (nc >= n) return;
-#pragma unroll
-  for (int tm = 0; tm < TM; tm++)
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int m = m0 + 16 * tm + 4 * g + q;
-      if (m >= T) continue;
-      if (gridDim.z > 1)
-        a.part[((size_t)blockIdx.z * T + m) * n + nc] = acc[tm][q];
-      else
-        conv_out<EPI>(a, m, nc, acc[tm][q]);
-    }
 }
 
-// the slices of a split product added in slice order, then the epilogue
-template <int EPI>
-__global__ __launch_bounds__(256) void k_conv_reduce(ConvArgs a, int S) {
+// f32 weights [n][K] into operand tiles (split, or f32), one thread per 8
+__global__ __launch_bounds__(256) void k_conv_tiles(const float *__restrict__ f, int n, int K,
+                                                    void *__restrict__ o, bool f32) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)a.T * a.n) return;
-  const size_t plane = (size_t)a.T * a.n;
-  float v = a.part[i];
-  for (int s = 1; s < S; s++) v += a.part[s * plane + i];
-  conv_out<EPI>(a, (int)(i / a.n), (int)(i % a.n), v);
+  if (i >= (size_t)n * K / 8) return;
+  if (f32)
+    x3_f32_lane(f, n, K, i, static_cast<float *>(o));
+  else
+    x3_tile_lane(f, n, K, i, static_cast<uint16_t *>(o));
+}
+
+// The slices of a split product (up to 16 of them loaded together) added in
+// slice order, then the epilogue: bias, GELU / residual / layer scale, the
+// stores to y and (SnakeBeta of the value) to z.
+// (The operands of the first loads are plain arguments, preloaded in SGPRs.)
+__global__ __launch_bounds__(256) void k_conv_reduce(const float *__restrict__ part, int S,
+                                                     int plane, int n, int epi,
+                                                     const float *__restrict__ b,
+                                                     const float *__restrict__ rp, ConvArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= plane) return;
+  const int c = i % n;
+  const float bias = b[c];
+  const float res = epi >= CE_RES ? rp[i] : 0.f, g = epi == CE_SCALED_RES ? a.g[c] : 0.f;
+  float sa = 0.f, sib = 0.f;
+  if (a.z) {
+    sa = a.sa[c % a.sc];
+    sib = a.sib[c % a.sc];
+  }
+  float v = 0.f;
+  for (int s0 = 0; s0 < S; s0 += 16) {
+    float p[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) p[s] = part[(size_t)min(s0 + s, S - 1) * plane + i];
+#pragma unroll
+    for (int s = 0; s < 16; s++)
+      if (s0 + s < S) v = s0 + s ? __fadd_rn(v, p[s]) : p[s];
+  }
+  v = __fadd_rn(v, bias);
+  if (epi == CE_GELU) v = gelu(v);
+  if (epi == CE_RES) v = __fadd_rn(res, v);
+  if (epi == CE_SCALED_RES) v = fmaf(g, v, res);
+  if (a.y) a.y[i] = v;
+  if (a.z) a.z[i] = snake(v, sa, sib);
 }
 
 // ConvNeXt's causal depthwise convolution (kernel 7) and LayerNorm (eps 1e-6)
@@ -351,34 +324,26 @@ struct HistEntry {
   int past, cols, mult;  // rows of the pass = frames x mult
 };
 
-// One workgroup per sequence: rows T .. T + past - 1 move to 0 .. past - 1,
-// in blocks of min(T, past) rows from the top (a block never reads what an
-// earlier block wrote, nor what it writes itself).
-// (the loads of a block are all issued before its stores: up to 32 values
-// per thread, 8192 per block, more than any history holds)
-__global__ __launch_bounds__(256) void k_save_hist(const HistEntry *__restrict__ e, int frames) {
+// Rows T .. T + past - 1 move to 0 .. past - 1, a thread per 4 columns of a
+// sequence (blockIdx.x) walking the rows in order, 18 at a time (histories are
+// 1, 6, 18 or 54 rows): a batch is loaded whole before it is stored, and later
+// batches read rows below every row stored before them, so rows that are both
+// source and target (T < past) need no second buffer.
+__global__ __launch_bounds__(64) void k_save_hist(const HistEntry *__restrict__ e, int frames) {
   const HistEntry h = e[blockIdx.x];
-  const int T = frames * h.mult;
-  const int B = min(T, h.past);
+  const int T = frames * h.mult, c = (blockIdx.y * 64 + threadIdx.x) * 4;
+  if (c >= h.cols) return;
+  float *dst = global_ptr(h.buf) + c;
+  const float *src = dst + (size_t)T * h.cols;
+  constexpr int B = 18;
   for (int d0 = 0; d0 < h.past; d0 += B) {
-    const int rows = min(B, h.past - d0);
-    const int n = rows * h.cols;
-    float *dst = global_ptr(h.buf) + (size_t)d0 * h.cols;
-    const float *src = global_ptr(h.buf) + (size_t)(d0 + T) * h.cols;
-    for (int base = 0; base < n; base += 32 * 256) {
-      float v[32];
+    x3_v4f v[B];
 #pragma unroll
-      for (int j = 0; j < 32; j++) {
-        const int i = base + j * 256 + threadIdx.x;
-        v[j] = i < n ? src[i] : 0.f;
-      }
+    for (int j = 0; j < B; j++)
+      v[j] = *reinterpret_cast<const x3_v4f *>(src + (size_t)min(d0 + j, h.past - 1) * h.cols);
 #pragma unroll
-      for (int j = 0; j < 32; j++) {
-        const int i = base + j * 256 + threadIdx.x;
-        if (i < n) dst[i] = v[j];
-      }
-    }
-    __syncthreads();
+    for (int j = 0; j < B; j++)
+      if (d0 + j < h.past) *reinterpret_cast<x3_v4f *>(dst + (size_t)(d0 + j) * h.cols) = v[j];
   }
 }
 
@@ -391,7 +356,10 @@ namespace {
 
 // a convolution as the product kernels take it
 struct DConv {
-  float *w = nullptr, *b = nullptr;
+  void *w = nullptr;  // operand tiles: split, or f32
+  float *b = nullptr;
+  bool f32 = false;
+  int su = 1;  // units per slice
   int cin = 0, n = 0, taps = 1, dil = 1;
 };
 
@@ -424,6 +392,8 @@ struct q3h_codec {
   hipStream_t stream = nullptr;
   std::vector<void *> allocs;
   int64_t bytes = 0;
+  float *staging = nullptr;  // the weights of one layer as they are uploaded
+  size_t staging_floats = 0;
   DConv up[2];
   DNext next[2];
   DConv conv0;
@@ -460,28 +430,62 @@ float *upload_f(q3h_codec *c, const std::vector<float> &v) {
   return p;
 }
 
+// column of channel ch at tap k in the walk's order
+inline size_t walk_column(int ch, int k, int taps) {
+  return (size_t)((ch >> 5) * taps + k) * 32 + (ch & 31);
+}
+
+// A weight matrix v [n][taps cin], columns in the walk's order, as operand
+// tiles. Layers of 1 to 4 rows per frame (the front ones, most of the weights)
+// keep them as f32: a pass streams their weights once for at most a few row
+// tiles.
+void upload_tiles(q3h_codec *c, DConv &d, const std::vector<float> &v, bool front) {
+  const size_t bytes = (front ? 4 : 6) * v.size();
+  d.f32 = front;
+  d.w = dev_alloc(bytes);
+  c->allocs.push_back(d.w);
+  c->bytes += (int64_t)bytes;
+  if (c->staging_floats < v.size()) {
+    dev_free(c->staging);
+    c->staging = nullptr;
+    c->staging_floats = 0;
+    c->staging = (float *)dev_alloc(sizeof(float) * v.size());
+    c->staging_floats = v.size();
+  }
+  check_hip(hipMemcpyAsync(c->staging, v.data(), sizeof(float) * v.size(), hipMemcpyHostToDevice,
+                           c->stream),
+            "codec upload");
+  hipLaunchKernelGGL(k_conv_tiles, dim3((unsigned)((v.size() / 8 + 255) / 256)), dim3(256), 0,
+                     c->stream, c->staging, d.n, d.taps * d.cin, d.w, front);
+  check_hip(hipGetLastError(), "codec weight tiles");
+  check_hip(hipStreamSynchronize(c->stream), "codec weight tiles");
+  // units per slice: 6 to 14 chunks (a fixed split per layer)
+  const int U = d.cin / 32;
+  d.su = d.taps == 7 ? (U <= 3 ? 1 : 2) : (d.taps == 2 || U % 8 != 0 ? 6 : 8);
+}
+
 const float *need(const float *p, const char *what) {
   require(p != nullptr, Q3H_E_ARG, std::string("q3h_codec_create: NULL ") + what);
   return p;
 }
 
-// torch Conv1d weight [out][in][k] -> [out][k in + c]
+// torch Conv1d weight [out][in][k]
 DConv make_conv(q3h_codec *c, const float *w, const float *b, int cin, int out, int k, int dil,
-                const char *what) {
+                const char *what, bool front = false) {
   need(w, what);
   need(b, what);
   std::vector<float> wp((size_t)out * k * cin), bp(b, b + out);
   for (int o = 0; o < out; o++)
     for (int ch = 0; ch < cin; ch++)
       for (int j = 0; j < k; j++)
-        wp[(size_t)o * k * cin + (size_t)j * cin + ch] = w[((size_t)o * cin + ch) * k + j];
+        wp[(size_t)o * k * cin + walk_column(ch, j, k)] = w[((size_t)o * cin + ch) * k + j];
   DConv d;
-  d.w = upload_f(c, wp);
   d.b = upload_f(c, bp);
   d.cin = cin;
   d.n = out;
   d.taps = k;
   d.dil = dil;
+  upload_tiles(c, d, wp, front);
   return d;
 }
 
@@ -489,7 +493,7 @@ DConv make_conv(q3h_codec *c, const float *w, const float *b, int cin, int out, 
 // convolution of `taps` over [history ; x]: output column j out + o of row t
 // (the sample t stride + j), tap k reading input row t - (taps - 1 - k)
 DConv make_tconv(q3h_codec *c, const float *w, const float *b, int cin, int out, int K,
-                 int stride, const char *what) {
+                 int stride, const char *what, bool front = false) {
   need(w, what);
   need(b, what);
   const int taps = K / stride, n = stride * out;
@@ -500,23 +504,23 @@ DConv make_tconv(q3h_codec *c, const float *w, const float *b, int cin, int out,
       for (int k = 0; k < taps; k++) {
         const int i = taps - 1 - k;
         for (int ch = 0; ch < cin; ch++)
-          wp[((size_t)j * out + o) * taps * cin + (size_t)k * cin + ch] =
+          wp[((size_t)j * out + o) * taps * cin + walk_column(ch, k, taps)] =
               w[((size_t)ch * out + o) * K + j + i * stride];
       }
     }
   DConv d;
-  d.w = upload_f(c, wp);
   d.b = upload_f(c, bp);
   d.cin = cin;
   d.n = n;
   d.taps = taps;
   d.dil = 1;
+  upload_tiles(c, d, wp, front);
   return d;
 }
 
 DConv make_linear(q3h_codec *c, const float *w, const float *b, int cin, int out,
                   const char *what) {
-  return make_conv(c, w, b, cin, out, 1, 1, what);
+  return make_conv(c, w, b, cin, out, 1, 1, what, true);
 }
 
 DSnake make_snake(q3h_codec *c, const float *alpha, const float *beta, int n, const char *what) {
@@ -538,10 +542,113 @@ float *copy_vec(q3h_codec *c, const float *p, int n, const char *what) {
   return upload_f(c, std::vector<float>(p, p + n));
 }
 
-// the K slices of a layer's product (fixed per layer)
-int slices(const DConv &d) {
-  const int nch = d.taps * d.cin / 32;
-  return (nch + kSliceChunks - 1) / kSliceChunks;
+// the slices of a layer's product (fixed per layer)
+int slices(const DConv &d) { return (d.cin / 32 + d.su - 1) / d.su; }
+
+constexpr int kWalkWorkgroups = 256, kShortWorkgroups = 640;
+
+template <int MT, int NT, int WN, int SG, int TAPS, bool WF32, int MODE, int SU = 0>
+void conv_launch(q3h_codec *c, const DConv &d, const ConvArgs &a, int T, int epi, int S) {
+  using W = ConvWalk<MT, NT, WN, SG, TAPS, WF32, MODE, SU>;
+  const dim3 grid(d.n / (16 * NT * WN), (T + 16 * MT - 1) / (16 * MT), MODE == CM_PART ? S : 1);
+  const size_t lds = std::max(sizeof(uint16_t) * SG * W::kLds,
+                              sizeof(float) * (SG - 1) * MT * NT * WN * 256);
+  auto *k = &k_conv_x3<MT, NT, WN, SG, TAPS, WF32, MODE, SU>;
+  if (lds > (64 << 10))
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+              "codec LDS");
+  hipLaunchKernelGGL(k, grid, dim3(64 * WN * SG), lds, c->stream, a.x, a.w, d.cin, d.dil, T, d.n,
+                     d.su, epi, a);
+}
+
+// The modes of a layer of TAPS taps over T rows, nb its 16 WN-column blocks:
+// one 16-row tile per slice and workgroup while these are few (calls of a
+// frame, the front layers), the 2 to 4 slices of a layer as sets of waves of
+// one workgroup (no partial sums through memory, no second launch); else 64-
+// or 32-row tiles walked whole where they fill the chip, a workgroup per slice
+// otherwise.
+// (The kernels are built for the decoder's layers only: the front layers, f32
+// tiles, have 4 slices at one tap, more than 4 otherwise; the blocks' transposed
+// convolutions of two taps have 4, 2 and 1, their dilated convolutions 12, 6, 3
+// and 3, and their pointwise ones 3, 2, 1 and 1.)
+template <int WN, int TAPS, bool WF32, int SU>
+bool conv_short(q3h_codec *c, const DConv &d, const ConvArgs &a, int T, int epi, int S) {
+  const int tiles = (T + 15) / 16 * (d.n / (16 * WN));
+  if (d.su != SU || tiles * (S > 4 ? S : 1) > kShortWorkgroups) return false;
+  if constexpr (!WF32 && ((TAPS == 2 && WN == 3) || (TAPS == 1 && SU == 6)))
+    if (S == 1) {
+      conv_launch<1, 1, WN, 1, TAPS, WF32, CM_WALK, SU>(c, d, a, T, epi, S);
+      return true;
+    }
+  if constexpr (!WF32 && WN == 4 && (TAPS == 2 || (TAPS == 1 && SU == 6)))
+    if (S == 2) {
+      conv_launch<1, 1, WN, 2, TAPS, WF32, CM_GROUP, SU>(c, d, a, T, epi, S);
+      return true;
+    }
+  if constexpr (!WF32 && (TAPS == 7 || (TAPS == 1 && SU == 8)))
+    if (S == 3) {
+      conv_launch<1, 1, WN, 3, TAPS, WF32, CM_GROUP, SU>(c, d, a, T, epi, S);
+      return true;
+    }
+  if constexpr (WN == 4 && (WF32 ? TAPS == 1 : TAPS == 2))
+    if (S == 4) {
+      conv_launch<1, 1, WN, 4, TAPS, WF32, CM_GROUP, SU>(c, d, a, T, epi, S);
+      return true;
+    }
+  if constexpr (WN == 4 && (WF32 || (TAPS == 7 && SU == 2)))
+    if (S > 4) {
+      conv_launch<1, 1, WN, 1, TAPS, WF32, CM_PART, SU>(c, d, a, T, epi, S);
+      return true;
+    }
+  return false;
+}
+
+// The rule's lines, measured on the four dilated convolutions of a 16-frame
+// pass (us; columns per wave x rows per workgroup): n = 768, 512 rows: split
+// 16 x 64 29.7, 32 x 64 30.9; n = 384, 2560 rows: walked 16 x 32 35, 16 x 64
+// 43, split 32 x 64 30 + 6 for the reduction; n = 192, 10240 rows: walked 16 x
+// 64 32, 16 x 32 39, 32 x 64 45 (320 workgroups on 256 CUs); n = 96, 30720
+// rows: 32 x 64 (all columns) 26, 16 x 64 33. (With f32 MFMAs and partial sums
+// through memory: 47 + 8 each.)
+template <int WN, int TAPS, bool WF32>
+void conv_mode(q3h_codec *c, const DConv &d, const ConvArgs &a, int T, int epi) {
+  const int S = slices(d), r32 = (T + 31) / 32, r64 = (T + 63) / 64;
+  const int nb = d.n / (16 * WN);
+  bool done = false;
+  if constexpr (TAPS == 7)
+    done = conv_short<WN, TAPS, WF32, WN == 4 ? 2 : 1>(c, d, a, T, epi, S);
+  else if constexpr (TAPS == 2)
+    done = conv_short<WN, TAPS, WF32, 6>(c, d, a, T, epi, S);
+  else
+    done = (WN == 4 && conv_short<WN, TAPS, WF32, 8>(c, d, a, T, epi, S)) ||
+           (!WF32 && conv_short<WN, TAPS, false, 6>(c, d, a, T, epi, S));
+  if (done) {
+    if (S <= 4) return;
+  } else {
+    if constexpr (!WF32) {
+      if constexpr (WN == 3 && TAPS != 2)
+        if (nb == 2 && r64 >= kWalkWorkgroups) {  // the whole width in one workgroup
+          conv_launch<4, 2, WN, 1, TAPS, WF32, CM_WALK>(c, d, a, T, epi, S);
+          return;
+        }
+      if (r64 * nb >= 448) {
+        conv_launch<4, 1, WN, 1, TAPS, WF32, CM_WALK>(c, d, a, T, epi, S);
+        return;
+      }
+      if (TAPS != 7 || r32 * nb >= kWalkWorkgroups) {
+        conv_launch<2, 1, WN, 1, TAPS, WF32, CM_WALK>(c, d, a, T, epi, S);
+        return;
+      }
+    }
+    if constexpr (WN == 4 && (WF32 || TAPS == 7))
+      conv_launch<4, 1, WN, 1, TAPS, WF32, CM_PART>(c, d, a, T, epi, S);
+    else  // a layer of another shape
+      require(false, Q3H_E_ARG, "codec: layer shape");
+  }
+  const int plane = T * d.n;
+  hipLaunchKernelGGL(k_conv_reduce, dim3((plane + 255) / 256), dim3(256), 0, c->stream, a.part, S,
+                     plane, d.n, epi, a.b, a.r, a);
 }
 
 // y / z of a product over T output rows of sequence x
@@ -558,67 +665,26 @@ void conv(q3h_codec *c, const DConv &d, const float *x, int T, float *y, int epi
   a.z = z;
   a.sa = sn ? sn->a : nullptr;
   a.sib = sn ? sn->ib : nullptr;
-  a.cin = d.cin;
-  a.taps = d.taps;
-  a.dil = d.dil;
-  a.T = T;
-  a.n = d.n;
   a.sc = sc;
   a.part = c->part;
-  const int S = slices(d);
-  const int wn = d.n % 64 == 0 ? 4 : 2;
-  const int tm = T <= 16 ? 1 : (T <= 32 ? 2 : 4);
-  const dim3 grid(d.n / (16 * wn), (T + 16 * tm - 1) / (16 * tm), S);
-  // few workgroups: the deep load ring (a frame per call: 0.77 -> 0.68 ms per
-  // frame); the single-chunk lookahead otherwise (16-frame passes were 10-30 %
-  // slower on the ring)
-  const bool ring = (size_t)grid.x * grid.y * grid.z <= kRingWorkgroups;
-#define Q3H_C(WN, TM, E)                                                                     \
-  do {                                                                                       \
-    if (ring)                                                                                \
-      hipLaunchKernelGGL((k_conv_gemm_ring<WN, TM, E>), grid, dim3(64 * WN), 0, c->stream,   \
-                         a.x, a.w, a.cin, a.taps, a.dil, a.T, a.n, a);                       \
-    else                                                                                     \
-      hipLaunchKernelGGL((k_conv_gemm<WN, TM, E>), grid, dim3(64 * WN), 0, c->stream, a);    \
+  require(d.n % 64 == 0 || (d.n % 48 == 0 && !d.f32), Q3H_E_ARG, "codec: layer width");
+  const bool w4 = d.n % 64 == 0;
+#define Q3H_C(TAPS)                                  \
+  do {                                               \
+    if (d.f32)                                       \
+      conv_mode<4, TAPS, true>(c, d, a, T, epi);     \
+    else if (w4)                                     \
+      conv_mode<4, TAPS, false>(c, d, a, T, epi);    \
+    else                                             \
+      conv_mode<3, TAPS, false>(c, d, a, T, epi);    \
   } while (0)
-#define Q3H_E(WN, TM)                      \
-  do {                                     \
-    if (epi == CE_BIAS)                    \
-      Q3H_C(WN, TM, CE_BIAS);              \
-    else if (epi == CE_GELU)               \
-      Q3H_C(WN, TM, CE_GELU);              \
-    else if (epi == CE_RES)                \
-      Q3H_C(WN, TM, CE_RES);               \
-    else                                   \
-      Q3H_C(WN, TM, CE_SCALED_RES);        \
-  } while (0)
-#define Q3H_T(WN)         \
-  do {                    \
-    if (tm == 1)          \
-      Q3H_E(WN, 1);       \
-    else if (tm == 2)     \
-      Q3H_E(WN, 2);       \
-    else                  \
-      Q3H_E(WN, 4);       \
-  } while (0)
-  if (wn == 4)
-    Q3H_T(4);
+  if (d.taps == 1)
+    Q3H_C(1);
+  else if (d.taps == 2)
+    Q3H_C(2);
   else
-    Q3H_T(2);
-#undef Q3H_T
-#undef Q3H_E
+    Q3H_C(7);
 #undef Q3H_C
-  if (S > 1) {
-    const dim3 rg((unsigned)(((size_t)T * d.n + 255) / 256));
-    if (epi == CE_BIAS)
-      hipLaunchKernelGGL(k_conv_reduce<CE_BIAS>, rg, dim3(256), 0, c->stream, a, S);
-    else if (epi == CE_GELU)
-      hipLaunchKernelGGL(k_conv_reduce<CE_GELU>, rg, dim3(256), 0, c->stream, a, S);
-    else if (epi == CE_RES)
-      hipLaunchKernelGGL(k_conv_reduce<CE_RES>, rg, dim3(256), 0, c->stream, a, S);
-    else
-      hipLaunchKernelGGL(k_conv_reduce<CE_SCALED_RES>, rg, dim3(256), 0, c->stream, a, S);
-  }
 }
 
 // one pass of F <= max_frames frames: x already in c->x_in, pcm to c->pcm
@@ -673,8 +739,8 @@ void pass(q3h_codec *c, int F) {
   }
   hipLaunchKernelGGL(k_conv_out, dim3((rows + 63) / 64), dim3(256), 0, st, c->s_out, c->out_w,
                      c->out_b, rows, c->pcm);
-  hipLaunchKernelGGL(k_save_hist, dim3((unsigned)c->hist_host.size()), dim3(256), 0, st, c->hist,
-                     F);
+  hipLaunchKernelGGL(k_save_hist, dim3((unsigned)c->hist_host.size(), kDecDim / 256), dim3(64), 0, st,
+                     c->hist, F);
   check_hip(hipGetLastError(), "codec kernels");
 }
 
@@ -695,6 +761,7 @@ void codec_release(q3h_codec *c) {
   for (hipGraphExec_t e : c->exec)
     if (e) (void)hipGraphExecDestroy(e);
   for (void *p : c->allocs) dev_free(p);
+  dev_free(c->staging);
   if (c->stream) (void)hipStreamDestroy(c->stream);
 }
 
@@ -715,7 +782,7 @@ extern "C" int q3h_codec_create(q3h_device *dev, const q3h_codec_weights *w, int
     check_hip(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
     const int L = kLatent;
     for (int i = 0; i < 2; i++) {
-      c->up[i] = make_tconv(c, w->up_w[i], w->up_b[i], L, L, 2, 2, "upsample conv");
+      c->up[i] = make_tconv(c, w->up_w[i], w->up_b[i], L, L, 2, 2, "upsample conv", true);
       DNext &n = c->next[i];
       n.dw = copy_vec(c, w->dw_w[i], 7 * L, "dwconv weight");
       n.db = copy_vec(c, w->dw_b[i], L, "dwconv bias");
@@ -725,7 +792,8 @@ extern "C" int q3h_codec_create(q3h_device *dev, const q3h_codec_weights *w, int
       n.pw1 = make_linear(c, w->pw1_w[i], w->pw1_b[i], L, 4 * L, "pwconv1");
       n.pw2 = make_linear(c, w->pw2_w[i], w->pw2_b[i], 4 * L, L, "pwconv2");
     }
-    c->conv0 = make_conv(c, w->conv0_w, w->conv0_b, L, kDecDim, 7, 1, "decoder.0.conv");
+    c->conv0 = make_conv(c, w->conv0_w, w->conv0_b, L, kDecDim, 7, 1, "decoder.0.conv",
+                         true);
     for (int b = 0; b < 4; b++) {
       DBlock &B = c->blocks[b];
       const q3h_codec_block &bw = w->block[b];
@@ -733,7 +801,8 @@ extern "C" int q3h_codec_create(q3h_device *dev, const q3h_codec_weights *w, int
       B.cout = kDecDim >> (b + 1);
       B.rate = kRates[b];
       B.act = make_snake(c, bw.act_alpha, bw.act_beta, B.cin, "block snake");
-      B.up = make_tconv(c, bw.up_w, bw.up_b, B.cin, B.cout, 2 * B.rate, B.rate, "block conv");
+      B.up = make_tconv(c, bw.up_w, bw.up_b, B.cin, B.cout, 2 * B.rate, B.rate, "block conv",
+                        b == 0);
       for (int u = 0; u < 3; u++) {
         const q3h_codec_res &rw = bw.res[u];
         B.res[u].a1 = make_snake(c, rw.a1_alpha, rw.a1_beta, B.cout, "act1");
@@ -752,6 +821,9 @@ extern "C" int q3h_codec_create(q3h_device *dev, const q3h_codec_weights *w, int
       c->out_w = upload_f(c, ow);
       c->out_b = w->out_b[0];
     }
+    dev_free(c->staging);
+    c->staging = nullptr;
+    c->staging_floats = 0;
     // sequences and work buffers for max_frames frames
     const size_t F = max_frames;
     c->x_in = calloc_dev<float>(c, F * L);

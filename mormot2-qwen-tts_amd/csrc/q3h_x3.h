@@ -1,0 +1,317 @@
+// q3h_x3.h - f32 x f32 products on the bf16 matrix cores, exact to the fp32
+// rounding of the sums: the inner walk shared by the many-row products of f32
+// stacks and the decoder's convolutions.
+//
+// Each operand is split into three bf16 parts, x = hi + mid + lo exactly
+// (split3), and the six part products whose weight is at least 2^-16 of the
+// product are accumulated in fp32 (hi hi, hi mid, mid hi, hi lo, lo hi, mid
+// mid; a bf16 product is exact in fp32; the dropped three weigh below 2^-23
+// of the product).
+//
+// v_mfma_f32_16x16x32_bf16: lane l holds A[l % 16][8 (l / 16) .. + 7] and
+// B[8 (l / 16) .. + 7][l % 16] and receives D[4 (l / 16) + r][l % 16]. A is
+// 16 activation rows, B 16 weight rows. The weights come pre-split in operand
+// order (x3_tiles): [16-row tile][32-column chunk][part][lane][8], so an
+// operand is one coalesced 16-byte load per lane, straight to registers; the
+// activations are split as they go to LDS, shared by the workgroup's waves.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "q3h_math.h"
+
+namespace q3h {
+
+typedef float x3_v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 x3_bf8 __attribute__((ext_vector_type(8)));
+typedef unsigned int x3_u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kX3Stride = 40;  // LDS row of a unit, bf16 (32 + 8: 80 bytes)
+
+// weights f [N][K] row-major into the operand tiles x3 (3 N K bf16; N % 16 ==
+// 0, K % 32 == 0), or the same tiles unsplit (WF32): one thread per (tile,
+// chunk, lane)
+__device__ inline void x3_f32_lane(const float *f, int N, int K, size_t i, float *o) {
+  const int lane = i & 63, nq = K >> 5;
+  const size_t tq = i >> 6;
+  const float *s = f + ((tq / nq) * 16 + (lane & 15)) * K + 32 * (tq % nq) + 8 * (lane >> 4);
+  float *d = o + tq * 512 + lane * 4;
+  for (int e = 0; e < 4; e++) {
+    d[e] = s[e];
+    d[256 + e] = s[4 + e];
+  }
+}
+
+__device__ inline void x3_tile_lane(const float *f, int N, int K, size_t i, uint16_t *x3) {
+  const int lane = i & 63, nq = K >> 5;
+  const size_t tq = i >> 6;  // tile * nq + chunk
+  const int q = (int)(tq % nq), n = (int)(tq / nq) * 16 + (lane & 15);
+  const float *s = f + (size_t)n * K + 32 * q + 8 * (lane >> 4);
+  uint16_t *d = x3 + tq * 3 * 512 + lane * 8;
+  for (int e = 0; e < 8; e++) {
+    uint32_t h, m, l;
+    split3(s[e], h, m, l);
+    d[e] = (uint16_t)h;
+    d[512 + e] = (uint16_t)m;
+    d[1024 + e] = (uint16_t)l;
+  }
+}
+
+// The walk of WN waves over a product's columns: wave w owns NT 16-row weight
+// tiles, all share MT 16-row activation tiles; acc[j][i]: the sums of weight
+// tile j and activation tile i. The columns come in units of 32 channels of
+// TAPS taps (a dilated convolution; TAPS = 1: a plain product), chunk u TAPS +
+// k the channels of unit u at tap k, which reads the activation rows k dil
+// further down. A unit's rows (16 MT + (TAPS - 1) dil of them, up to HALO more
+// than the tile) are split and staged in LDS once for all its taps, in two
+// buffers with one barrier per unit; the rows are loaded up to three units
+// ahead of their use, the weights (registers) two chunks ahead. SUM: the units
+// come in slices of su; each slice is summed alone in acc from zero and added
+// to tot in order (what separate workgroups per slice and a reduction give).
+// WF32: the weights as f32 in the same tile order, split in registers (2 / 3 of
+// the bytes, for layers whose time is their weights' stream).
+template <int MT, int NT, int WN, int TAPS, int HALO, bool WF32>
+struct X3Walk {
+  static constexpr int kThreads = 64 * WN;
+  static constexpr int kRows = 16 * MT + HALO;
+  static constexpr int kXF4 = (kRows * 8 + kThreads - 1) / kThreads;  // float4 per thread
+  static constexpr int kPlane = kRows * kX3Stride;  // a part's plane in LDS
+  static constexpr int kLds = 2 * 3 * kPlane;       // uint16_t
+  static constexpr int kWords = WF32 ? 128 : 192;   // 16-byte words of a weight tile's chunk
+
+  // x: the tile's first row, channel 0 (row stride ld); rmax: its last row that
+  // exists; t: the thread among the WN waves; u0 .. u1 - 1: the units; nu: the
+  // barriers to take part in (units of the longest walk of the workgroup)
+  template <bool SUM>
+  static __device__ __forceinline__ void run(const float *__restrict__ x, int ld, int rmax, int dil,
+                                             const x3_u4 *__restrict__ wt, size_t tile_stride,
+                                             int t, int u0, int u1, int nu, int su, uint16_t *xs,
+                                             x3_v4f (&acc)[NT][MT], x3_v4f (&tot)[NT][MT]) {
+    const int lane = t & 63, r = lane & 15, g = lane >> 4;
+    const int q1 = u1 * TAPS;
+    int xo[kXF4];
+#pragma unroll
+    for (int i = 0; i < kXF4; i++) {
+      const int f = t + kThreads * i;
+      xo[i] = min(f >> 3, rmax) * ld + 4 * (f & 7);
+    }
+    float4 xr[2][kXF4];
+    x3_u4 w[2][NT][WF32 ? 2 : 3];
+    auto load_x = [&](int u, int s) {
+      const float *p = x + 32 * min(u, u1 - 1);
+#pragma unroll
+      for (int i = 0; i < kXF4; i++) xr[s][i] = *reinterpret_cast<const float4 *>(p + xo[i]);
+    };
+    auto load_w = [&](int q, int s) {
+      const x3_u4 *p = wt + (size_t)min(q, q1 - 1) * kWords;
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int k = 0; k < (WF32 ? 2 : 3); k++) w[s][j][k] = p[j * tile_stride + 64 * k];
+    };
+    auto stage = [&](int b, int s) {
+#pragma unroll
+      for (int i = 0; i < kXF4; i++) {
+        const int f = t + kThreads * i;
+        uint32_t h[4], m[4], l[4];
+        split3(xr[s][i].x, h[0], m[0], l[0]);
+        split3(xr[s][i].y, h[1], m[1], l[1]);
+        split3(xr[s][i].z, h[2], m[2], l[2]);
+        split3(xr[s][i].w, h[3], m[3], l[3]);
+        if (kRows * 8 % kThreads == 0 || f < kRows * 8) {
+          uint16_t *d = xs + b * 3 * kPlane + (f >> 3) * kX3Stride + 4 * (f & 7);
+          *reinterpret_cast<uint2 *>(d) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+          *reinterpret_cast<uint2 *>(d + kPlane) =
+              make_uint2(m[0] | (m[1] << 16), m[2] | (m[3] << 16));
+          *reinterpret_cast<uint2 *>(d + 2 * kPlane) =
+              make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+        }
+      }
+    };
+    auto unit = [&](int u, auto buf, auto par) {
+      constexpr int b = decltype(buf)::value, p0 = decltype(par)::value;
+#pragma unroll
+      for (int k = 0; k < TAPS; k++) {
+        constexpr int kParts = 3;
+        const int wb = (p0 + k) & 1;
+        x3_bf8 a[MT][kParts], bw[NT][kParts];
+        const uint16_t *s = xs + b * 3 * kPlane + (r + k * dil) * kX3Stride + 8 * g;
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+          for (int c = 0; c < kParts; c++)
+            a[i][c] = __builtin_bit_cast(
+                x3_bf8, *reinterpret_cast<const x3_u4 *>(s + c * kPlane + 16 * i * kX3Stride));
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+          if constexpr (WF32) {
+            x3_u4 part[3];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              uint32_t h0, m0, l0, h1, m1, l1;
+              split3(__uint_as_float(w[wb][j][e >> 1][2 * (e & 1)]), h0, m0, l0);
+              split3(__uint_as_float(w[wb][j][e >> 1][2 * (e & 1) + 1]), h1, m1, l1);
+              part[0][e] = h0 | (h1 << 16);
+              part[1][e] = m0 | (m1 << 16);
+              part[2][e] = l0 | (l1 << 16);
+            }
+#pragma unroll
+            for (int c = 0; c < kParts; c++) bw[j][c] = __builtin_bit_cast(x3_bf8, part[c]);
+          } else {
+#pragma unroll
+            for (int c = 0; c < kParts; c++) bw[j][c] = __builtin_bit_cast(x3_bf8, w[wb][j][c]);
+          }
+        }
+        // the small part products first; a part of every tile before the next
+        // part (independent sums back to back)
+        constexpr int pa[6] = {1, 2, 0, 1, 0, 0}, pb[6] = {1, 0, 2, 0, 1, 0};
+#pragma unroll
+        for (int c = 0; c < 6; c++)
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+              acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][pa[c]], bw[j][pb[c]],
+                                                                  acc[j][i], 0, 0, 0);
+        load_w(u * TAPS + k + 2, wb);
+      }
+      if (SUM && (u + 1 - u0) % su == 0) {
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int i = 0; i < MT; i++) {
+            tot[j][i] = u + 1 - u0 == su ? acc[j][i] : tot[j][i] + acc[j][i];
+            acc[j][i] = x3_v4f{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int i = 0; i < MT; i++) acc[j][i] = x3_v4f{0.f, 0.f, 0.f, 0.f};
+    load_x(u0, 0);
+    load_w(u0 * TAPS, 0);
+    load_x(u0 + 1, 1);
+    load_w(u0 * TAPS + 1, 1);
+    stage(0, 0);
+    load_x(u0 + 2, 0);
+    __syncthreads();
+    // unit u: its products from buffer u & 1, unit u + 1 staged in the other
+    for (int i = 0; i < nu; i += 2) {
+      const int u = u0 + i;
+      if (u < u1) unit(u, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+      stage(1, 1);
+      load_x(u + 3, 1);
+      __syncthreads();
+      if (i + 1 >= nu) break;
+      if (u + 1 < u1)
+        unit(u + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, TAPS & 1>{});
+      stage(0, 0);
+      load_x(u + 4, 0);
+      __syncthreads();
+    }
+    if (SUM) {
+      const int n = u1 - u0, last = n % su;
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+          acc[j][i] = last == 0 ? tot[j][i] : (n < su ? acc[j][i] : tot[j][i] + acc[j][i]);
+    }
+  }
+};
+
+// The same sums for one slice of at most SU units, one 16-row activation tile
+// and one 16-row weight tile per wave: the walk of calls of few rows, whose
+// time is the latency of its loads. The rows of all units are loaded and staged
+// at once, with one barrier, the first D chunks' weights in flight meanwhile.
+template <int WN, int TAPS, int HALO, int SU, bool WF32>
+struct X3Short {
+  static constexpr int kThreads = 64 * WN;
+  static constexpr int kRows = 16 + HALO;
+  static constexpr int kUnitF4 = kRows * 8;
+  static constexpr int kXF4 = (SU * kUnitF4 + kThreads - 1) / kThreads;
+  static constexpr int kPlane = kRows * kX3Stride;
+  static constexpr int kLds = SU * 3 * kPlane;  // uint16_t
+  static constexpr int kWords = WF32 ? 128 : 192;
+  static constexpr int NC = SU * TAPS;
+  static constexpr int D = NC < (WF32 ? 6 : 4) ? NC : (WF32 ? 6 : 4);
+
+  static __device__ __forceinline__ x3_v4f run(const float *__restrict__ x, int ld, int rmax,
+                                               int dil, const x3_u4 *__restrict__ wt, int t,
+                                               int u0, int u1, uint16_t *xs) {
+    const int lane = t & 63, r = lane & 15, g = lane >> 4, q1 = u1 * TAPS;
+    float4 xr[kXF4];
+    x3_u4 w[D][WF32 ? 2 : 3];
+    auto load_w = [&](int c) {
+      const x3_u4 *p = wt + (size_t)min(u0 * TAPS + c, q1 - 1) * kWords;
+#pragma unroll
+      for (int k = 0; k < (WF32 ? 2 : 3); k++) w[c % D][k] = p[64 * k];
+    };
+#pragma unroll
+    for (int i = 0; i < kXF4; i++) {
+      const int f = t + kThreads * i, u = f / kUnitF4, e = f - u * kUnitF4;
+      xr[i] = *reinterpret_cast<const float4 *>(x + (size_t)min(e >> 3, rmax) * ld +
+                                                32 * min(u0 + u, u1 - 1) + 4 * (e & 7));
+    }
+#pragma unroll
+    for (int c = 0; c < D; c++) load_w(c);
+#pragma unroll
+    for (int i = 0; i < kXF4; i++) {
+      const int f = t + kThreads * i, u = f / kUnitF4, e = f - u * kUnitF4;
+      uint32_t h[4], m[4], l[4];
+      split3(xr[i].x, h[0], m[0], l[0]);
+      split3(xr[i].y, h[1], m[1], l[1]);
+      split3(xr[i].z, h[2], m[2], l[2]);
+      split3(xr[i].w, h[3], m[3], l[3]);
+      if (SU * kUnitF4 % kThreads == 0 || f < SU * kUnitF4) {
+        uint16_t *d = xs + u * 3 * kPlane + (e >> 3) * kX3Stride + 4 * (e & 7);
+        *reinterpret_cast<uint2 *>(d) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+        *reinterpret_cast<uint2 *>(d + kPlane) = make_uint2(m[0] | (m[1] << 16), m[2] | (m[3] << 16));
+        *reinterpret_cast<uint2 *>(d + 2 * kPlane) =
+            make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+      }
+    }
+    __syncthreads();
+    x3_v4f acc = x3_v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      constexpr int pa[6] = {1, 2, 0, 1, 0, 0}, pb[6] = {1, 0, 2, 0, 1, 0};
+      const int u = c / TAPS, k = c % TAPS;
+      x3_bf8 a[3], bw[3];
+#pragma unroll
+      for (int e = 0; e < 3; e++)
+        a[e] = __builtin_bit_cast(x3_bf8, *reinterpret_cast<const x3_u4 *>(
+                                              xs + u * 3 * kPlane + e * kPlane +
+                                              (r + k * dil) * kX3Stride + 8 * g));
+      if constexpr (WF32) {
+        x3_u4 part[3];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          uint32_t h0, m0, l0, h1, m1, l1;
+          split3(__uint_as_float(w[c % D][e >> 1][2 * (e & 1)]), h0, m0, l0);
+          split3(__uint_as_float(w[c % D][e >> 1][2 * (e & 1) + 1]), h1, m1, l1);
+          part[0][e] = h0 | (h1 << 16);
+          part[1][e] = m0 | (m1 << 16);
+          part[2][e] = l0 | (l1 << 16);
+        }
+#pragma unroll
+        for (int e = 0; e < 3; e++) bw[e] = __builtin_bit_cast(x3_bf8, part[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; e++) bw[e] = __builtin_bit_cast(x3_bf8, w[c % D][e]);
+      }
+      if (c + D < NC) load_w(c + D);
+      x3_v4f n = acc;
+#pragma unroll
+      for (int e = 0; e < 6; e++)
+        n = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa[e]], bw[pb[e]], n, 0, 0, 0);
+      acc = u0 + u < u1 ? n : acc;
+    }
+    return acc;
+  }
+};
+
+}  // namespace q3h

@@ -53,6 +53,23 @@ def test_codec_chunks_give_the_same_samples(device, weights):
     assert np.array_equal(one, passes)
 
 
+@pytest.mark.parametrize("chunks, max_frames", [([17], 64), ([16, 1], 16), ([9, 8], 16),
+                                                ([5, 12], 16)])
+def test_codec_kernel_choice_keeps_the_samples(device, weights, chunks, max_frames):
+    """The products change their kernels with the rows of a call (one to a few
+    frames: slices in parallel; many: walked in one workgroup, 32- or 64-row
+    tiles; 64 frames: the widest of the front layers): 17 frames in calls on
+    both sides of those lines give the samples of 17 calls."""
+    x = synth.prompt(6, 17)
+    one = _gpu(device, weights, x, [1] * 17)
+    assert np.array_equal(one, _gpu(device, weights, x, chunks, max_frames))
+
+
+def test_codec_many_frames_in_one_pass(device, weights):
+    x = synth.prompt(7, 64)
+    assert np.array_equal(_gpu(device, weights, x, [64], 64), _gpu(device, weights, x, [64], 7))
+
+
 def test_codec_reset_and_errors(device, weights):
     x = synth.prompt(5, 2)
     c = q3h.Codec(device, weights, max_frames=4)
