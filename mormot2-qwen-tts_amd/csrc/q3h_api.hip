@@ -78,6 +78,9 @@ void work_fields(const q3h_stack *s, size_t R, int splits, int head_rows, Work &
     pn = std::max(pn, sr * (H / 256) * ldq);
     pn = std::max(pn, sr * std::min<size_t>(kMaxPartSlices, std::max(NQ, I) / 256) * H);
     each((void **)&w.gpart, sizeof(float) * pn);
+    const bool many = R > (size_t)kManyRows;
+    each((void **)&w.x3n, many ? x3_bytes(R, H) : 0);
+    each((void **)&w.x3a, many ? x3_bytes(R, std::max(NQ, I)) : 0);
   }
 }
 
@@ -121,6 +124,9 @@ void Work::release() {
   dev_free(xa.q);
   dev_free(xb.q);
   dev_free(gpart);
+  dev_free(x3n);
+  dev_free(x3a);
+  x3n = x3a = nullptr;
   xa = QAct{};
   xb = QAct{};
   gpart = nullptr;
@@ -154,6 +160,11 @@ void linear(const q3h_stack *s, Work &w, const Mat &W, const float *x, int ldx, 
       launch_rmsnorm_rows(x, ldx, M, W.K, norm_w, c.rms_eps, xn, W.K, st);
       x = xn;
       ldx = W.K;
+    }
+    if (M > kManyRows && epi == EPI_STORE && W.K == c.hidden && gemm_x3_supported(W, 1)) {
+      launch_x3_rows(x, ldx, M, W.K, w.x3n, st);
+      launch_gemm_x3(W, w.x3n, M, y, ldy, st);
+      return;
     }
     launch_gemm_f32(W, x, ldx, M, epi, y, ldy, st);
   } else {
@@ -257,6 +268,62 @@ bool f32_slice_path(const q3h_stack *s, int M) {
          gemm_f32_slices_supported(H, I);
 }
 
+// The same over more than kManyRows rows: every product's activations are
+// written as operand tiles by the kernel that makes them, and a row's result
+// does not depend on the other rows (prompts run together give the bits of
+// each alone).
+bool x3_path(const q3h_stack *s, int M) {
+  if (M <= kManyRows || !f32_slice_path(s, M)) return false;
+  const Layer &L = s->layers[0];
+  return gemm_x3_supported(L.qkv, 1) && gemm_x3_supported(L.gu, 1) &&
+         gemm_x3_supported(L.o, kF32Slices) && gemm_x3_supported(L.down, kF32Slices);
+}
+
+static void run_layers_x3(const q3h_stack *s, Work &w, int M, int positions, bool fused,
+                          const LayerIO &io, hipStream_t st) {
+  const q3h_stack_config &c = s->cfg;
+  const int H = c.hidden, hd = c.head_dim, NQ = c.heads * hd, NKV = c.kv_heads * hd;
+  const int ldq = NQ + 2 * NKV;
+  const bool kv16 = c.kv_f16 != 0;
+  const float eps = c.rms_eps;
+  launch_resid_norm(w.h, nullptr, M, H, s->layers[0].in_norm, eps, nullptr, 0, st, w.x3n);
+  for (int l = 0; l < c.layers; l++) {
+    const Layer &L = s->layers[l];
+    launch_gemm_x3(L.qkv, w.x3n, M, w.qkv, ldq, st);
+    if (!fused)
+      launch_qk_rope_append(w.qkv, ldq, w.rd, M, l, c.heads, c.kv_heads, hd, L.q_norm, L.k_norm,
+                            eps, s->rope_cs, kv16, st);
+    AttnArgs at{};
+    at.qkv = w.qkv;
+    at.ldq = ldq;
+    at.rd = w.rd;
+    at.layer = l;
+    at.heads = c.heads;
+    at.kvh = c.kv_heads;
+    at.qkn = L.q_norm;
+    at.rope_cs = reinterpret_cast<const float2 *>(s->rope_cs);
+    at.out = w.att;
+    at.part = w.part;
+    at.tiles = io.tiles;
+    at.n_tiles = io.n_tiles;
+    at.tile_rows = io.tile_rows;
+    if (!fused && (io.tiles || io.single_context)) {
+      at.out3 = w.x3a;
+      launch_attn_prefill(at, M, kv16, st);
+    } else {
+      launch_attn(at, M, positions, fused, kv16, st);
+      launch_x3_rows(w.att, NQ, M, NQ, w.x3a, st);
+    }
+    const int so = launch_gemm_x3_part(L.o, w.x3a, M, w.gpart, st);
+    launch_resid_norm(w.h, w.gpart, M, H, L.post_norm, eps, nullptr, so, st, w.x3n);
+    launch_gemm_x3_swiglu(L.gu, w.x3n, M, w.x3a, st);
+    const int sd = launch_gemm_x3_part(L.down, w.x3a, M, w.gpart, st);
+    const float *next = l + 1 < c.layers ? s->layers[l + 1].in_norm : nullptr;
+    launch_resid_norm(w.h, w.gpart, M, H, next, eps, nullptr, sd, st, w.x3n);
+    probe_layer(io, w, l, M, H, st);
+  }
+}
+
 static void run_layers_f32(const q3h_stack *s, Work &w, int M, int positions, bool fused,
                            const LayerIO &io, hipStream_t st) {
   const bool single_context = io.single_context;
@@ -291,9 +358,7 @@ static void run_layers_f32(const q3h_stack *s, Work &w, int M, int positions, bo
     at.rope_cs = reinterpret_cast<const float2 *>(s->rope_cs);
     at.out = w.att;
     at.part = w.part;
-    at.tiles = io.tiles;
-    at.n_tiles = io.n_tiles;
-    if (!fused && (io.tiles || (single_context && M >= kPrefillRows)))
+    if (!fused && single_context && M >= kPrefillRows)
       launch_attn_prefill(at, M, kv16, st);
     else
       launch_attn(at, M, positions, fused, kv16, st);
@@ -321,6 +386,10 @@ void run_layers(const q3h_stack *s, Work &w, int M, int positions, bool fused, h
   const bool kv16 = c.kv_f16 != 0;
   if (partial_path(s, M)) {
     run_layers_partial(s, w, M, positions, fused, io, st);
+    return;
+  }
+  if (x3_path(s, M)) {
+    run_layers_x3(s, w, M, positions, fused, io, st);
     return;
   }
   if (f32_slice_path(s, M)) {

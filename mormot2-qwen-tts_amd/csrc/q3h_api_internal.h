@@ -112,6 +112,9 @@ struct Work {
   CtxDev **ctx_arr = nullptr;
   QAct xa, xb;              // quantized activations (act_q8 stacks)
   float *gpart = nullptr;   // chunk partials of the int8 products (act_q8)
+  // operand tiles of the products over more than kManyRows rows (f32
+  // activations): the normed rows, and the attention / SwiGLU outputs
+  uint16_t *x3n = nullptr, *x3a = nullptr;
   void ensure(const struct ::q3h_stack *s, int rows, int splits, int head_rows);
   void release();
 };
@@ -175,8 +178,9 @@ struct LayerIO {
 // whether run_layers takes the int8 partial-product path for M rows of stack s
 bool partial_path(const struct ::q3h_stack *s, int M);
 
-// whether run_layers takes the sliced f32-activation path for M rows of stack s
-bool f32_slice_path(const struct ::q3h_stack *s, int M);
+// whether run_layers takes the path of products over split activations for M
+// rows of stack s (f32 activations, M > kManyRows)
+bool x3_path(const struct ::q3h_stack *s, int M);
 
 // fused: every row is the single new position of its own context; positions:
 // the most positions any row attends to (its own included), Work sized for

@@ -22,6 +22,7 @@
 #include "q3h_internal.h"
 #include "q3h_math.h"
 #include "q3h_wave.h"
+#include "q3h_x3.h"
 
 namespace q3h {
 
@@ -978,44 +979,57 @@ __device__ __forceinline__ v4f mfma_x3(const u32x4 (&a)[3], const u32x4 (&b)[3],
 //     eight keys in dims 16 t + l % 16;
 //   - the 4 waves' (max, sum, output) merged in LDS; each output element
 //     rescaled to the largest of the waves' maxima.
-template <typename KV, int GRP>
-__global__ __launch_bounds__(256) void k_attn_prefill_x3(const RowDesc *__restrict__ rd,
-                                                         const float *__restrict__ qkv, int ldq,
-                                                         int layer, int kvh, int M,
-                                                         float *__restrict__ outp,
-                                                         const int2 *__restrict__ tiles) {
-  __shared__ float ms[4][16], ls[4][16];
+// QT tiles of 16 queries per workgroup (2 where these still fill the chip):
+// the keys and values of a block are loaded and split once for all of them,
+// which is most of the kernel's instructions; the queries' split operands in
+// LDS.
+template <typename KV, int GRP, int QT>
+__global__ __launch_bounds__(256, 2) void k_attn_prefill_x3(const RowDesc *__restrict__ rd,
+                                                            const float *__restrict__ qkv, int ldq,
+                                                            int layer, int kvh, int M,
+                                                            float *__restrict__ outp,
+                                                            const int2 *__restrict__ tiles,
+                                                            uint16_t *__restrict__ out3) {
+  __shared__ float ms[QT][4][16], ls[QT][4][16];
   __shared__ float os[4][8][4][64];
+  __shared__ u32x4 qs[QT][4][3][64];
   // the tiles with the most keys first; a kv head's query heads on one XCD
   const int g = blockIdx.x % kvh, h = g * GRP + blockIdx.x / kvh;
-  const int2 tile = tiles ? tiles[blockIdx.y] : make_int2((gridDim.y - 1 - blockIdx.y) * 16, 16);
-  const int q0 = tile.x, nq = tiles ? tile.y : min(16, M - q0);
+  constexpr int R = 16 * QT;
+  const int2 tile = tiles ? tiles[blockIdx.y] : make_int2((gridDim.y - 1 - blockIdx.y) * R, R);
+  const int q0 = tile.x, nq = tiles ? tile.y : min(R, M - q0);
   const int heads = GRP * kvh;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r16 = lane & 15, gq = lane >> 4;
   const RowDesc d = rd[q0];
   const int p_hi = d.pos + nq - 1;  // the tile's last position
-  const int pq = d.pos + r16;       // this lane's query position
   const size_t head_off = ((size_t)layer * kvh + g) * d.max_pos * HD;
   const KV *kc = global_ptr(reinterpret_cast<const KV *>(d.k)) + head_off;
   const KV *vc = global_ptr(reinterpret_cast<const KV *>(d.v)) + head_off;
-  // this lane's query: row q0 + min(r16, nq - 1), dims 32 c + 8 gq .. + 7
-  u32x4 qp[4][3];
-  {
-    const float *qr = qkv + (size_t)(q0 + min(r16, nq - 1)) * ldq + h * HD + 8 * gq;
+  // queries: row q0 + min(16 j + r16, nq - 1), dims 32 c + 8 gq .. + 7, c = wave
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const float4 a = *reinterpret_cast<const float4 *>(qr + 32 * c);
-      const float4 b = *reinterpret_cast<const float4 *>(qr + 32 * c + 4);
-      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      split8(x, qp[c][0], qp[c][1], qp[c][2]);
-    }
+  for (int j = 0; j < QT; j++) {
+    const float *qr =
+        qkv + (size_t)(q0 + min(16 * j + r16, nq - 1)) * ldq + h * HD + 32 * wave + 8 * gq;
+    const float4 a = *reinterpret_cast<const float4 *>(qr);
+    const float4 b = *reinterpret_cast<const float4 *>(qr + 4);
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    u32x4 p[3];
+    split8(x, p[0], p[1], p[2]);
+#pragma unroll
+    for (int c = 0; c < 3; c++) qs[j][wave][c][lane] = p[c];
   }
+  __syncthreads();
   const float scale = (float)(1.0 / sqrt((double)HD));
-  float m_run = -INFINITY, l_run = 0.f;
-  v4f o[8];
+  float m_run[QT], l_run[QT];
+  v4f o[QT][8];
 #pragma unroll
-  for (int i = 0; i < 8; i++) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < QT; j++) {
+    m_run[j] = -INFINITY;
+    l_run[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) o[j][i] = v4f{0.f, 0.f, 0.f, 0.f};
+  }
   const int nblk = p_hi / 32 + 1;
   for (int b = wave; b < nblk; b += 4) {
     const int kb = 32 * b;
@@ -1031,91 +1045,136 @@ __global__ __launch_bounds__(256) void k_attn_prefill_x3(const RowDesc *__restri
         kf[hf][c][1] = ld4kv(kr + 32 * c + 4);
       }
     }
-    v4f sa[2];
+    v4f sa[QT][2];
 #pragma unroll
-    for (int hf = 0; hf < 2; hf++) {
-      sa[hf] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < QT; j++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
+      for (int hf = 0; hf < 2; hf++) sa[j][hf] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      u32x4 kp[2][3];
+#pragma unroll
+      for (int hf = 0; hf < 2; hf++) {
         const float x[8] = {kf[hf][c][0].x, kf[hf][c][0].y, kf[hf][c][0].z, kf[hf][c][0].w,
                             kf[hf][c][1].x, kf[hf][c][1].y, kf[hf][c][1].z, kf[hf][c][1].w};
-        u32x4 kp[3];
-        split8(x, kp[0], kp[1], kp[2]);
-        sa[hf] = mfma_x3(kp, qp[c], sa[hf]);
+        split8(x, kp[hf][0], kp[hf][1], kp[hf][2]);
+      }
+#pragma unroll
+      for (int j = 0; j < QT; j++) {
+        const u32x4 qp[3] = {qs[j][c][0][lane], qs[j][c][1][lane], qs[j][c][2][lane]};
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++) sa[j][hf] = mfma_x3(kp[hf], qp, sa[j][hf]);
       }
     }
     // the values, loaded once the keys are consumed (both in flight together
     // would take the registers of a second wave per SIMD)
-    float vv[8][8];
+    // (two query tiles: in two halves of the dims, for the registers)
+    constexpr int VH = QT > 1 ? 4 : 8;
+    float vv[VH][8];
+    auto load_v = [&](int i0) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int key = kb + (j < 4 ? 4 * gq + j : 16 + 4 * gq + j - 4);
-      const KV *vr = vc + (size_t)min(key, p_hi) * HD + r16;
+      for (int j = 0; j < 8; j++) {
+        const int key = kb + (j < 4 ? 4 * gq + j : 16 + 4 * gq + j - 4);
+        const KV *vr = vc + (size_t)min(key, p_hi) * HD + r16 + 16 * i0;
 #pragma unroll
-      for (int i = 0; i < 8; i++) vv[i][j] = (float)vr[16 * i];
-    }
-    float p[8], bm = -INFINITY;
+        for (int i = 0; i < VH; i++) vv[i][j] = (float)vr[16 * i];
+      }
+    };
+    load_v(0);
+    u32x4 pp[QT][3];
 #pragma unroll
-    for (int hf = 0; hf < 2; hf++)
+    for (int jq = 0; jq < QT; jq++) {
+      const int pq = d.pos + 16 * jq + r16;  // this lane's query position
+      float p[8], bm = -INFINITY;
+#pragma unroll
+      for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float s = kb + 16 * hf + 4 * gq + r <= pq ? sa[jq][hf][r] * scale : -INFINITY;
+          p[4 * hf + r] = s;
+          bm = fmaxf(bm, s);
+        }
+      bm = rows4_max(bm);
+      const float m_new = fmaxf(m_run[jq], bm);
+      const float ref = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = m_run[jq] == -INFINITY ? 0.f : __expf(m_run[jq] - ref);
+      float ps = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        p[j] = __expf(p[j] - ref);
+        ps += p[j];
+      }
+      ps = rows4_sum(ps);
+      l_run[jq] = fmaf(l_run[jq], alpha, ps);
+      m_run[jq] = m_new;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const float s = kb + 16 * hf + 4 * gq + r <= pq ? sa[hf][r] * scale : -INFINITY;
-        p[4 * hf + r] = s;
-        bm = fmaxf(bm, s);
+        const float ar = __shfl(alpha, 4 * gq + r);
+#pragma unroll
+        for (int i = 0; i < 8; i++) o[jq][i][r] *= ar;
       }
-    bm = rows4_max(bm);
-    const float m_new = fmaxf(m_run, bm);
-    const float ref = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = m_run == -INFINITY ? 0.f : __expf(m_run - ref);
-    float ps = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      p[j] = __expf(p[j] - ref);
-      ps += p[j];
+      split8(p, pp[jq][0], pp[jq][1], pp[jq][2]);
     }
-    ps = rows4_sum(ps);
-    l_run = fmaf(l_run, alpha, ps);
-    m_run = m_new;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const float ar = __shfl(alpha, 4 * gq + r);
+    for (int i0 = 0; i0 < 8; i0 += VH) {
+      if (i0) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(i0);
+      }
 #pragma unroll
-      for (int i = 0; i < 8; i++) o[i][r] *= ar;
-    }
-    u32x4 pp[3];
-    split8(p, pp[0], pp[1], pp[2]);
+      for (int i = 0; i < VH; i++) {
+        u32x4 vp[3];
+        split8(vv[i], vp[0], vp[1], vp[2]);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      u32x4 vp[3];
-      split8(vv[i], vp[0], vp[1], vp[2]);
-      o[i] = mfma_x3(pp, vp, o[i]);
+        for (int j = 0; j < QT; j++) o[j][i0 + i] = mfma_x3(pp[j], vp, o[j][i0 + i]);
+      }
     }
   }
-  if (gq == 0) {
-    ms[wave][r16] = m_run;
-    ls[wave][r16] = l_run;
-  }
 #pragma unroll
-  for (int i = 0; i < 8; i++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) os[wave][i][r][lane] = o[i][r];
-  __syncthreads();
-  // output (query q, dim k): tile i = k / 16, lane 16 (q / 4) + k % 16, r = q % 4
-  for (int e = t; e < 16 * HD; e += 256) {
-    const int q = e / HD, k = e % HD;
-    if (q >= nq) break;
-    const int i = k >> 4, l = 16 * (q >> 2) + (k & 15), r = q & 3;
-    float mx = ms[0][q];
-#pragma unroll
-    for (int w = 1; w < 4; w++) mx = fmaxf(mx, ms[w][q]);
-    float num = 0.f, den = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-      const float c = ms[w][q] == -INFINITY ? 0.f : __expf(ms[w][q] - mx);
-      num = fmaf(os[w][i][r][l], c, num);
-      den = fmaf(ls[w][q], c, den);
+  for (int j = 0; j < QT; j++)
+    if (gq == 0) {
+      ms[j][wave][r16] = m_run[j];
+      ls[j][wave][r16] = l_run[j];
     }
-    outp[(size_t)(q0 + q) * (heads * HD) + h * HD + k] = den > 0.f ? num / den : 0.f;
+  // output (query q, dims k .. k + 7): tile i = k / 16, lane 16 (q / 4) + k % 16,
+  // r = q % 4; a thread per 8 dims of a query, 16 queries at a time
+  static_assert(16 * HD == 8 * 256, "8 outputs per thread");
+#pragma unroll
+  for (int j = 0; j < QT; j++) {
+    if (j) __syncthreads();  // the outputs before are read
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) os[wave][i][r][lane] = o[j][i][r];
+    __syncthreads();
+    const int q = t >> 4, k0 = 8 * (t & 15), i = k0 >> 4, r = q & 3, row = 16 * j + q;
+    if (row < nq) {
+      float mx = ms[j][0][q];
+#pragma unroll
+      for (int w = 1; w < 4; w++) mx = fmaxf(mx, ms[j][w][q]);
+      float c[4], den = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; w++) {
+        c[w] = ms[j][w][q] == -INFINITY ? 0.f : __expf(ms[j][w][q] - mx);
+        den = fmaf(ls[j][w][q], c[w], den);
+      }
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int l = 16 * (q >> 2) + ((k0 + e) & 15);
+        float num = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) num = fmaf(os[w][i][r][l], c[w], num);
+        v[e] = den > 0.f ? num / den : 0.f;
+      }
+      if (out3) {
+        x3_store8(out3, q0 + row, h * HD + k0, heads * HD, v);
+      } else {
+        float *op = outp + (size_t)(q0 + row) * (heads * HD) + h * HD + k0;
+        *reinterpret_cast<float4 *>(op) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4 *>(op + 4) = make_float4(v[4], v[5], v[6], v[7]);
+      }
+    }
   }
 }
 
@@ -1295,12 +1354,27 @@ void launch_attn_merge_o(const AttnArgs &a, const Mat &wo, float *y, int positio
 }  // namespace q3h
 
 namespace q3h {
+// Rows per workgroup and query head: 32 (two query tiles) where that still makes
+// kPrefillWorkgroups of them (2048 rows, f16: 142 us against 190 with 16; 512
+// rows, f32: 26.0 against 24.0, 478 rows of 4 prompts 16.4 against 15.4)
+constexpr int kPrefillWorkgroups = 512;
+int attn_prefill_tile_rows(int heads, int M) {
+  return (M + 31) / 32 * heads >= kPrefillWorkgroups ? 32 : 16;
+}
+
 void launch_attn_prefill(const AttnArgs &a, int M, bool kv16, hipStream_t st) {
-  const dim3 grid(a.heads, a.tiles ? a.n_tiles : (M + kPrefillTile - 1) / kPrefillTile), block(256);
+  const int rows = a.tiles ? a.tile_rows : attn_prefill_tile_rows(a.heads, M);
+  const dim3 grid(a.heads, a.tiles ? a.n_tiles : (M + rows - 1) / rows), block(256);
   const int grp = a.heads / a.kvh;
-#define Q3H_P(KV, G)                                                                         \
-  hipLaunchKernelGGL((k_attn_prefill_x3<KV, G>), grid, block, 0, st, a.rd, a.qkv, a.ldq,      \
-                     a.layer, a.kvh, M, a.out, a.tiles)
+#define Q3H_P(KV, G)                                                                            \
+  do {                                                                                          \
+    if (rows == 32)                                                                             \
+      hipLaunchKernelGGL((k_attn_prefill_x3<KV, G, 2>), grid, block, 0, st, a.rd, a.qkv, a.ldq, \
+                         a.layer, a.kvh, M, a.out, a.tiles, a.out3);                            \
+    else                                                                                        \
+      hipLaunchKernelGGL((k_attn_prefill_x3<KV, G, 1>), grid, block, 0, st, a.rd, a.qkv, a.ldq, \
+                         a.layer, a.kvh, M, a.out, a.tiles, a.out3);                            \
+  } while (0)
   if (kv16) {
     if (grp == 1) Q3H_P(_Float16, 1);
     else if (grp == 2) Q3H_P(_Float16, 2);

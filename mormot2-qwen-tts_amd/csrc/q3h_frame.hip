@@ -1175,22 +1175,19 @@ struct StartArg {
 // Rows of one pass of a batched start (a prompt longer than this, which no
 // configuration reaches, goes alone): about 51 KB of work buffers a row.
 constexpr int kStartRows = 8192;
-// Rows from which a prompt of a stack with f32 activations joins a pass: the
-// products over more rows sum a row in one order whatever the row count, so
-// the pass gives the bits of one q3h_frame_start per stream. The int8 path
-// does so at any row count.
-constexpr int kStartJoinRows = 65;
-
+// Whether a prompt joins a pass: on the int8 path any does; with f32
+// activations those whose products sum a row in one order whatever the row
+// count (more than kManyRows rows), so the pass gives the bits of one
+// q3h_frame_start per stream.
 bool start_joins(const q3h_stack *s, int rows) {
-  if (rows > kStartRows) return false;
-  return s->cfg.act_q8 || (s->cfg.dtype == Q3H_Q8_0 && rows >= kStartJoinRows && f32_slice_path(s, rows));
+  return rows <= kStartRows && (s->cfg.act_q8 || x3_path(s, rows));
 }
 
 // The prompts args[0 .. n - 1] (start_joins, kStartRows rows in all) through
 // the talker as the rows of one pass, then the state of their streams: one
 // chain of launches over all rows instead of one chain per stream (32 int8
 // prompts of 16-256 rows: 7200 small launches on 32 streams, 46 ms, as
-// against 370 over 4350 rows). Enqueued on the first prompt's context stream;
+// against 250 over 4350 rows). Enqueued on the first prompt's context stream;
 // vals keeps the host values until the caller has synchronized it.
 void start_group(q3h_frame *f, const StartArg *args, int n, std::vector<StartPrompt> &vals,
                  std::vector<int2> &tiles) {
@@ -1209,7 +1206,7 @@ void start_group(q3h_frame *f, const StartArg *args, int n, std::vector<StartPro
   }
   // the query tiles, those with the most keys first
   const int tr = s->cfg.act_q8 ? attn_x_tile_rows(s->cfg.heads, s->cfg.kv_heads, M, longest)
-                               : kPrefillTile;
+                               : attn_prefill_tile_rows(s->cfg.heads, M);
   tiles.clear();
   if (tr > 0)
     for (int q0 = (longest - 1) / tr * tr; q0 >= 0; q0 -= tr)

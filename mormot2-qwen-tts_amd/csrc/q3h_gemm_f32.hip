@@ -23,8 +23,12 @@
 // the later tiles find in L2 / Infinity Cache.
 #include <hip/hip_runtime.h>
 
+#include <climits>
+
 #include "q3h_api_internal.h"
 #include "q3h_math.h"
+#include "q3h_wave.h"
+#include "q3h_x3.h"
 
 namespace q3h {
 namespace {
@@ -254,151 +258,11 @@ __global__ __launch_bounds__(64 * WN) void k_gemm_f32_m64(const float *__restric
     }
 }
 
-// f32 x f32 products on the bf16 matrix cores, exact to the fp32 rounding of
-// the sum: each operand split into three bf16 parts, x = x_hi + x_mid + x_lo
-// (the top 8 significant bits, the next 8, the last 8: exact, as an f32
-// significand has 24 bits), and the six part products whose weight is at
-// least 2^-16 of x w accumulated in fp32 (hi hi, hi mid, mid hi, hi lo,
-// lo hi, mid mid; each bf16 product is exact in fp32). The dropped three
-// weigh below 2^-23 of the product, under its fp32 rounding.
-//
-// v_mfma_f32_16x16x32_bf16: lane l holds A[l % 16][8 (l / 16) .. + 7] and
-// B[8 (l / 16) .. + 7][l % 16] (8 bf16 each) and receives
-// D[4 (l / 16) + r][l % 16]. The tile and pipeline are those of
-// k_gemm_f32_m64: 64 activation rows x 16 WN weight rows per workgroup, a 32-
-// column chunk at a time; the activations are split as they go to LDS (three
-// bf16 planes, double buffered), the weights come pre-split (Mat::x3) to
-// registers one chunk ahead. 24 MFMAs per wave and chunk instead of 32 of
-// the f32 kind, each a sixteenth of the cycles per flop.
-template <int WN, int EPI>
-__global__ __launch_bounds__(64 * WN) void k_gemm_x3_m64(const uint16_t *__restrict__ w3,
-                                                         const float *__restrict__ x, int ldx,
-                                                         int M, int N, int K, int kc,
-                                                         float *__restrict__ y, int ldy) {
-  constexpr int NT = 64 * WN;
-  constexpr int NB = 1;                  // 16-column weight tiles per wave
-  constexpr int XS = 40;                 // LDS row stride, bf16 (80 bytes)
-  constexpr int XF4 = 64 * 32 / 4 / NT;  // float4 of an activation chunk per thread
-  __shared__ uint16_t xs[2][3][64 * XS];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NB * WN + 16 * NB * wave, m0 = blockIdx.y * 64;
-  const int kz = blockIdx.z * kc;
-  const size_t plane = (size_t)N * K;
-  const uint16_t *wr[NB];
-#pragma unroll
-  for (int j = 0; j < NB; j++) wr[j] = w3 + (size_t)min(n0 + 16 * j + r, N - 1) * K + kz + 8 * g;
-  const float *xr[XF4];
-  int xo[XF4];
-#pragma unroll
-  for (int i = 0; i < XF4; i++) {
-    const int f = t + NT * i, row = f >> 3, c4 = f & 7;
-    xr[i] = x + (size_t)min(m0 + row, M - 1) * ldx + kz + 4 * c4;
-    xo[i] = row * XS + 4 * c4;
-  }
-  float4 xn[XF4];
-  u32x4v wn[NB][3], wc[NB][3];
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < XF4; i++) xn[i] = ld4(xr[i] + k0);
-#pragma unroll
-    for (int j = 0; j < NB; j++)
-#pragma unroll
-      for (int p = 0; p < 3; p++)
-        wn[j][p] = *reinterpret_cast<const u32x4v *>(wr[j] + p * plane + k0);
-  };
-  // the chunk's activations into the three planes of LDS buffer b
-  auto stage = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < XF4; i++) {
-      uint32_t h[4], m[4], l[4];
-      split3(xn[i].x, h[0], m[0], l[0]);
-      split3(xn[i].y, h[1], m[1], l[1]);
-      split3(xn[i].z, h[2], m[2], l[2]);
-      split3(xn[i].w, h[3], m[3], l[3]);
-      *reinterpret_cast<uint2 *>(&xs[b][0][xo[i]]) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-      *reinterpret_cast<uint2 *>(&xs[b][1][xo[i]]) = make_uint2(m[0] | (m[1] << 16), m[2] | (m[3] << 16));
-      *reinterpret_cast<uint2 *>(&xs[b][2][xo[i]]) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
-    }
-  };
-  v4f acc[NB][4];
-#pragma unroll
-  for (int j = 0; j < NB; j++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) acc[j][i] = v4f{0.f, 0.f, 0.f, 0.f};
-  load(0);
-  stage(0);
-#pragma unroll
-  for (int j = 0; j < NB; j++)
-#pragma unroll
-    for (int p = 0; p < 3; p++) wc[j][p] = wn[j][p];
-  __syncthreads();
-  const int nc = kc / 32;
-  for (int c = 0; c < nc; c++) {
-    const int b = c & 1;
-    if (c + 1 < nc) load(32 * (c + 1));
-#pragma unroll
-    for (int tm = 0; tm < 4; tm++) {
-      const int o = (16 * tm + r) * XS + 8 * g;
-      const bf8v ah = __builtin_bit_cast(bf8v, *reinterpret_cast<const u32x4v *>(&xs[b][0][o]));
-      const bf8v am = __builtin_bit_cast(bf8v, *reinterpret_cast<const u32x4v *>(&xs[b][1][o]));
-      const bf8v al = __builtin_bit_cast(bf8v, *reinterpret_cast<const u32x4v *>(&xs[b][2][o]));
-#pragma unroll
-      for (int j = 0; j < NB; j++) {
-        const bf8v bh = __builtin_bit_cast(bf8v, wc[j][0]), bm = __builtin_bit_cast(bf8v, wc[j][1]),
-                   bl = __builtin_bit_cast(bf8v, wc[j][2]);
-        v4f a = acc[j][tm];
-        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bm, a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bh, a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bm, a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, a, 0, 0, 0);
-        acc[j][tm] = a;
-      }
-    }
-    if (c + 1 < nc) {
-      stage(b ^ 1);
-#pragma unroll
-      for (int j = 0; j < NB; j++)
-#pragma unroll
-        for (int p = 0; p < 3; p++) wc[j][p] = wn[j][p];
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < NB; j++) {
-    const int n = n0 + 16 * j + r;
-#pragma unroll
-    for (int tm = 0; tm < 4; tm++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int m = m0 + 16 * tm + 4 * g + q;
-        const float v = acc[j][tm][q];
-        if (EPI == EPI_SWIGLU) {
-          const float u = __shfl_xor(v, 1);
-          if (m < M && (r & 1) == 0) y[(size_t)m * ldy + n / 2] = silu_mul_f(v, u);
-        } else if (m < M) {
-          if (EPI == EPI_ADD)
-            y[(size_t)m * ldy + n] += v;
-          else if (EPI == EPI_PART)
-            y[((size_t)blockIdx.z * M + m) * ldy + n] = v;
-          else
-            y[(size_t)m * ldy + n] = v;
-        }
-      }
-  }
-}
-
-// the three bf16 planes of an f32 matrix
-__global__ void k_split3(const float *__restrict__ f, size_t n, uint16_t *__restrict__ x3) {
+// f32 weights [N][K] into x3 operand tiles, one thread per 8
+__global__ __launch_bounds__(256) void k_split3(const float *__restrict__ f, int N, int K,
+                                                uint16_t *__restrict__ x3) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  uint32_t h, m, l;
-  split3(f[i], h, m, l);
-  x3[i] = (uint16_t)h;
-  x3[n + i] = (uint16_t)m;
-  x3[2 * n + i] = (uint16_t)l;
+  if (i < (size_t)N * K / 8) x3_tile_lane(f, N, K, i, x3);
 }
 
 // The same products with Q8_0 weights (int8 quants [N][K], then fp16 scales
@@ -420,7 +284,7 @@ __global__ void k_split3(const float *__restrict__ f, size_t n, uint16_t *__rest
 // loads of all its weights and scales first, then of its activations D
 // blocks ahead of the arithmetic, so that it waits for few memory round
 // trips. (Its time is the activation loads: every workgroup reads all M rows
-// over its K range; k_gemm_q8x_m64 shares them over 64 weight rows.)
+// over its K range; above 64 rows k_gemm_x3 shares them, already split.)
 template <int KK>
 constexpr int q8x_blocks_per_wave() {
   return KK <= 256 ? 2 : KK <= 1024 ? 4 : KK / 256;  // 4 to 8 waves
@@ -532,180 +396,253 @@ __global__ __launch_bounds__(64 * (KK / (32 * q8x_blocks_per_wave<KK>()))) void 
   for (int j = 0; j < NB; j++) epilogue<TM, KW, EPI>(red[j], m0, n0 + 16 * j, M, y, ldy);
 }
 
-// Q8_0 products over many rows with the activations staged in LDS: a
-// workgroup of WN waves owns 64 activation rows and 16 WN weight rows (wave w:
-// rows n0 + 16 w .. + 15) over the K range of its slice, so each activation
-// chunk crosses the vector memory path once per 16 WN weight rows instead of
-// once per 16 (k_gemm_q8x). Per 64-column chunk (two 32-blocks): the 64 x 64
-// activations are split into three bf16 planes in LDS (double buffered, one
-// barrier per chunk), each wave's quants and block scales go to registers one
-// chunk ahead; per block and 16-row tile three v_mfma_f32_16x16x32_bf16 (low,
-// middle, high part) into the block sum, scaled by the block scale into the
-// fp32 sum, as in k_gemm_q8x. Lane l holds weight row n0 + 16 w + l % 16 and
-// receives rows 4 (l / 16) + q of each tile: a wave's sums are complete, the
-// epilogue stores them directly. Used above 64 rows: with fewer, its
-// N / (16 WN) workgroups leave most CUs idle.
-template <int WN, int EPI>
-__global__ __launch_bounds__(64 * WN) void k_gemm_q8x_m64(const int8_t *__restrict__ wq,
-                                                          const float *__restrict__ x, int ldx,
-                                                          int M, int N, int K, int kc,
-                                                          float *__restrict__ y, int ldy) {
-  constexpr int NT = 64 * WN;
-  constexpr int CW = 64;                  // chunk columns
-  constexpr int XS = CW + 8;              // LDS row stride, bf16 (144 bytes)
-  constexpr int SF = 64 * CW / 4 / NT;    // float4 of a chunk per thread
-  __shared__ uint16_t xs[2][3][64 * XS];
+// Products over many rows (more than 64), the activations already split into
+// operand tiles by the kernel that made them (x3_offset: RMSNorm, attention,
+// SwiGLU), so that no product spends vector instructions on it: with the split
+// in the staging of every 64 x 64 tile the Q8_0 products were bound by it (about
+// 1200 VALU cycles to 384 of MFMA per 64 columns). Q8 == false: f32 weights in
+// the same tiles (Mat::x3), six part products per chunk (x3 x x3, q3h_x3.h).
+// Q8: int8 quants row-major and block scales; a quant is exact in bf16, so a
+// 32-block is three part products into a block sum (low, middle, high part),
+// scaled by the block scale into the fp32 sum.
+//
+// A workgroup of 4 waves owns 16 MT activation rows and 64 NT weight rows (NT
+// 16-row tiles per wave) over the K range of its slice. Per step of KC 32-column
+// chunks the activation tiles are copied to LDS (contiguous, two buffers, one
+// barrier per step; loaded three steps ahead, through registers) and read as
+// operands by every wave; the weights go to registers two steps ahead. A lane
+// loads 16 quants of its row's 64 columns; v_permlane32_swap of the two halves
+// leaves block 0 in the first and block 1 in the second, with the 8-column
+// groups in the order 0, 2, 1, 3, which the activation operands are read in.
+// The order of a row's sums is that of its chunks alone: any tile shape and
+// row count gives the same bits.
+template <bool Q8, int MT, int NT, int EPI>
+struct GemmX3 {
+  static constexpr int WN = 4, kThreads = 64 * WN, KC = Q8 ? 2 : 1;
+  static constexpr int kStep = MT * KC * 192;           // 16-byte words of a step's activations
+  static constexpr int kXW = (kStep + kThreads - 1) / kThreads;  // per thread
+  static constexpr int kWW = Q8 ? 1 : 3;                // words per weight tile and step
+  static constexpr int kOutLd = 8 * NT + 4;             // a wave's SwiGLU outputs in LDS
+  static constexpr size_t kLds = 2 * kStep * 16;
+  static_assert((size_t)WN * 16 * MT * kOutLd * 4 <= kLds, "the outputs fit the staging buffers");
+};
+
+template <bool Q8, int MT, int NT, int EPI>
+__global__ __launch_bounds__(256, 2) void k_gemm_x3(const void *__restrict__ wp,
+                                                    const uint16_t *__restrict__ x3, int M, int N,
+                                                    int K, int kc, float *__restrict__ y, int ldy,
+                                                    uint16_t *__restrict__ y3) {
+  using G = GemmX3<Q8, MT, NT, EPI>;
+  constexpr int KC = G::KC;
+  __shared__ x3_u4 xs[2 * G::kStep];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * WN + 16 * wave, m0 = blockIdx.y * 64;
-  const int kz = blockIdx.z * kc;
-  const int row = min(n0 + r, N - 1);
-  const int8_t *wr = wq + (size_t)row * K + kz + 8 * g;
-  const _Float16 *dr =
-      reinterpret_cast<const _Float16 *>(wq + (size_t)N * K) + (size_t)row * (K / 32) + kz / 32;
-  // this thread's float4 of a chunk: global and LDS offsets
-  const float *xg[SF];
-  int lo[SF];
+  const int n0 = (blockIdx.x * G::WN + wave) * 16 * NT, mt0 = blockIdx.y * MT;
+  const int nq = K >> 5, mt16 = (M + 15) >> 4;
+  const int s0 = blockIdx.z * kc / (32 * KC), s1 = s0 + kc / (32 * KC);
+  // this thread's words of a step: tile, then chunk, part and lane
+  const x3_u4 *xg[G::kXW];
 #pragma unroll
-  for (int i = 0; i < SF; i++) {
-    const int f = t + NT * i, rw = f / (CW / 4), c4 = f % (CW / 4);
-    xg[i] = x + (size_t)min(m0 + rw, M - 1) * ldx + kz + 4 * c4;
-    lo[i] = rw * XS + 4 * c4;
+  for (int i = 0; i < G::kXW; i++) {
+    const int f = min(t + G::kThreads * i, G::kStep - 1), tile = f / (KC * 192);
+    xg[i] = reinterpret_cast<const x3_u4 *>(x3) + (size_t)min(mt0 + tile, mt16 - 1) * nq * 192 +
+            (f - tile * KC * 192);
   }
-  float4 xn[SF];
-  uint2 wn[2], wc[2];
-  uint32_t dn, dc;  // the chunk's two block scales
-  auto load = [&](int k0) {
+  const int8_t *wq = reinterpret_cast<const int8_t *>(wp);
+  const x3_u4 *wt = Q8 ? reinterpret_cast<const x3_u4 *>(wq + (size_t)(n0 + r) * K + 16 * g)
+                       : reinterpret_cast<const x3_u4 *>(wp) + (size_t)(n0 >> 4) * nq * 192 + lane;
+  const uint32_t *dr = reinterpret_cast<const uint32_t *>(
+      reinterpret_cast<const _Float16 *>(wq + (size_t)N * K) + (size_t)(n0 + r) * nq);
+  x3_u4 a[2][G::kXW], w[2][NT][G::kWW];
+  uint32_t d[2][NT];
+  auto load_x = [&](int s, int b) {
 #pragma unroll
-    for (int i = 0; i < SF; i++) xn[i] = ld4(xg[i] + k0);
-    wn[0] = *reinterpret_cast<const uint2 *>(wr + k0);
-    wn[1] = *reinterpret_cast<const uint2 *>(wr + k0 + 32);
-    dn = *reinterpret_cast<const uint32_t *>(dr + k0 / 32);
+    for (int i = 0; i < G::kXW; i++) a[b][i] = xg[i][(size_t)min(s, s1 - 1) * KC * 192];
   };
-  auto stage = [&](int b) {
+  auto load_w = [&](int s, int b) {
+    const int sc = min(s, s1 - 1);
 #pragma unroll
-    for (int i = 0; i < SF; i++) {
-      uint32_t h[4], md[4], l[4];
-      split3(xn[i].x, h[0], md[0], l[0]);
-      split3(xn[i].y, h[1], md[1], l[1]);
-      split3(xn[i].z, h[2], md[2], l[2]);
-      split3(xn[i].w, h[3], md[3], l[3]);
-      *reinterpret_cast<uint2 *>(&xs[b][0][lo[i]]) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-      *reinterpret_cast<uint2 *>(&xs[b][1][lo[i]]) = make_uint2(md[0] | (md[1] << 16), md[2] | (md[3] << 16));
-      *reinterpret_cast<uint2 *>(&xs[b][2][lo[i]]) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
-    }
-  };
-  v4f acc[4];
+    for (int j = 0; j < NT; j++) {
+      if constexpr (Q8) {
+        w[b][j][0] = wt[(size_t)j * K + 4 * sc];  // 16 rows of K bytes on: K words
+        d[b][j] = dr[(size_t)j * 8 * nq + sc];
+      } else {
 #pragma unroll
-  for (int i = 0; i < 4; i++) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
-  load(0);
-  stage(0);
-  wc[0] = wn[0];
-  wc[1] = wn[1];
-  dc = dn;
-  __syncthreads();
-  const int nc = kc / CW;
-  for (int c = 0; c < nc; c++) {
-    const int b = c & 1;
-    if (c + 1 < nc) load(CW * (c + 1));
-#pragma unroll
-    for (int kb = 0; kb < 2; kb++) {
-      const bf8v bw = q8_bf16x8(wc[kb]);
-      const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(dc >> (16 * kb)));
-#pragma unroll
-      for (int tm = 0; tm < 4; tm++) {
-        const int o = (16 * tm + r) * XS + 32 * kb + 8 * g;
-        const bf8v ah = __builtin_bit_cast(bf8v, *reinterpret_cast<const u32x4v *>(&xs[b][0][o]));
-        const bf8v am = __builtin_bit_cast(bf8v, *reinterpret_cast<const u32x4v *>(&xs[b][1][o]));
-        const bf8v al = __builtin_bit_cast(bf8v, *reinterpret_cast<const u32x4v *>(&xs[b][2][o]));
-        v4f sm = v4f{0.f, 0.f, 0.f, 0.f};
-        sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bw, sm, 0, 0, 0);
-        sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bw, sm, 0, 0, 0);
-        sm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bw, sm, 0, 0, 0);
-#pragma unroll
-        for (int q = 0; q < 4; q++) acc[tm][q] = fmaf(d, sm[q], acc[tm][q]);
+        for (int c = 0; c < 3; c++) w[b][j][c] = wt[((size_t)j * nq + sc) * 192 + 64 * c];
       }
     }
-    if (c + 1 < nc) {
-      stage(b ^ 1);
-      wc[0] = wn[0];
-      wc[1] = wn[1];
-      dc = dn;
+  };
+  auto stage = [&](int b, int sl) {
+#pragma unroll
+    for (int i = 0; i < G::kXW; i++) {
+      const int f = t + G::kThreads * i;
+      if (G::kStep % G::kThreads == 0 || f < G::kStep) xs[b * G::kStep + f] = a[sl][i];
     }
+  };
+  v4f acc[NT][MT];
+#pragma unroll
+  for (int j = 0; j < NT; j++)
+#pragma unroll
+    for (int i = 0; i < MT; i++) acc[j][i] = v4f{0.f, 0.f, 0.f, 0.f};
+  // the operand's lane in LDS: the 8-column groups in the weights' order
+  const int la = Q8 ? ((g == 1 ? 2 : g == 2 ? 1 : g) * 16 + r) : lane;
+  auto step = [&](int s, auto buf) {
+    constexpr int b = decltype(buf)::value;
+#pragma unroll
+    for (int k = 0; k < KC; k++) {
+      bf8v x[MT][3];
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+          x[i][c] = __builtin_bit_cast(bf8v, xs[b * G::kStep + ((i * KC + k) * 3 + c) * 64 + la]);
+      if constexpr (Q8) {
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+          const x3_u4 &q = w[b][j][0];
+          const auto s0_ = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false);
+          const auto s1_ = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
+          const bf8v bw = q8_bf16x8(make_uint2(s0_[k], s1_[k]));
+          const float dv = (float)__builtin_bit_cast(_Float16, (uint16_t)(d[b][j] >> (16 * k)));
+          v4f sm[MT];
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+            sm[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i][2], bw, v4f{0.f, 0.f, 0.f, 0.f},
+                                                            0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+            sm[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i][1], bw, sm[i], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+            sm[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i][0], bw, sm[i], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[j][i][e] = fmaf(dv, sm[i][e], acc[j][i][e]);
+        }
+      } else {
+        constexpr int pa[6] = {1, 2, 0, 1, 0, 0}, pb[6] = {1, 0, 2, 0, 1, 0};
+#pragma unroll
+        for (int c = 0; c < 6; c++)
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+              acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  x[i][pa[c]], __builtin_bit_cast(bf8v, w[b][j][pb[c] % G::kWW]), acc[j][i], 0, 0,
+                  0);
+      }
+    }
+    load_w(s + 2, b);
+    stage(b ^ 1, b ^ 1);
+    load_x(s + 3, b ^ 1);
     __syncthreads();
+  };
+  load_x(s0, 0);
+  load_w(s0, 0);
+  load_x(s0 + 1, 1);
+  load_w(s0 + 1, 1);
+  stage(0, 0);
+  load_x(s0 + 2, 0);
+  __syncthreads();
+  int s = s0;
+  for (; s + 1 < s1; s += 2) {
+    step(s, std::integral_constant<int, 0>{});
+    step(s + 1, std::integral_constant<int, 1>{});
   }
-  const int n = n0 + r;
+  if (s < s1) step(s, std::integral_constant<int, 0>{});
+  // lane l holds (m = 16 (mt0 + i) + 4 g + e, n = n0 + 16 j + r)
+  if constexpr (EPI == EPI_SWIGLU) {
+    // silu(gate) * up through the wave's part of LDS (the steps are done: every
+    // wave has passed the last barrier), then 8 columns per lane split into the
+    // tiles of the next product's activations
+    float *o = reinterpret_cast<float *>(xs) + wave * 16 * MT * G::kOutLd;
 #pragma unroll
-  for (int tm = 0; tm < 4; tm++)
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int m = m0 + 16 * tm + 4 * g + q;
-      const float v = acc[tm][q];
-      if (EPI == EPI_SWIGLU) {
-        const float u = __shfl_xor(v, 1);  // up: the odd row after its gate
-        if (m < M && (r & 1) == 0) y[(size_t)m * ldy + n / 2] = silu_mul_f(v, u);
-      } else if (m < M) {
-        if (EPI == EPI_ADD)
-          y[(size_t)m * ldy + n] += v;
-        else if (EPI == EPI_PART)
-          y[((size_t)blockIdx.z * M + m) * ldy + n] = v;
-        else
-          y[(size_t)m * ldy + n] = v;
-      }
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float v = acc[j][i][e], u = dpp_f<kQuadXor1>(v);
+          if ((r & 1) == 0) o[(16 * i + 4 * g + e) * G::kOutLd + 8 * j + (r >> 1)] = silu_mul_f(v, u);
+        }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int f = lane; f < 16 * MT * NT; f += 64) {
+      const int row = f / NT, j = f % NT, m = 16 * mt0 + row;
+      const float4 p0 = *reinterpret_cast<const float4 *>(&o[row * G::kOutLd + 8 * j]);
+      const float4 p1 = *reinterpret_cast<const float4 *>(&o[row * G::kOutLd + 8 * j + 4]);
+      const float v[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+      if (m < M) x3_store8(y3, m, n0 / 2 + 8 * j, N / 2, v);
     }
+  } else {
+    float *yo = y + (EPI == EPI_PART ? (size_t)blockIdx.z * M * ldy : 0) + n0 + r;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int m = 16 * (mt0 + i) + 4 * g + e;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < NT; j++) yo[(size_t)m * ldy + 16 * j] = acc[j][i][e];
+      }
+  }
 }
 
-// h[m] += slices 0 .. S-1 of part [S][M][K], added in slice order; then, with
-// a norm weight, xn[m] = w * (h[m] * inv), inv = 1 / sqrt(mean(h[m]^2) + eps)
-// (sum of squares in double). One workgroup per row, K <= 4096: a thread
-// holds columns t + 256 i of each 1024-column round in registers, and the norm
-// weights are loaded before the partials, so the normalization needs no
-// second trip to memory.
+// rows x [M][ldx] split into operand tiles, a thread per 4 columns
+__global__ __launch_bounds__(256) void k_x3_rows(const float *__restrict__ x, int ldx, int M, int K,
+                                                 uint16_t *__restrict__ o) {
+  const int i = blockIdx.x * 256 + threadIdx.x, m = i / (K / 4), k = 4 * (i - m * (K / 4));
+  if (m >= M) return;
+  const float4 v = ld4(x + (size_t)m * ldx + k);
+  const float v4[4] = {v.x, v.y, v.z, v.w};
+  x3_store4(o, m, k, K, v4);
+}
+
+// h[m] += slices 0 .. S-1 of part [S][M][K], added in slice order (S == 0: h
+// as it is); then, with a norm weight, w * (h[m] * inv), inv = 1 / sqrt(mean(
+// h[m]^2) + eps) (sum of squares in double), to xn [M][K] or, split, to the
+// operand tiles x3. One workgroup per row, K <= 4096, K % 4 == 0: a thread
+// holds columns 4 t .. + 3 of each 1024-column round in registers (16-byte
+// loads, all of a round issued together), and the norm weights are loaded
+// before the partials, so the normalization needs no second trip to memory.
 constexpr int kResidNormRounds = 4;
 
 template <int S>
 __global__ __launch_bounds__(256) void k_resid_norm(float *__restrict__ h,
                                                     const float *__restrict__ part, int M,
                                                     int K, const float *__restrict__ w,
-                                                    float eps, float *__restrict__ xn) {
+                                                    float eps, float *__restrict__ xn,
+                                                    uint16_t *__restrict__ x3) {
   constexpr int NR = kResidNormRounds;
   __shared__ double red[4];
-  const int m = blockIdx.x, t = threadIdx.x;
+  // operand tiles: the 16 rows of a tile on one XCD (workgroups go to the XCDs
+  // in turn), whose L2 joins their 16-byte pieces of each line
+  const int b = blockIdx.x, t = threadIdx.x;
+  const int m = x3 ? (b & ~127) + (b & 7) * 16 + ((b >> 3) & 15) : b;
+  if (m >= M) return;
   float *hr = h + (size_t)m * K;
-  float wv[NR][4];
+  float4 wv[NR], hv[NR];
   if (w) {
 #pragma unroll
     for (int r = 0; r < NR; r++)
-      if (1024 * r < K)
-#pragma unroll
-        for (int i = 0; i < 4; i++) wv[r][i] = w[min(1024 * r + t + 256 * i, K - 1)];
+      if (1024 * r < K) wv[r] = ld4(w + min(1024 * r + 4 * t, K - 4));
   }
-  float hv[NR][4];
   double ss = 0.0;
 #pragma unroll
   for (int r = 0; r < NR; r++) {
-    const int k0 = 1024 * r;
-    if (k0 >= K) break;
-    // four columns per thread, every load (clamped) issued before the sums
-    float a[4][S];
+    if (1024 * r >= K) break;
+    const int k = 1024 * r + 4 * t, kc = min(k, K - 4);
+    float4 a[S ? S : 1];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int k = min(k0 + t + 256 * i, K - 1);
+    for (int s = 0; s < S; s++) a[s] = ld4(part + ((size_t)s * M + m) * K + kc);
+    float4 v = ld4(hr + kc);
 #pragma unroll
-      for (int s = 0; s < S; s++) a[i][s] = part[((size_t)s * M + m) * K + k];
-      hv[r][i] = hr[k];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int k = k0 + t + 256 * i;
-      float v = hv[r][i];
-#pragma unroll
-      for (int s = 0; s < S; s++) v += a[i][s];
-      hv[r][i] = v;
-      if (k < K) {
-        hr[k] = v;
-        ss += (double)v * v;
-      }
+    for (int s = 0; s < S; s++) v.x += a[s].x, v.y += a[s].y, v.z += a[s].z, v.w += a[s].w;
+    hv[r] = v;
+    if (k < K) {
+      if (S) *reinterpret_cast<float4 *>(hr + k) = v;
+      ss += (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
     }
   }
   if (w == nullptr) return;
@@ -716,12 +653,14 @@ __global__ __launch_bounds__(256) void k_resid_norm(float *__restrict__ h,
   const float inv = (float)(1.0 / sqrt(tot / K + (double)eps));
 #pragma unroll
   for (int r = 0; r < NR; r++) {
-    if (1024 * r >= K) break;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int k = 1024 * r + t + 256 * i;
-      if (k < K) xn[(size_t)m * K + k] = wv[r][i] * (hv[r][i] * inv);
-    }
+    const int k = 1024 * r + 4 * t;
+    if (1024 * r >= K || k >= K) break;
+    const float o[4] = {wv[r].x * (hv[r].x * inv), wv[r].y * (hv[r].y * inv),
+                        wv[r].z * (hv[r].z * inv), wv[r].w * (hv[r].w * inv)};
+    if (x3)
+      x3_store4(x3, m, k, K, o);
+    else
+      *reinterpret_cast<float4 *>(xn + (size_t)m * K + k) = make_float4(o[0], o[1], o[2], o[3]);
   }
 }
 
@@ -765,22 +704,6 @@ void launch_m64(const Mat &W, const float *x, int ldx, int M, int epi, float *y,
                 hipStream_t st, int ks = 1) {
   const dim3 grid(W.N / (16 * WN), (M + 63) / 64, ks), block(64 * WN);
   const int kc = W.K / ks;
-  if (W.x3 && epi != EPI_ADD_SILU) {
-    const dim3 gx(W.N / (16 * WN), (M + 63) / 64, ks);  // one 16-column tile per wave
-#define Q3H_X(E)                                                                              \
-  hipLaunchKernelGGL((k_gemm_x3_m64<WN, E>), gx, block, 0, st, W.x3, x, ldx, M, W.N, W.K, kc, \
-                     y, ldy)
-    if (epi == EPI_STORE)
-      Q3H_X(EPI_STORE);
-    else if (epi == EPI_ADD)
-      Q3H_X(EPI_ADD);
-    else if (epi == EPI_PART)
-      Q3H_X(EPI_PART);
-    else
-      Q3H_X(EPI_SWIGLU);
-#undef Q3H_X
-    return;
-  }
 #define Q3H_G(E)                                                                               \
   hipLaunchKernelGGL((k_gemm_f32_m64<WN, E>), grid, block, 0, st, W.f, x, ldx, M, W.N, W.K, kc, \
                      y, ldy)
@@ -843,35 +766,37 @@ void launch_q8x_t(const Mat &W, const float *x, int ldx, int M, int epi, float *
   }
 }
 
-constexpr int kQ8M64Waves = 4;  // 64 weight rows per workgroup
-
-void launch_q8x_m64(const Mat &W, const float *x, int ldx, int M, int epi, float *y, int ldy,
-                    int ks, hipStream_t st) {
-  constexpr int WN = kQ8M64Waves;
-  const dim3 grid(W.N / (16 * WN), (M + 63) / 64, ks), block(64 * WN);
-  const int kc = W.K / ks;
-#define Q3H_Q(E)                                                                           \
-  hipLaunchKernelGGL((k_gemm_q8x_m64<WN, E>), grid, block, 0, st, W.q, x, ldx, M, W.N, W.K, \
-                     kc, y, ldy)
-  if (epi == EPI_STORE)
-    Q3H_Q(EPI_STORE);
-  else if (epi == EPI_ADD)
-    Q3H_Q(EPI_ADD);
-  else if (epi == EPI_SWIGLU)
-    Q3H_Q(EPI_SWIGLU);
-  else if (epi == EPI_PART)
-    Q3H_Q(EPI_PART);
+// The tile of a product over M rows, by rounds of 256 workgroups (one per CU)
+// and the time of a round of each: 64 x 128 tiles 100, 64 x 64 58, 32 x 64 38
+// (measured, K = 1024: f32 q/k/v at 2048 rows 4, 8 and 16 rounds 78, 88 and 114
+// us; Q8_0 gate/up 6, 12 and 24 rounds 92, 111 and 142 us; 203 rows, f32 q/k/v:
+// 1, 1 and 2 rounds 21.1, 14.8 and 14.3 us). 64 x 256 tiles spilled registers.
+// Before (64 x 64 tiles that split their own activations), Q8_0: gate/up 172
+// us at 2048 rows and 30.5 at 203; f32 q/k/v 34 us at 512 rows, 25 now.
+template <bool Q8, int EPI>
+void launch_x3(const Mat &W, const uint16_t *x3, int M, int ks, float *y, int ldy, uint16_t *y3,
+               hipStream_t st) {
+  const void *wp = Q8 ? (const void *)W.q : (const void *)W.x3;
+  const int r32 = (M + 31) / 32, r64 = (M + 63) / 64, nb = W.N / 64;
+  auto cost = [&](int tiles, int round) { return (tiles * ks + 255) / 256 * round; };
+  const int c42 = nb % 2 == 0 ? cost(nb / 2 * r64, 100) : INT_MAX, c41 = cost(nb * r64, 58),
+            c21 = cost(nb * r32, 38);
+#define Q3H_X(MT, NT, R)                                                                        \
+  hipLaunchKernelGGL((k_gemm_x3<Q8, MT, NT, EPI>), dim3(W.N / (64 * NT), R, ks), dim3(256), 0, \
+                     st, wp, x3, M, W.N, W.K, W.K / ks, y, ldy, y3)
+  if (c42 <= c41 && c42 <= c21)
+    Q3H_X(4, 2, r64);
+  else if (c41 < c21)
+    Q3H_X(4, 1, r64);
   else
-    require(false, Q3H_E_ARG, "EPI_ADD_SILU takes f32 weights");
-#undef Q3H_Q
+    Q3H_X(2, 1, r32);
+#undef Q3H_X
 }
 
 // Q8_0 weights, f32 activations [M][ldx], over K slices of K / ks columns
 void launch_q8x(const Mat &W, const float *x, int ldx, int M, int epi, float *y, int ldy, int ks,
                 hipStream_t st) {
-  if (M > 64 && W.N % (16 * kQ8M64Waves) == 0 && (W.K / ks) % 64 == 0) {
-    launch_q8x_m64(W, x, ldx, M, epi, y, ldy, ks, st);
-  } else if (M <= 16) {
+  if (M <= 16) {
     launch_q8x_t<1, 1>(W, x, ldx, M, epi, y, ldy, ks, st);
   } else if (W.N % 32 != 0) {
     if (M <= 32)
@@ -907,8 +832,41 @@ void launch_m(const Mat &W, const float *x, int ldx, int M, int epi, float *y, i
 }  // namespace
 
 void launch_split3(const Mat &m, hipStream_t st) {
-  const size_t n = (size_t)m.N * m.K;
-  hipLaunchKernelGGL(k_split3, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m.f, n, m.x3);
+  const size_t n = (size_t)m.N * m.K / 8;
+  hipLaunchKernelGGL(k_split3, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m.f, m.N, m.K,
+                     m.x3);
+}
+
+bool gemm_x3_supported(const Mat &W, int ks) {
+  return (W.q || W.x3) && W.N % 64 == 0 && W.K % (64 * ks) == 0;
+}
+
+void launch_gemm_x3(const Mat &W, const uint16_t *x3, int M, float *y, int ldy, hipStream_t st) {
+  if (W.q)
+    launch_x3<true, EPI_STORE>(W, x3, M, 1, y, ldy, nullptr, st);
+  else
+    launch_x3<false, EPI_STORE>(W, x3, M, 1, y, ldy, nullptr, st);
+}
+
+void launch_gemm_x3_swiglu(const Mat &W, const uint16_t *x3, int M, uint16_t *y3, hipStream_t st) {
+  if (W.q)
+    launch_x3<true, EPI_SWIGLU>(W, x3, M, 1, nullptr, 0, y3, st);
+  else
+    launch_x3<false, EPI_SWIGLU>(W, x3, M, 1, nullptr, 0, y3, st);
+}
+
+int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hipStream_t st) {
+  if (W.q)
+    launch_x3<true, EPI_PART>(W, x3, M, kF32Slices, part, W.N, nullptr, st);
+  else
+    launch_x3<false, EPI_PART>(W, x3, M, kF32Slices, part, W.N, nullptr, st);
+  return kF32Slices;
+}
+
+void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, hipStream_t st) {
+  const size_t n = (size_t)M * (K / 4);
+  hipLaunchKernelGGL(k_x3_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, ldx, M, K,
+                     o);
 }
 
 bool gemm_f32_supported(int N, int K) {
@@ -953,11 +911,13 @@ int launch_gemm_f32_part(const Mat &W, const float *x, int ldx, int M, float *pa
 }
 
 void launch_resid_norm(float *h, const float *part, int M, int K, const float *norm_w,
-                       float eps, float *xn, int slices, hipStream_t st) {
-  require(K <= 1024 * kResidNormRounds, Q3H_E_ARG, "launch_resid_norm: K above 4096");
-#define Q3H_RN(S)                                                                              \
-  hipLaunchKernelGGL(k_resid_norm<S>, dim3(M), dim3(256), 0, st, h, part, M, K, norm_w, eps, xn)
+                       float eps, float *xn, int slices, hipStream_t st, uint16_t *x3) {
+  require(K <= 1024 * kResidNormRounds && K % 4 == 0, Q3H_E_ARG, "launch_resid_norm: K above 4096");
+#define Q3H_RN(S)                                                                               \
+  hipLaunchKernelGGL(k_resid_norm<S>, dim3(x3 ? (M + 127) / 128 * 128 : M), dim3(256), 0, st, h, \
+                     part, M, K, norm_w, eps, xn, x3)
   switch (slices) {
+    case 0: Q3H_RN(0); break;
     case 1: Q3H_RN(1); break;
     case 2: Q3H_RN(2); break;
     case 3: Q3H_RN(3); break;
@@ -965,7 +925,7 @@ void launch_resid_norm(float *h, const float *part, int M, int K, const float *n
     case 6: Q3H_RN(6); break;
     case 8: Q3H_RN(8); break;
     case 12: Q3H_RN(12); break;
-    default: require(false, Q3H_E_ARG, "launch_resid_norm: 1-4, 6, 8 or 12 slices");
+    default: require(false, Q3H_E_ARG, "launch_resid_norm: 0-4, 6, 8 or 12 slices");
   }
 #undef Q3H_RN
 }

@@ -19,8 +19,8 @@ struct Mat {
   _Float16 *d = nullptr;
   float *f = nullptr;
   // f32 matrices of stacks that prefill many rows: the same values as three
-  // bf16 planes [3][N][K] (w = hi + mid + lo exactly), the operands of the
-  // split-bf16 matrix-core products (null: not made)
+  // bf16 parts (w = hi + mid + lo exactly) in operand tiles, the operands of
+  // the split-bf16 matrix-core products (q3h_x3.h; null: not made)
   uint16_t *x3 = nullptr;
 };
 
@@ -144,8 +144,22 @@ bool launch_gemv_q8_code(const GemvArgs &a, const float *logits, int vocab, cons
 // the quants exact in bf16 and the activations split exactly into three bf16
 // parts; taken for more than kGemvRows rows)
 bool gemm_f32_supported(int N, int K);
-// the three bf16 planes of m.f into m.x3 (allocated by the caller)
+// m.f as operand tiles into m.x3 (allocated by the caller)
 void launch_split3(const Mat &m, hipStream_t st);
+// The products over more than kManyRows rows whose activations are split into
+// operand tiles (x3_offset, q3h_x3.h; x3_bytes(M, K)) by the kernel that makes
+// them: y [M][ldy] = W . x; silu(gate) * up of interleaved rows into the tiles
+// y3 of the next product; the kF32Slices slices of K (returned) to part
+// [slices][M][N]. A row's sums do not depend on the row count. Q8_0 weights,
+// or f32 ones with Mat::x3.
+constexpr int kManyRows = 64;
+inline size_t x3_bytes(size_t M, size_t K) { return (M + 15) / 16 * 16 * K * 6; }
+bool gemm_x3_supported(const Mat &W, int ks);
+void launch_gemm_x3(const Mat &W, const uint16_t *x3, int M, float *y, int ldy, hipStream_t st);
+void launch_gemm_x3_swiglu(const Mat &W, const uint16_t *x3, int M, uint16_t *y3, hipStream_t st);
+int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hipStream_t st);
+// rows x [M][ldx] split into operand tiles
+void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, hipStream_t st);
 constexpr int kGemvRows = 4;
 void launch_gemm_f32(const Mat &W, const float *x, int ldx, int M, int epi, float *y, int ldy,
                      hipStream_t st);
@@ -165,11 +179,11 @@ int launch_gemm_f32_part(const Mat &W, const float *x, int ldx, int M, float *pa
                          hipStream_t st);
 // K / 256 when W takes the 256-column slices over M rows, else 0
 int q8x_slices(const Mat &W, int M);
-// h [M][K] += the `slices` slices of part (1-4, 6, 8 or 12), in slice order; then,
-// when norm_w != nullptr, xn [M][K] = RMSNorm(h) with norm_w (double sum of
-// squares)
+// h [M][K] += the `slices` slices of part (0-4, 6, 8 or 12), in slice order; then,
+// when norm_w != nullptr, RMSNorm(h) with norm_w (double sum of squares) to xn
+// [M][K], or to the operand tiles x3 when that is non-null
 void launch_resid_norm(float *h, const float *part, int M, int K, const float *norm_w,
-                       float eps, float *xn, int slices, hipStream_t st);
+                       float eps, float *xn, int slices, hipStream_t st, uint16_t *x3 = nullptr);
 // the int8 path (q3h_gemm.hip): shapes it takes (N % 16 == 0, K % 256 == 0,
 // K <= 3072)
 bool gemm_i8_supported(int N, int K);
@@ -234,6 +248,7 @@ struct AttnArgs {
   const float *qkn;  // [q_norm | k_norm | eps] of the layer
   const float2 *rope_cs;
   float *out;    // [M][heads * head_dim]
+  uint16_t *out3;  // launch_attn_prefill: the outputs as operand tiles instead, when non-null
   float *part;   // [M][heads][attn_splits slots][head_dim + 2]
   int layers;    // > layer + 1: a decode launch also loads layer + 1's cache rows ahead
   // launch_attn_prefill and launch_attn_x_prompt over several contexts' rows:
@@ -242,8 +257,8 @@ struct AttnArgs {
   const int2 *tiles;
   int n_tiles, tile_rows;
 };
-// rows per query tile of launch_attn_prefill
-constexpr int kPrefillTile = 16;
+// rows per query tile of launch_attn_prefill over M rows
+int attn_prefill_tile_rows(int heads, int M);
 // how the decode attention cuts contexts of up to `positions` positions: len
 // positions per split (a multiple of 16), threads per workgroup (0: one
 // workgroup per query head over at most 256 positions, no split); fold: the

@@ -30,6 +30,42 @@ typedef unsigned int x3_u4 __attribute__((ext_vector_type(4)));
 
 constexpr int kX3Stride = 40;  // LDS row of a unit, bf16 (32 + 8: 80 bytes)
 
+// element (m, k) of part p (0 hi, 1 mid, 2 lo) of K-column rows in operand
+// tiles; 8 columns from a multiple of 8 are 16 contiguous bytes
+__host__ __device__ inline size_t x3_offset(int m, int k, int K) {
+  return ((size_t)(m >> 4) * (K >> 5) + (k >> 5)) * 1536 + ((k & 31) >> 3) * 128 + (m & 15) * 8 +
+         (k & 7);
+}
+constexpr int kX3Part = 512;  // elements from a part of a tile to the next
+
+// 4 columns from k (a multiple of 4) of row m, split into the tiles at o
+__device__ __forceinline__ void x3_store4(uint16_t *o, int m, int k, int K, const float (&v)[4]) {
+  uint32_t h[4], md[4], l[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) split3(v[e], h[e], md[e], l[e]);
+  uint16_t *d = o + x3_offset(m, k, K);
+  *reinterpret_cast<uint2 *>(d) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+  *reinterpret_cast<uint2 *>(d + kX3Part) = make_uint2(md[0] | (md[1] << 16), md[2] | (md[3] << 16));
+  *reinterpret_cast<uint2 *>(d + 2 * kX3Part) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+}
+
+// 8 columns from k (a multiple of 8)
+__device__ __forceinline__ void x3_store8(uint16_t *o, int m, int k, int K, const float (&v)[8]) {
+  x3_u4 part[3];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    uint32_t h0, m0, l0, h1, m1, l1;
+    split3(v[2 * e], h0, m0, l0);
+    split3(v[2 * e + 1], h1, m1, l1);
+    part[0][e] = h0 | (h1 << 16);
+    part[1][e] = m0 | (m1 << 16);
+    part[2][e] = l0 | (l1 << 16);
+  }
+  uint16_t *d = o + x3_offset(m, k, K);
+#pragma unroll
+  for (int c = 0; c < 3; c++) *reinterpret_cast<x3_u4 *>(d + c * kX3Part) = part[c];
+}
+
 // weights f [N][K] row-major into the operand tiles x3 (3 N K bf16; N % 16 ==
 // 0, K % 32 == 0), or the same tiles unsplit (WF32): one thread per (tile,
 // chunk, lane)

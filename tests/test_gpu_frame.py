@@ -189,17 +189,18 @@ def test_frame_start_batch_equals_starts(small, synth, q3h):
         b.destroy()
 
 
-@pytest.mark.parametrize("act_q8, lens", [
-    (0, [70, 16, 130, 65, 64, 1]),         # prompts of 65 rows or more join one pass
-    (1, [70, 16, 130, 65, 64, 1]),         # the int8 path: all of them
-    (1, [1900, 2001, 1999, 2000, 1500])])  # more rows than one pass takes
-def test_frame_start_batch_joined_prompts(device, synth, act_q8, lens):
+@pytest.mark.parametrize("act_q8, lens, dtype", [
+    (0, [70, 16, 130, 65, 64, 1], q3h.Q8_0),         # prompts of 65 rows or more join one pass
+    (0, [70, 40, 600, 465], q3h.F32),                # (32-query attention tiles)
+    (1, [70, 16, 130, 65, 64, 1], q3h.Q8_0),         # the int8 path: all of them
+    (1, [1900, 2001, 1999, 2000, 1500], q3h.Q8_0)])  # more rows than one pass takes
+def test_frame_start_batch_joined_prompts(device, synth, act_q8, lens, dtype):
     """Prompts run as the rows of one pass (start_group) leave the bits of one
     q3h_frame_start per stream: logits, states and the codes that follow."""
     print(f"case act_q8={act_q8} lens={lens}", flush=True)
     n, top = len(lens), max(lens) + 8
     m = Model(device, seed=23, talker_layers=2, cp_layers=1, act_q8=act_q8, norm_std=0.1,
-              max_positions=top)
+              max_positions=top, dtype=dtype)
     pres = [synth.prompt(170 + s, k) for s, k in enumerate(lens)]
     trs = [synth.normal(171 + s, "trailing", (s % 3, 1024), 0.02) if s % 3 else None
            for s in range(n)]

@@ -74,3 +74,69 @@ def test_q8_prefill_other_slice_counts(device):
         oc.destroy()
         st.destroy()
         ost.destroy()
+
+
+# Relative bar of the many-row products against the oracle's fp32 forward: sums
+# of up to 3072 fp32-exact products in another order, about sqrt(3072) * 2^-24 =
+# 3e-6 each, through the residual stream of one layer; 2e-5 leaves the softmax
+# and the norms their share.
+MANY_ROWS_BAR = 2e-5
+
+
+def _one_layer(device, dtype, positions, kv16=0):
+    dims = dict(synth.TALKER, layers=1)
+    quant = q3o.quantize_q8_0 if dtype == q3h.Q8_0 else None
+    layers, final = synth.stack_weights(47, "talker.model.", dims, norm_std=0.1, quantize=quant)
+    st = q3h.Stack(device, dict(dims, dtype=dtype, kv_f16=kv16, act_q8=0,
+                                max_positions=positions), layers, final, dtype)
+    odt = q3o.Q8_0 if dtype == q3h.Q8_0 else q3o.F32
+    return st, q3o.Stack(dims, layers, final, odt, kv_f16=kv16, act_q8=0)
+
+
+@pytest.mark.parametrize("f32", [0, 1], ids=["q8", "f32"])
+@pytest.mark.parametrize("rows", [65, 97, 203, 321, 1030])
+def test_many_row_tiles(device, f32, rows):
+    """The products over split activations (more than 64 rows) at row counts
+    that take each tile (32 x 64, 64 x 64, 64 x 128 by rounds of the chip),
+    last tiles of 1, 11 and 6 rows, and the 32-query attention tiles (1030):
+    the layer output of every row."""
+    print(f"case f32={f32} rows={rows}", flush=True)
+    st, ost = _one_layer(device, q3h.F32 if f32 else q3h.Q8_0, rows)
+    ctx, oc = q3h.Context(st, rows), q3o.Ctx(ost, rows)
+    try:
+        x = synth.prompt(720, rows)
+        _, normed, lo, _ = ctx.forward_probe(x)
+        onormed, olo = oc.forward(x, layer_out=True)
+        worst = max(rel(lo[0], olo[0]), rel(normed, onormed))
+        print(f"relative error {worst:.2e}", flush=True)
+        assert worst < MANY_ROWS_BAR, worst
+    finally:
+        ctx.destroy()
+        oc.destroy()
+        st.destroy()
+        ost.destroy()
+
+
+@pytest.mark.parametrize("f32", [0, 1], ids=["q8", "f32"])
+def test_many_contexts_one_row_each(device, f32):
+    """70 contexts of 1 to 5 positions, one row each in one call: the many-row
+    products behind the decode attention."""
+    n = 70
+    st, ost = _one_layer(device, q3h.F32 if f32 else q3h.Q8_0, 72)
+    ctxs = [q3h.Context(st, 8) for _ in range(n)]
+    octxs = [q3o.Ctx(ost, 8) for _ in range(n)]
+    try:
+        for i in range(n):
+            p = synth.prompt(730 + i, 1 + i % 5)
+            ctxs[i].forward(p, want_logits=False, want_normed=False)
+            octxs[i].forward(p)
+        x = synth.prompt(729, n)
+        _, normed = q3h.forward_batch(ctxs, x)
+        worst = max(rel(normed[i], octxs[i].forward(x[i:i + 1])) for i in range(n))
+        print(f"relative error {worst:.2e}", flush=True)
+        assert worst < MANY_ROWS_BAR, worst
+    finally:
+        for c in ctxs + octxs:
+            c.destroy()
+        st.destroy()
+        ost.destroy()
