@@ -1191,20 +1191,18 @@ void enqueue_forward(q3h_context *c, Work &w, int rows, int positions, int head,
   launch_advance(c->dev_arr, nullptr, 1, rows, st);
 }
 
-// the captured single-row forward of (head, cover) on c's Work buffers
-hipGraphExec_t forward_graph(q3h_context *c, int head, int positions) {
+// the graph of key among c's captured forwards on its Work buffers, captured
+// from enqueue() at its first use
+template <class F>
+hipGraphExec_t context_graph(q3h_context *c, uint64_t key, F &&enqueue) {
   constexpr size_t kMaxGraphs = 32;  // per context: a code predictor's heads, a talker's covers
   if (c->graphs_gen != c->w.gen || c->graphs.size() >= kMaxGraphs) {
     drop_graphs(c);
     c->graphs_gen = c->w.gen;
   }
-  const uint64_t key = ((uint64_t)(uint32_t)(head + 1) << 32) | (uint32_t)positions;
   for (auto &g : c->graphs)
     if (g.first == key) return g.second;
-  LayerIO io;
-  io.single_context = true;
-  hipGraph_t graph =
-      capture_graph(c->stream, [&] { enqueue_forward(c, c->w, 1, positions, head, io, c->stream); });
+  hipGraph_t graph = capture_graph(c->stream, enqueue);
   hipGraphExec_t exec = nullptr;
   const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
@@ -1213,36 +1211,53 @@ hipGraphExec_t forward_graph(q3h_context *c, int head, int positions) {
   return exec;
 }
 
+// the captured single-row forward of (head, cover) on c's Work buffers
+hipGraphExec_t forward_graph(q3h_context *c, int head, int positions) {
+  return context_graph(c, ((uint64_t)(uint32_t)(head + 1) << 32) | (uint32_t)positions, [&] {
+    LayerIO io;
+    io.single_context = true;
+    enqueue_forward(c, c->w, 1, positions, head, io, c->stream);
+  });
+}
+
+// c's pinned host staging of at least `floats` floats (c's stream idle)
+float *context_pin(q3h_context *c, size_t floats) {
+  if (c->pin_floats < floats) {
+    if (c->pin) check_hip(hipHostFree(c->pin), "hipHostFree");
+    c->pin = nullptr;
+    c->pin_floats = 0;
+    check_hip(hipHostMalloc((void **)&c->pin, sizeof(float) * floats, hipHostMallocDefault),
+              "hipHostMalloc");
+    c->pin_floats = floats;
+  }
+  return c->pin;
+}
+
 // TQwenLm.Forward on the work buffers w (sized for rows, the attention splits
 // of forward_positions and the head's rows), replayed from a captured graph
 // when graph: blocks until the outputs are in host memory
 void forward_rows(q3h_context *c, Work &w, const float *x, int rows, int head, float *logits,
                   float *normed_last, float *layer_out = nullptr, bool graph = false,
-                  float *normed_rows = nullptr) {
+                  float *normed_rows = nullptr, bool pinned = false) {
   q3h_stack *s = c->s;
   const q3h_stack_config &cf = s->cfg;
   const int H = cf.hidden;
   const int head_rows = head >= 0 ? s->heads[head].N : 0;
   const int positions = forward_positions(c, rows);
   hipStream_t st = c->stream;
-  // the replayed single-row forward copies through pinned host memory (a
-  // pageable copy is staged by the runtime on every call)
-  float *pin_x = nullptr, *pin_lg = nullptr, *pin_n = nullptr;
-  if (graph) {
-    const size_t need = (size_t)2 * H + head_rows;
-    if (c->pin_floats < need) {
-      if (c->pin) check_hip(hipHostFree(c->pin), "hipHostFree");
-      c->pin = nullptr;
-      c->pin_floats = 0;
-      check_hip(hipHostMalloc((void **)&c->pin, sizeof(float) * need, hipHostMallocDefault),
-                "hipHostMalloc");
-      c->pin_floats = need;
+  // results (and a single row) are copied through pinned host memory where the
+  // call may allocate it (a pageable copy is staged by the runtime, which waits
+  // for the stream at each: 10 us a copy)
+  float *pin_lg = nullptr, *pin_n = nullptr;
+  pinned = pinned || graph;
+  if (pinned) {
+    float *pin = context_pin(c, (size_t)2 * H + head_rows);
+    pin_n = pin + H;
+    pin_lg = pin + 2 * H;
+    if (rows == 1) {
+      std::memcpy(pin, x, sizeof(float) * H);
+      x = pin;
     }
-    pin_x = c->pin;
-    pin_n = c->pin + H;
-    pin_lg = c->pin + 2 * H;
-    std::memcpy(pin_x, x, sizeof(float) * H);
-    x = pin_x;
   }
   check_hip(hipMemcpyAsync(w.h, x, sizeof(float) * rows * H, hipMemcpyHostToDevice, st),
             "upload x");
@@ -1273,11 +1288,11 @@ void forward_rows(q3h_context *c, Work &w, const float *x, int rows, int head, f
                         st);
   check_hip(hipGetLastError(), "forward kernels");
   if (normed_last)
-    check_hip(hipMemcpyAsync(graph ? pin_n : normed_last, w.normed, sizeof(float) * H,
+    check_hip(hipMemcpyAsync(pinned ? pin_n : normed_last, w.normed, sizeof(float) * H,
                              hipMemcpyDeviceToHost, st),
               "download state");
   if (logits && head >= 0)
-    check_hip(hipMemcpyAsync(graph ? pin_lg : logits, w.logits, sizeof(float) * head_rows,
+    check_hip(hipMemcpyAsync(pinned ? pin_lg : logits, w.logits, sizeof(float) * head_rows,
                              hipMemcpyDeviceToHost, st),
               "download logits");
   if (layer_out)
@@ -1289,7 +1304,7 @@ void forward_rows(q3h_context *c, Work &w, const float *x, int rows, int head, f
                              hipMemcpyDeviceToHost, st),
               "download normed rows");
   check_hip(hipStreamSynchronize(st), "forward sync");
-  if (graph) {
+  if (pinned) {
     if (normed_last) std::memcpy(normed_last, pin_n, sizeof(float) * H);
     if (logits && head >= 0) std::memcpy(logits, pin_lg, sizeof(float) * head_rows);
   }
@@ -1307,7 +1322,7 @@ extern "C" int q3h_forward_embeds(q3h_context *c, const float *x, int rows, int 
     const int head_rows = head >= 0 ? s->heads[head].N : 0;
     c->w.ensure(s, rows, forward_splits(c, rows), head_rows);
     // one row (a decode step): the forward replayed from a captured graph
-    forward_rows(c, c->w, x, rows, head, logits, normed_last, nullptr, rows == 1);
+    forward_rows(c, c->w, x, rows, head, logits, normed_last, nullptr, rows == 1, nullptr, true);
   });
 }
 
@@ -1349,6 +1364,10 @@ extern "C" int q3h_forward_embeds_noalloc(q3h_context *c, const float *x, int ro
   });
 }
 
+// rows of a replayed batched forward (more run as direct launches; the key of
+// their graphs holds up to 2047 rows and 2^20 heads)
+constexpr int kBatchGraphRows = 256;
+
 extern "C" int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const float *x,
                                         const int *heads, float *logits, float *normed) {
   return guard([&] {
@@ -1380,42 +1399,68 @@ extern "C" int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const f
     check_hip(hipSetDevice(s->dev->ordinal), "hipSetDevice");
     for (int i = 1; i < n; i++) check_hip(hipStreamSynchronize(ctxs[i]->stream), "batch sync");
     const int H = cf.hidden;
+    // contexts of one size and one head: the launches replayed from a graph
+    // captured per (rows, head, cover), as the single-row forward's are (the
+    // contexts themselves are read from w.ctx_arr on the device)
+    bool same = true, replay = n <= kBatchGraphRows;
+    for (int i = 1; i < n; i++) {
+      same = same && (!heads || heads[i] == heads[0]);
+      replay = replay && ctxs[i]->max_pos == c0->max_pos;
+    }
+    replay = replay && same;
+    const int positions = replay ? graph_cover(maxlen, c0->max_pos) : maxlen;
     Work &w = c0->w;
-    w.ensure(s, n, attention_splits(s, maxlen), head_rows);
+    w.ensure(s, n, attention_splits(s, positions), head_rows);
     hipStream_t st = c0->stream;
-    std::vector<CtxDev *> arr(n);
-    for (int i = 0; i < n; i++) arr[i] = ctxs[i]->dev;
-    check_hip(hipMemcpyAsync(w.ctx_arr, arr.data(), sizeof(CtxDev *) * n, hipMemcpyHostToDevice,
-                             st),
-              "upload contexts");
-    check_hip(hipMemcpyAsync(w.h, x, sizeof(float) * n * H, hipMemcpyHostToDevice, st),
-              "upload x");
-    launch_prep(w.ctx_arr, nullptr, n, 1, w.rd, st);
-    run_layers(s, w, n, maxlen, true, st);
-    launch_rmsnorm_rows(w.h, H, n, H, s->final_norm, cf.rms_eps, w.normed, H, st);
-    if (heads) {
-      bool same = true;
-      for (int i = 1; i < n; i++) same = same && heads[i] == heads[0];
-      if (same) {
-        linear(s, w, s->heads[heads[0]], w.normed, H, n, nullptr, w.logits, head_rows,
-               EPI_STORE, nullptr, st);
-      } else {
+    auto enqueue = [&] {
+      launch_prep(w.ctx_arr, nullptr, n, 1, w.rd, st);
+      run_layers(s, w, n, positions, true, st);
+      launch_rmsnorm_rows(w.h, H, n, H, s->final_norm, cf.rms_eps, w.normed, H, st);
+      if (heads && same)
+        linear(s, w, s->heads[heads[0]], w.normed, H, n, nullptr, w.logits, head_rows, EPI_STORE,
+               nullptr, st);
+      else if (heads)
         for (int i = 0; i < n; i++)
           linear(s, w, s->heads[heads[i]], w.normed + (size_t)i * H, H, 1, nullptr,
                  w.logits + (size_t)i * head_rows, head_rows, EPI_STORE, nullptr, st);
-      }
+      launch_advance(w.ctx_arr, nullptr, n, 1, st);
+    };
+    const size_t nx = (size_t)n * H, nl = (size_t)n * head_rows;
+    std::vector<CtxDev *> arr(n);
+    for (int i = 0; i < n; i++) arr[i] = ctxs[i]->dev;
+    const CtxDev *const *src = arr.data();
+    float *lg = logits, *nm = normed;
+    if (replay) {  // through pinned host memory: [contexts | x | normed | logits]
+      check_hip(hipStreamSynchronize(st), "batch sync");
+      float *pin = context_pin(c0, 2 * (size_t)n + 2 * nx + nl);
+      std::memcpy(pin, arr.data(), sizeof(CtxDev *) * n);
+      std::memcpy(pin + 2 * n, x, sizeof(float) * nx);
+      src = reinterpret_cast<const CtxDev *const *>(pin);
+      x = pin + 2 * n;
+      nm = pin + 2 * n + nx;
+      lg = nm + nx;
     }
-    launch_advance(w.ctx_arr, nullptr, n, 1, st);
+    check_hip(hipMemcpyAsync(w.ctx_arr, src, sizeof(CtxDev *) * n, hipMemcpyHostToDevice, st),
+              "upload contexts");
+    check_hip(hipMemcpyAsync(w.h, x, sizeof(float) * nx, hipMemcpyHostToDevice, st), "upload x");
+    if (replay) {
+      const int head = heads ? heads[0] : -1;
+      const uint64_t key = (1ull << 63) | ((uint64_t)n << 52) |
+                           ((uint64_t)(uint32_t)(head + 1) << 32) | (uint32_t)positions;
+      check_hip(hipGraphLaunch(context_graph(c0, key, enqueue), st), "batch graph launch");
+    } else {
+      enqueue();
+    }
     check_hip(hipGetLastError(), "batch kernels");
     if (normed)
-      check_hip(hipMemcpyAsync(normed, w.normed, sizeof(float) * n * H, hipMemcpyDeviceToHost,
-                               st),
+      check_hip(hipMemcpyAsync(nm, w.normed, sizeof(float) * nx, hipMemcpyDeviceToHost, st),
                 "download states");
     if (logits && heads)
-      check_hip(hipMemcpyAsync(logits, w.logits, sizeof(float) * n * head_rows,
-                               hipMemcpyDeviceToHost, st),
+      check_hip(hipMemcpyAsync(lg, w.logits, sizeof(float) * nl, hipMemcpyDeviceToHost, st),
                 "download logits");
     check_hip(hipStreamSynchronize(st), "batch sync");
+    if (replay && normed) std::memcpy(normed, nm, sizeof(float) * nx);
+    if (replay && logits && heads) std::memcpy(logits, lg, sizeof(float) * nl);
     for (int i = 0; i < n; i++) ctxs[i]->len += 1;
   });
 }

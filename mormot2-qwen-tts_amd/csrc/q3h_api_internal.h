@@ -215,12 +215,14 @@ struct q3h_context {
   q3h::Work w;
   float *probe = nullptr;  // the layer outputs of q3h_forward_embeds_probe
   size_t probe_bytes = 0;
-  // the captured single-row forwards, keyed by (head + 1) << 32 | cover, valid
-  // for the Work buffers of generation graphs_gen
+  // the captured single-row forwards, keyed by (head + 1) << 32 | cover, and
+  // the batched forwards this context leads (bit 63 and the rows besides),
+  // valid for the Work buffers of generation graphs_gen
   std::vector<std::pair<uint64_t, hipGraphExec_t>> graphs;
   unsigned graphs_gen = 0;
-  // pinned host staging of a single-row forward: the input row, the logits,
-  // the normed state (hipHostMalloc'ed on first use, pin_floats floats)
+  // pinned host staging of a forward: the input row, the normed state, the
+  // logits (a batched one: contexts, rows, states, logits); hipHostMalloc'ed on
+  // first use, pin_floats floats, at most those of kBatchGraphRows rows
   float *pin = nullptr;
   size_t pin_floats = 0;
 };

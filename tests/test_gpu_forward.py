@@ -143,6 +143,40 @@ def test_batch_equals_single(q8model, q3h, synth):
         c.destroy()
 
 
+def test_batch_replays_follow_the_contexts(q8model, q3h, synth):
+    """Batched forwards replay a graph captured per (rows, head, position
+    cover) on the first context's buffers: steps across a cover's end (62 to 66
+    positions), with the other contexts in a new order and single-row forwards
+    of the first between them, with and without a head, against contexts run
+    one by one; contexts of another size run as direct launches."""
+    m = q8model
+    lens = [60, 41, 61]
+    a = [q3h.Context(m.ts, 128) for _ in lens]
+    b = [q3h.Context(m.ts, 128) for _ in lens]
+    odd, odd_b = q3h.Context(m.ts, 64), q3h.Context(m.ts, 64)
+    try:
+        for i, n in enumerate(lens):
+            for c in (a[i], b[i]):
+                c.forward(synth.prompt(30 + i, n), want_normed=False)
+        for step in range(6):
+            order = [0, 1, 2] if step % 2 else [0, 2, 1]
+            ca, cb = [a[i] for i in order], [b[i] for i in order]
+            if step == 5:
+                ca, cb = ca + [odd], cb + [odd_b]
+            x = synth.prompt(140 + step, len(ca))
+            heads = None if step == 3 else [0] * len(ca)
+            lg, normed = q3h.forward_batch(ca, x, heads=heads)
+            for i, c in enumerate(cb):
+                l1, n1 = c.forward(x[i], head=0)
+                assert rel(normed[i], n1) < 1e-6, (step, i)
+                assert heads is None or rel(lg[i], l1) < 1e-6, (step, i)
+            one = synth.prompt(150 + step, 1)
+            assert rel(a[0].forward(one, head=0)[0], b[0].forward(one, head=0)[0]) < 1e-6, step
+    finally:
+        for c in a + b + [odd, odd_b]:
+            c.destroy()
+
+
 def test_graph_forward_equals_direct(q8model, q3h, synth):
     """A one-row q3h_forward_embeds replays a graph captured per (head,
     position cover); the no-alloc forward launches the same kernels directly.
