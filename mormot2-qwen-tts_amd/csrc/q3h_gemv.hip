@@ -115,14 +115,13 @@ __global__ __launch_bounds__(1024) void k_gemv_q8v(const int8_t *__restrict__ wq
       sc[r][c] = (float)d[c * 32];
     }
   }
-  float yres[MR][R];
-  if (EPI == EPI_ADD) {
-#pragma unroll
-    for (int m = 0; m < MR; m++)
-#pragma unroll
-      for (int r = 0; r < R; r++)
-        yres[m][r] = y[(MR == 1 ? 0 : (size_t)min(m, M - 1) * ldy) + min(row0 + r, N - 1)];
-  }
+  // lane o < MR RO finishes output o: activation row o / RO, weight row (SwiGLU:
+  // row pair) o % RO of the wave
+  constexpr int RO = EPI == EPI_SWIGLU ? R / 2 : R;
+  const int mo = MR == 1 ? 0 : lane / RO, ro = MR == 1 ? lane : lane % RO;
+  float yres = 0.f;
+  if (EPI == EPI_ADD)
+    yres = y[(MR == 1 ? 0 : (size_t)min(mo, M - 1) * ldy) + min(row0 + ro, N - 1)];
   // every load above is issued before any arithmetic
   __builtin_amdgcn_sched_barrier(0);
   if (NP > 0) {
@@ -211,33 +210,33 @@ __global__ __launch_bounds__(1024) void k_gemv_q8v(const int8_t *__restrict__ wq
       }
     }
   }
+  // every sum is uniform: each lane takes its output's, so one SwiGLU and one
+  // store serve them all (lane 0 finishing 8 SwiGLU outputs of four rows one
+  // after another was 0.4 us of the gate/up product)
+  float v = 0.f, u = 0.f, iv = inv[0];
 #pragma unroll
   for (int m = 0; m < MR; m++)
 #pragma unroll
-    for (int r = 0; r < R; r++) acc[m][r] = wave_sum_dpp(acc[m][r]) * inv[m];
-  if (lane != 0 || row0 >= N) return;
-#pragma unroll
-  for (int m = 0; m < MR; m++) {
-    if (MR > 1 && m >= M) break;
-    float *ym = MR == 1 ? y : y + (size_t)m * ldy;
-    if (EPI == EPI_SWIGLU) {
-#pragma unroll
-      for (int p = 0; p < R / 2; p++) {
-        const float g = acc[m][2 * p], u = acc[m][2 * p + 1];
-        ym[row0 / 2 + p] = g / (1.0f + expf(-g)) * u;
+    for (int o = 0; o < RO; o++) {
+      const bool mine = lane == m * RO + o;
+      if (EPI == EPI_SWIGLU) {
+        const float g = wave_sum_dpp(acc[m][2 * o % R]), w = wave_sum_dpp(acc[m][(2 * o + 1) % R]);
+        v = mine ? g : v;
+        u = mine ? w : u;
+      } else {
+        const float g = wave_sum_dpp(acc[m][o]);
+        v = mine ? g : v;
       }
-    } else {
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        if (row0 + r < N) {
-          if (EPI == EPI_ADD)
-            ym[row0 + r] = yres[m][r] + acc[m][r];
-          else
-            ym[row0 + r] = acc[m][r];
-        }
-      }
+      if (MR > 1) iv = mine ? inv[m] : iv;
     }
-  }
+  v *= iv;
+  u *= iv;
+  if (lane >= MR * RO || row0 + (EPI == EPI_SWIGLU ? 2 : 1) * ro >= N || (MR > 1 && mo >= M)) return;
+  float *ym = MR == 1 ? y : y + (size_t)mo * ldy;
+  if (EPI == EPI_SWIGLU)
+    ym[row0 / 2 + ro] = v / (1.0f + expf(-v)) * u;
+  else
+    ym[row0 + ro] = EPI == EPI_ADD ? yres + v : v;
 }
 
 // The single-row product (EPI_STORE, RMSNorm prologue) whose activation row
@@ -356,18 +355,20 @@ __global__ __launch_bounds__(W * 64) void k_gemv_q8v_code(
       acc[r] = fmaf(sc[r][c], p0 + p1, acc[r]);
     }
   }
+  float v = 0.f;
 #pragma unroll
-  for (int r = 0; r < R; r++) acc[r] = wave_sum_dpp(acc[r]) * inv;
+  for (int r = 0; r < R; r++) {
+    const float w = wave_sum_dpp(acc[r]);
+    v = lane == r ? w : v;
+  }
+  v *= inv;
   // the code and the raw row, after every load of the product has been used
   if (blockIdx.x == 0 && *alive) {
     if (tid == 0) *code_out = code;
 #pragma unroll
     for (int j = 0; j < C; j++) reinterpret_cast<float4 *>(h_out)[tid + 256 * j] = xv[j];
   }
-  if (lane != 0 || row0 >= N) return;
-#pragma unroll
-  for (int r = 0; r < R; r++)
-    if (row0 + r < N) y[row0 + r] = acc[r];
+  if (lane < R && row0 + lane < N) y[row0 + lane] = v;
 }
 
 // ev0 / ev1 (optional): events recorded at the start and the end of the
@@ -508,10 +509,16 @@ bool launch_gemv_q8_wide(const GemvArgs &a, int epi, hipStream_t st, hipEvent_t 
   const int rpb = a.N / 256;  // rows per workgroup, 256 workgroups
   // measured on the Qwen3-TTS shapes, for one row and for two: one wave per
   // SIMD (R = rpb / 4 rows per wave) for the plain products; the gate/up
-  // pairs (SwiGLU) as 4-row waves (6 per workgroup: 3.47 us per launch against
-  // 3.78 for 2-row waves at one row, 4.45 against 4.54 at two)
+  // pairs (SwiGLU) as 4-row waves (6 per workgroup: 3.33 us per launch against
+  // 3.70 for 2-row waves at one row, 4.01 against 4.20 at two), at three and four
+  // activation rows as 2-row waves (5.43 against 5.65; with one lane finishing
+  // every output 6.61)
   int R1 = rpb / 4, W = 4;
   if (epi == EPI_SWIGLU && !swiglu_shape(a.N, R1, W)) return false;
+  if (epi == EPI_SWIGLU && a.M > 2 && R1 == 4 && 2 * W <= kMaxWaves) {
+    R1 = 2;
+    W *= 2;
+  }
   if (R1 < 1 || R1 * W != rpb || W > kMaxWaves) return false;
   if (a.M == 1) return launch_rows<1>(a, epi, R1, W, st, ev0, ev1);
   if (W < 4) return false;  // more rows: 4 loader waves
