@@ -322,7 +322,7 @@ __device__ __forceinline__ void chunk_chains(const int8_t *wq, const int8_t *xq,
 // chains land in their own LDS slot, and the slots are added in chunk order.
 // EPI_SWIGLU: rows 2j / 2j + 1 are gate / up of output j.
 template <int TM, int KW, int EPI>
-__global__ __launch_bounds__(KW * 64) void k_gemm_i8(const int8_t *wq, const int8_t *xq,
+__global__ __launch_bounds__(KW * 64, 2) void k_gemm_i8(const int8_t *wq, const int8_t *xq,
                                                       float *y, int N, int K, int M, int ldy) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -498,7 +498,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_i8r(const int8_t *wq, const int
 // multiple of 8 for the Qwen3-TTS shapes), so they run on one XCD and share
 // the weight tile through its L2.
 template <int TM>
-__global__ __launch_bounds__(64) void k_gemm_i8p(const int8_t *wq, const int8_t *xq,
+__global__ __launch_bounds__(64, 2) void k_gemm_i8p(const int8_t *wq, const int8_t *xq,
                                                   float *part, int N, int K, int M) {
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int n0 = blockIdx.x * 16, ch = blockIdx.y, mt0 = blockIdx.z * TM;

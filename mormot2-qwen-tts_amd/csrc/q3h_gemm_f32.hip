@@ -490,6 +490,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_x3(const void *__restrict__ wp,
     constexpr int b = decltype(buf)::value;
 #pragma unroll
     for (int k = 0; k < KC; k++) {
+      // (the operands of one chunk at a time: both took all 256 registers)
+      if (KC > 1 && k) __builtin_amdgcn_sched_barrier(0);
       bf8v x[MT][3];
 #pragma unroll
       for (int i = 0; i < MT; i++)
