@@ -232,7 +232,11 @@ struct q3h_text_proj {
   q3h_device *dev = nullptr;
   q3h_text_config cfg{};
   void *emb = nullptr;  // [text_vocab][text_hidden], BF16 or f32
-  q3h::Mat fc1, fc2;    // f32
+  q3h::Mat fc1, fc2;    // f32; as split operand tiles only (x3) when split
+  // both products over split operands, K in kTextSlices slices (widths that are
+  // multiples of 64 and 512): e and h hold operand tiles, part the slices' sums
+  bool split = false;
+  float *part = nullptr;
   float *b1 = nullptr, *b2 = nullptr;
   int cap = 0;               // rows of the work buffers
   int32_t *ids = nullptr;    // [cap]

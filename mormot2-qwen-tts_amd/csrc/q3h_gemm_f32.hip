@@ -41,11 +41,6 @@ __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast
 
 __device__ __forceinline__ float silu_mul_f(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
-// SiLU of the text projection: 0 below -80 (where e^-v would overflow)
-__device__ __forceinline__ float silu_clamp_f(float v) {
-  return v < -80.0f ? 0.0f : v / (1.0f + expf(-v));
-}
-
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 
@@ -857,12 +852,13 @@ void launch_gemm_x3_swiglu(const Mat &W, const uint16_t *x3, int M, uint16_t *y3
     launch_x3<false, EPI_SWIGLU>(W, x3, M, 1, nullptr, 0, y3, st);
 }
 
-int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hipStream_t st) {
+int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hipStream_t st,
+                        int ks) {
   if (W.q)
-    launch_x3<true, EPI_PART>(W, x3, M, kF32Slices, part, W.N, nullptr, st);
+    launch_x3<true, EPI_PART>(W, x3, M, ks, part, W.N, nullptr, st);
   else
-    launch_x3<false, EPI_PART>(W, x3, M, kF32Slices, part, W.N, nullptr, st);
-  return kF32Slices;
+    launch_x3<false, EPI_PART>(W, x3, M, ks, part, W.N, nullptr, st);
+  return ks;
 }
 
 void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, hipStream_t st) {

@@ -117,7 +117,7 @@ __global__ __launch_bounds__(1024) void k_gemv_q8v(const int8_t *__restrict__ wq
   }
   // lane o < MR RO finishes output o: activation row o / RO, weight row (SwiGLU:
   // row pair) o % RO of the wave
-  constexpr int RO = EPI == EPI_SWIGLU ? R / 2 : R;
+  constexpr int RO = EPI == EPI_SWIGLU ? (R + 1) / 2 : R;
   const int mo = MR == 1 ? 0 : lane / RO, ro = MR == 1 ? lane : lane % RO;
   float yres = 0.f;
   if (EPI == EPI_ADD)

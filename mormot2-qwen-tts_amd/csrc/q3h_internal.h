@@ -149,15 +149,16 @@ void launch_split3(const Mat &m, hipStream_t st);
 // The products over more than kManyRows rows whose activations are split into
 // operand tiles (x3_offset, q3h_x3.h; x3_bytes(M, K)) by the kernel that makes
 // them: y [M][ldy] = W . x; silu(gate) * up of interleaved rows into the tiles
-// y3 of the next product; the kF32Slices slices of K (returned) to part
-// [slices][M][N]. A row's sums do not depend on the row count. Q8_0 weights,
+// y3 of the next product; the ks slices of K (returned) to part [ks][M][N]. A row's sums do not depend on the row count. Q8_0 weights,
 // or f32 ones with Mat::x3.
 constexpr int kManyRows = 64;
+constexpr int kF32Slices = 4;  // K slices of o_proj and down
 inline size_t x3_bytes(size_t M, size_t K) { return (M + 15) / 16 * 16 * K * 6; }
 bool gemm_x3_supported(const Mat &W, int ks);
 void launch_gemm_x3(const Mat &W, const uint16_t *x3, int M, float *y, int ldy, hipStream_t st);
 void launch_gemm_x3_swiglu(const Mat &W, const uint16_t *x3, int M, uint16_t *y3, hipStream_t st);
-int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hipStream_t st);
+int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hipStream_t st,
+                        int ks = kF32Slices);
 // rows x [M][ldx] split into operand tiles
 void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, hipStream_t st);
 constexpr int kGemvRows = 4;
@@ -171,7 +172,6 @@ void launch_gemm_f32(const Mat &W, const float *x, int ldx, int M, int epi, floa
 // a quarter or less of the rows' activations (48 rows: q/k/v 11.1 -> 7.3 us,
 // o_proj 7.9 -> 5.3 us, down 9.7 -> 7.2 us); kF32Slices slices otherwise.
 // Returns the slice count.
-constexpr int kF32Slices = 4;
 constexpr int kQ8SliceRows = 64;
 constexpr int kMaxPartSlices = 12;  // the most 256-column slices of a product
 bool gemm_f32_slices_supported(int N, int K);

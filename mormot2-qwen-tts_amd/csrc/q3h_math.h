@@ -36,6 +36,11 @@ __device__ __forceinline__ float silu_mul_ieee(float g, float u) {
   return __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, exp_ieee(-g))), u);
 }
 
+// SiLU of the text projection: 0 below -80 (where e^-v would overflow)
+__device__ __forceinline__ float silu_clamp_f(float v) {
+  return v < -80.0f ? 0.0f : v / (1.0f + expf(-v));
+}
+
 // sinf, kept out of line
 __device__ __attribute__((noinline)) inline float sin_far(float x) { return sinf(x); }
 

@@ -2,21 +2,27 @@
 // (TQwenTalker.TextProject, src/tts/mormot.ai.tts.qwen.talker.pas:390-421):
 // y[r] = fc2 . SiLU(fc1 . emb[ids[r]] + b1) + b2, SiLU(v) = 0 below -80.
 //
-// Three launches over all n rows at once:
-//  1. k_text_rows: row r of the embedding widened to f32 (BF16 is the high
-//     half of an f32: exact), and the biases written where the products add:
-//     h[r] = b1, y[r] = b2;
-//  2. fc1 on the f32 matrix cores, epilogue h = SiLU(h + sum) (EPI_ADD_SILU);
-//  3. fc2 on the f32 matrix cores, epilogue y += sum (EPI_ADD).
-// Weights and products stay in f32 (the reference's idtF32 products). The
-// embedding table stays in the dtype it came in (BF16: 622 MB for 151936 x
+// Five launches over all n rows at once: the rows of the embedding (BF16 is the
+// high half of an f32: exact) split into operand tiles (k_text_rows); fc1 on
+// the bf16 matrix cores with both operands split exactly (k_gemm_x3), K in 8
+// slices so that its workgroups fill the chip at the row counts of a prompt;
+// the slices added to b1, SiLU, split for fc2 (k_text_mid); fc2; the slices
+// added to b2 (k_text_end). The products are exact to the fp32 rounding of
+// their sums (the reference's idtF32 products). 48 rows: 48 us of kernels as
+// three launches on the f32 matrix cores, whose 128 and 64 workgroups walked
+// all of K (23 + 20 us); widths that are no multiples of 64 and 512 still take
+// those: e = the rows, h = b1, y = b2, then fc1 with h = SiLU(h + sum)
+// (EPI_ADD_SILU) and fc2 with y += sum (EPI_ADD). The embedding table stays in the dtype it came in (BF16: 622 MB for 151936 x
 // 2048), gathered one row per token.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 
 #include "q3h_api_internal.h"
+#include "q3h_math.h"
+#include "q3h_x3.h"
 
 namespace q3h {
 namespace {
@@ -54,10 +60,87 @@ __global__ __launch_bounds__(256) void k_text_rows(const void *__restrict__ emb,
   for (int i = t; i < H; i += 256) yr[i] = b2[i];
 }
 
+constexpr int kTextSlices = 8;
+
+// one workgroup per row: emb[ids[r]] split into operand tiles (TH % 32 == 0)
+template <bool BF16>
+__global__ __launch_bounds__(256) void k_text_rows_x3(const void *__restrict__ emb,
+                                                      const int32_t *__restrict__ ids, int TH,
+                                                      uint16_t *__restrict__ e) {
+  const int r = blockIdx.x;
+  const size_t id = (size_t)ids[r];
+  for (int k = 8 * threadIdx.x; k < TH; k += 8 * 256) {
+    float v[8];
+    if (BF16) {
+      const uint4 u = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(emb) + id * TH + k);
+      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[2 * i] = bf_lo(w[i]), v[2 * i + 1] = bf_hi(w[i]);
+    } else {
+      const float4 *s = reinterpret_cast<const float4 *>(static_cast<const float *>(emb) + id * TH + k);
+      const float4 a = s[0], b = s[1];
+      v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    }
+    x3_store8(e, r, k, TH, v);
+  }
+}
+
+// 4 columns per thread: the slices' sums added in order, then to the bias
+__device__ __forceinline__ void text_sum4(const float *__restrict__ part,
+                                          const float *__restrict__ b, int M, int N, int m, int k,
+                                          float (&v)[4]) {
+  float4 p[kTextSlices];
+#pragma unroll
+  for (int s = 0; s < kTextSlices; s++)
+    p[s] = *reinterpret_cast<const float4 *>(part + ((size_t)s * M + m) * N + k);
+  const float4 bias = *reinterpret_cast<const float4 *>(b + k);
+  float4 a = p[0];
+#pragma unroll
+  for (int s = 1; s < kTextSlices; s++) a.x += p[s].x, a.y += p[s].y, a.z += p[s].z, a.w += p[s].w;
+  v[0] = bias.x + a.x, v[1] = bias.y + a.y, v[2] = bias.z + a.z, v[3] = bias.w + a.w;
+}
+
+// h = SiLU(b1 + sum), split
+__global__ __launch_bounds__(256) void k_text_mid(const float *__restrict__ part,
+                                                  const float *__restrict__ b1, int M, int TH,
+                                                  uint16_t *__restrict__ h) {
+  const int i = blockIdx.x * 256 + threadIdx.x, m = i / (TH / 4), k = 4 * (i - m * (TH / 4));
+  if (m >= M) return;
+  float v[4];
+  text_sum4(part, b1, M, TH, m, k, v);
+#pragma unroll
+  for (int e = 0; e < 4; e++) v[e] = silu_clamp_f(v[e]);
+  x3_store4(h, m, k, TH, v);
+}
+
+// y = b2 + sum
+__global__ __launch_bounds__(256) void k_text_end(const float *__restrict__ part,
+                                                  const float *__restrict__ b2, int M, int H,
+                                                  float *__restrict__ y, int ldy) {
+  const int i = blockIdx.x * 256 + threadIdx.x, m = i / (H / 4), k = 4 * (i - m * (H / 4));
+  if (m >= M) return;
+  float v[4];
+  text_sum4(part, b2, M, H, m, k, v);
+  *reinterpret_cast<float4 *>(y + (size_t)m * ldy + k) = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// w as split operand tiles instead of f32
+void split_weights(Mat &w, hipStream_t st) {
+  w.x3 = (uint16_t *)dev_alloc((size_t)3 * w.N * w.K * 2);
+  launch_split3(w, st);
+  check_hip(hipGetLastError(), "split3");
+  check_hip(hipStreamSynchronize(st), "split sync");
+  dev_free(w.f);
+  w.f = nullptr;
+}
+
 void text_release(q3h_text_proj *t) {
   dev_free(t->emb);
   dev_free(t->fc1.f);
   dev_free(t->fc2.f);
+  dev_free(t->fc1.x3);
+  dev_free(t->fc2.x3);
+  dev_free(t->part);
   dev_free(t->b1);
   dev_free(t->b2);
   dev_free(t->ids);
@@ -85,13 +168,15 @@ void text_ensure(q3h_text_proj *t, int n) {
   dev_free(t->e);
   dev_free(t->h);
   dev_free(t->y);
+  dev_free(t->part);
   t->ids = nullptr;
-  t->e = t->h = t->y = nullptr;
+  t->e = t->h = t->y = t->part = nullptr;
   t->cap = 0;
   const size_t TH = t->cfg.text_hidden, H = t->cfg.hidden;
   t->ids = (int32_t *)dev_alloc(sizeof(int32_t) * cap);
-  t->e = (float *)dev_alloc(sizeof(float) * cap * TH);
-  t->h = (float *)dev_alloc(sizeof(float) * cap * TH);
+  t->e = (float *)dev_alloc(t->split ? x3_bytes(cap, TH) : sizeof(float) * cap * TH);
+  t->h = (float *)dev_alloc(t->split ? x3_bytes(cap, TH) : sizeof(float) * cap * TH);
+  if (t->split) t->part = (float *)dev_alloc(sizeof(float) * kTextSlices * cap * std::max(TH, H));
   t->y = (float *)dev_alloc(sizeof(float) * cap * H);
   t->cap = cap;
 }
@@ -100,6 +185,20 @@ void text_project_dev(q3h_text_proj *t, const int32_t *ids_dev, int n, float *y,
                       hipStream_t st) {
   const q3h_text_config &c = t->cfg;
   const int TH = c.text_hidden, H = c.hidden;
+  if (t->split) {
+    uint16_t *e = reinterpret_cast<uint16_t *>(t->e), *h = reinterpret_cast<uint16_t *>(t->h);
+    if (c.emb_dtype == Q3H_BF16)
+      hipLaunchKernelGGL(k_text_rows_x3<true>, dim3(n), dim3(256), 0, st, t->emb, ids_dev, TH, e);
+    else
+      hipLaunchKernelGGL(k_text_rows_x3<false>, dim3(n), dim3(256), 0, st, t->emb, ids_dev, TH, e);
+    auto blocks = [&](int N) { return dim3((unsigned)(((size_t)n * (N / 4) + 255) / 256)); };
+    launch_gemm_x3_part(t->fc1, e, n, t->part, st, kTextSlices);
+    hipLaunchKernelGGL(k_text_mid, blocks(TH), dim3(256), 0, st, t->part, t->b1, n, TH, h);
+    launch_gemm_x3_part(t->fc2, h, n, t->part, st, kTextSlices);
+    hipLaunchKernelGGL(k_text_end, blocks(H), dim3(256), 0, st, t->part, t->b2, n, H, y, ldy);
+    check_hip(hipGetLastError(), "text projection kernels");
+    return;
+  }
   if (c.emb_dtype == Q3H_BF16)
     hipLaunchKernelGGL(k_text_rows<true>, dim3(n), dim3(256), 0, st, t->emb, ids_dev, TH, H,
                        t->b1, t->b2, t->e, t->h, y, ldy);
@@ -146,8 +245,15 @@ extern "C" int q3h_text_create(q3h_device *dev, const q3h_text_config *cfg, cons
     t->fc2.f = upload(fc2_w, H * TH, "fc2_w");
     t->b1 = upload(fc1_b, TH, "fc1_b");
     t->b2 = upload(fc2_b, H, "fc2_b");
-    t->bytes = (int64_t)(es * c.text_vocab * TH + 4 * (TH * TH + H * TH + TH + H));
     check_hip(hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking), "hipStreamCreate");
+    // slices of whole 64-column steps, 16-byte rows
+    t->split = H % 64 == 0 && TH % (64 * kTextSlices) == 0;
+    if (t->split) {
+      split_weights(t->fc1, t->stream);
+      split_weights(t->fc2, t->stream);
+    }
+    t->bytes = (int64_t)(es * c.text_vocab * TH + (t->split ? 6 : 4) * (TH * TH + H * TH) +
+                         4 * (TH + H));
     dev->bytes += t->bytes;
     dev->stacks++;
     *out = t;

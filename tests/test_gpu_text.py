@@ -34,8 +34,8 @@ def _oracle(tables, ids):
 
 @pytest.mark.parametrize("n", [1, 3, 16, 17, 40, 100, 520])
 def test_text_project_parity(proj, tables, n):
-    # 1..16 rows: 16-row tiles; 17..32: 32-row tiles; 40, 100: 64-row tiles of
-    # the K-split kernel; 520: fc1 on the 64-row full-K kernel
+    # the products over split operands, 32- and 64-row tiles of 64 and 128 columns
+    # by the rounds of the chip their 8 K slices make
     rng = np.random.default_rng(n)
     ids = rng.integers(0, TV, n).astype(np.int32)
     ids[n // 2] = ids[0]  # a repeated token
@@ -46,6 +46,25 @@ def test_text_project_parity(proj, tables, n):
     assert rel(y, ref) < 1e-4, rel(y, ref)
     # rows are independent: a repeated token gives the same row within the bar
     assert rel(y[n // 2], ref[0]) < 1e-4
+
+
+@pytest.mark.parametrize("hidden", [32, 192], ids=["f32_products", "split_products"])
+def test_text_project_other_widths(device, hidden):
+    """Widths on both sides of the split products' rule (hidden a multiple of
+    64): 1024 text columns, 7 and 70 rows."""
+    rng = np.random.default_rng(hidden)
+    emb = (rng.standard_normal((64, 1024)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    tables = (emb, rng.standard_normal((1024, 1024), np.float32) * np.float32(0.02),
+              rng.standard_normal(1024, np.float32) * np.float32(0.02),
+              rng.standard_normal((hidden, 1024), np.float32) * np.float32(0.02),
+              rng.standard_normal(hidden, np.float32) * np.float32(0.02))
+    p = q3h.TextProj(device, *tables)
+    try:
+        for n in (7, 70):
+            ids = rng.integers(0, 64, n).astype(np.int32)
+            assert rel(p.project(ids), _oracle(tables, ids)) < 2e-5, n
+    finally:
+        p.destroy()
 
 
 def test_text_project_f32_table(device, tables):
