@@ -148,8 +148,9 @@ int q3h_context_time_attention(q3h_context *c, int iters, float *us_per_launch,
    replays a HIP graph the context captures per (head, position cover)
    (covers of 64 positions up to 256, of 256 beyond; at most 32 graphs per
    context, dropped when its work buffers grow) and copies its row, logits
-   and state through a pinned host buffer of the context; the results are
-   those of the same launches made directly (q3h_forward_embeds_noalloc). ---- */
+   and state through a pinned host buffer of the context (several rows: the
+   logits and state); the results are those of the same launches made
+   directly (q3h_forward_embeds_noalloc). ---- */
 int q3h_forward_embeds(q3h_context *c, const float *x, int rows, int head,
                        float *logits, float *normed_last);
 
@@ -192,7 +193,10 @@ int q3h_forward_embeds_probe(q3h_context *c, const float *x, int rows, int head,
    context, n contexts of the same stack at their own positions;
    x [n][hidden]; heads [n] (or NULL: no logits); logits [n][head rows of
    heads[0]] (all heads of one call must have the same rows); normed [n][hidden]
-   (nullable). */
+   (nullable). Up to 256 contexts of one max_positions with one head: replayed
+   from a HIP graph that ctxs[0] captures per (n, head, position cover of the
+   longest context), the contexts read on the device, so any contexts of the
+   same n may follow. */
 int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const float *x,
                              const int *heads, float *logits, float *normed);
 
@@ -225,9 +229,11 @@ int q3h_frame_create(q3h_stack *talker, q3h_stack *cp, const q3h_frame_config *c
 int q3h_frame_start(q3h_frame *f, int stream, const float *prefill, int rows,
                     const float *trailing, int trailing_rows);
 /* no reference counterpart (batched serving; the reference starts one
-   sentence at a time): q3h_frame_start for n distinct streams at once, each
-   prefill on its stream's own talker context and HIP stream so that the
-   prefills overlap on the device; blocks until all are done. streams [n];
+   sentence at a time): q3h_frame_start for n distinct streams at once. The
+   prompts of an int8 stack, and those over 64 rows of the others, run as the
+   rows of one pass (of at most 8192 rows; further passes follow); the rest
+   each on its stream's own talker context and HIP stream, so that they overlap
+   on the device; blocks until all are done. streams [n];
    prefill[i] [rows[i]][hidden]; trailing (nullable) and trailing_rows
    (nullable: none) as q3h_frame_start's per stream. The results equal n
    calls of q3h_frame_start. Every argument is checked before any prefill is
