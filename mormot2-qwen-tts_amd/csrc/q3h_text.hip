@@ -252,6 +252,7 @@ extern "C" int q3h_text_create(q3h_device *dev, const q3h_text_config *cfg, cons
       split_weights(t->fc1, t->stream);
       split_weights(t->fc2, t->stream);
     }
+    text_ensure(t, 1);  // the first call's workspace: 0.3 ms of allocations
     t->bytes = (int64_t)(es * c.text_vocab * TH + (t->split ? 6 : 4) * (TH * TH + H * TH) +
                          4 * (TH + H));
     dev->bytes += t->bytes;
