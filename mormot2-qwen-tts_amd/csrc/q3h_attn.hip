@@ -941,7 +941,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 &h, u32x4 &m, 
 // acc += A B for f32 operands given as three bf16 parts each: the six part
 // products of weight at least 2^-16 of the product (mid mid, lo hi, hi lo,
 // mid hi, hi mid, hi hi, smallest first), each exact in fp32; the three
-// dropped weigh below 2^-23 of the product, under its fp32 rounding
+// dropped weigh up to 2^-21 of the product (4e-8 on average), all of its sign
 __device__ __forceinline__ v4f mfma_x3(const u32x4 (&a)[3], const u32x4 (&b)[3], v4f acc) {
   const bf8v ah = __builtin_bit_cast(bf8v, a[0]), am = __builtin_bit_cast(bf8v, a[1]),
              al = __builtin_bit_cast(bf8v, a[2]);

@@ -82,8 +82,9 @@ __device__ __forceinline__ void rope_pair(float &a, float &b, float c, float s) 
 
 // x = hi + mid + lo exactly, each a bf16 (returned as its 16 bits in the low
 // half): hi the top 8 significant bits of x, mid the next 8, lo the last 8
-// (an f32 significand has 24; each difference is exact in f32). The
-// operands of the split-bf16 matrix-core products.
+// (an f32 significand has 24; each difference is exact in f32). For products
+// whose other operand is exact in bf16 (all three part products are summed);
+// where part products are dropped, the parts are rounded: split3_rn.
 __device__ __forceinline__ void split3(float x, uint32_t &h, uint32_t &m, uint32_t &l) {
   const uint32_t u = __float_as_uint(x);
   const uint32_t hb = u & 0xffff0000u;
@@ -93,6 +94,29 @@ __device__ __forceinline__ void split3(float x, uint32_t &h, uint32_t &m, uint32
   h = hb >> 16;
   m = mb >> 16;
   l = __float_as_uint(r2) >> 16;
+}
+
+// The same for a (low halves) and b (high halves), hi and mid rounded to
+// nearest: |mid| <= 2^-9 and |lo| <= 2^-18 of the binade's top, of either sign,
+// so the part products below hi lo that a six-part product leaves out (mid lo,
+// lo mid, lo lo) weigh at most 2^-24 of it and cancel on average. Cut off
+// instead of rounded (split3) they reach 2^-21 and all have the product's sign:
+// a product of one term 9.2e-8 off (RMS) instead of 3.6e-8. As many
+// instructions (the pair conversion of gfx950 packs as it rounds) and one more
+// per value: hi of a value within half a bf16 step of the largest float would
+// round to infinity, so it is taken of the value limited to the largest bf16.
+__device__ __forceinline__ void split3_rn(float a, float b, uint32_t &h, uint32_t &m,
+                                          uint32_t &l) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  auto pack = [](float x, float y) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{x, y}), b2));
+  };
+  constexpr float kMax = 0x1.fep127f;
+  h = pack(__builtin_amdgcn_fmed3f(a, -kMax, kMax), __builtin_amdgcn_fmed3f(b, -kMax, kMax));
+  const float a1 = a - __uint_as_float(h << 16), b1 = b - __uint_as_float(h & 0xffff0000u);
+  m = pack(a1, b1);
+  l = pack(a1 - __uint_as_float(m << 16), b1 - __uint_as_float(m & 0xffff0000u));
 }
 
 }  // namespace q3h

@@ -7,8 +7,9 @@
 // the bf16 matrix cores with both operands split exactly (k_gemm_x3), K in 8
 // slices so that its workgroups fill the chip at the row counts of a prompt;
 // the slices added to b1, SiLU, split for fc2 (k_text_mid); fc2; the slices
-// added to b2 (k_text_end). The products are exact to the fp32 rounding of
-// their sums (the reference's idtF32 products). 48 rows: 48 us of kernels as
+// added to b2 (k_text_end). The products are as exact as fp32 ones (q3h_x3.h;
+// the reference's idtF32 products): a result of two one-term products 3.6e-8 off
+// float64 (RMS) as on the f32 matrix cores. 48 rows: 48 us of kernels as
 // three launches on the f32 matrix cores, whose 128 and 64 workgroups walked
 // all of K (23 + 20 us); widths that are no multiples of 64 and 512 still take
 // those: e = the rows, h = b1, y = b2, then fc1 with h = SiLU(h + sum)

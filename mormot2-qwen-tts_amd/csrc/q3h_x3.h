@@ -1,19 +1,27 @@
-// q3h_x3.h - f32 x f32 products on the bf16 matrix cores, exact to the fp32
-// rounding of the sums: the inner walk shared by the many-row products of f32
-// stacks and the decoder's convolutions.
+// q3h_x3.h - f32 x f32 products on the bf16 matrix cores: the operand tiles of
+// the many-row products (k_gemm_x3, which walks them itself) and the walks of
+// the decoder's convolutions (X3Walk, X3Short).
 //
-// Each operand is split into three bf16 parts, x = hi + mid + lo exactly
-// (split3), and the six part products whose weight is at least 2^-16 of the
-// product are accumulated in fp32 (hi hi, hi mid, mid hi, hi lo, lo hi, mid
-// mid; a bf16 product is exact in fp32; the dropped three weigh below 2^-23
-// of the product).
+// Each operand is split into three bf16 parts, x = hi + mid + lo exactly, hi
+// and mid rounded to nearest (split3_rn), and six part products are accumulated
+// in fp32: hi hi in a sum of its own, and hi mid, mid hi, hi lo, lo hi, mid mid
+// in another that is added to it at the end (of a slice). A bf16 product is
+// exact in fp32; the three products left out weigh at most 2^-24 of the whole
+// and cancel on average. The matrix cores cut off where they align a product
+// with its sum, so with one sum every hi hi product of a chunk lost up to an
+// fp32 unit downwards and met six roundings instead of one: a sample of seven
+// one-term products of the decoder 1.5e-7 off (RMS, mean -1.2e-7), 7.1e-8 (mean
+// 0) with two sums, 6.7e-8 on the f32 matrix cores; the decoder's samples 2.1e-6
+// off float64 -> 8.9e-7 (2.3e-6 on the f32 matrix cores).
 //
 // v_mfma_f32_16x16x32_bf16: lane l holds A[l % 16][8 (l / 16) .. + 7] and
 // B[8 (l / 16) .. + 7][l % 16] and receives D[4 (l / 16) + r][l % 16]. A is
 // 16 activation rows, B 16 weight rows. The weights come pre-split in operand
-// order (x3_tiles): [16-row tile][32-column chunk][part][lane][8], so an
-// operand is one coalesced 16-byte load per lane, straight to registers; the
-// activations are split as they go to LDS, shared by the workgroup's waves.
+// order (x3_offset): [16-row tile][32-column chunk][part][lane][8], so an
+// operand is one coalesced 16-byte load per lane, straight to registers. The
+// many-row products' activations come in the same tiles, written by the kernel
+// that makes them (x3_store4 / x3_store8); the decoder's are split as they go to
+// LDS, shared by the workgroup's waves.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -40,13 +48,13 @@ constexpr int kX3Part = 512;  // elements from a part of a tile to the next
 
 // 4 columns from k (a multiple of 4) of row m, split into the tiles at o
 __device__ __forceinline__ void x3_store4(uint16_t *o, int m, int k, int K, const float (&v)[4]) {
-  uint32_t h[4], md[4], l[4];
-#pragma unroll
-  for (int e = 0; e < 4; e++) split3(v[e], h[e], md[e], l[e]);
+  uint2 h, md, l;
+  split3_rn(v[0], v[1], h.x, md.x, l.x);
+  split3_rn(v[2], v[3], h.y, md.y, l.y);
   uint16_t *d = o + x3_offset(m, k, K);
-  *reinterpret_cast<uint2 *>(d) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-  *reinterpret_cast<uint2 *>(d + kX3Part) = make_uint2(md[0] | (md[1] << 16), md[2] | (md[3] << 16));
-  *reinterpret_cast<uint2 *>(d + 2 * kX3Part) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+  *reinterpret_cast<uint2 *>(d) = h;
+  *reinterpret_cast<uint2 *>(d + kX3Part) = md;
+  *reinterpret_cast<uint2 *>(d + 2 * kX3Part) = l;
 }
 
 // 8 columns from k (a multiple of 8)
@@ -54,12 +62,11 @@ __device__ __forceinline__ void x3_store8(uint16_t *o, int m, int k, int K, cons
   x3_u4 part[3];
 #pragma unroll
   for (int e = 0; e < 4; e++) {
-    uint32_t h0, m0, l0, h1, m1, l1;
-    split3(v[2 * e], h0, m0, l0);
-    split3(v[2 * e + 1], h1, m1, l1);
-    part[0][e] = h0 | (h1 << 16);
-    part[1][e] = m0 | (m1 << 16);
-    part[2][e] = l0 | (l1 << 16);
+    uint32_t h, md, l;
+    split3_rn(v[2 * e], v[2 * e + 1], h, md, l);
+    part[0][e] = h;
+    part[1][e] = md;
+    part[2][e] = l;
   }
   uint16_t *d = o + x3_offset(m, k, K);
 #pragma unroll
@@ -86,12 +93,12 @@ __device__ inline void x3_tile_lane(const float *f, int N, int K, size_t i, uint
   const int q = (int)(tq % nq), n = (int)(tq / nq) * 16 + (lane & 15);
   const float *s = f + (size_t)n * K + 32 * q + 8 * (lane >> 4);
   uint16_t *d = x3 + tq * 3 * 512 + lane * 8;
-  for (int e = 0; e < 8; e++) {
+  for (int e = 0; e < 8; e += 2) {
     uint32_t h, m, l;
-    split3(s[e], h, m, l);
-    d[e] = (uint16_t)h;
-    d[512 + e] = (uint16_t)m;
-    d[1024 + e] = (uint16_t)l;
+    split3_rn(s[e], s[e + 1], h, m, l);
+    *reinterpret_cast<uint32_t *>(d + e) = h;
+    *reinterpret_cast<uint32_t *>(d + 512 + e) = m;
+    *reinterpret_cast<uint32_t *>(d + 1024 + e) = l;
   }
 }
 
@@ -116,6 +123,8 @@ struct X3Walk {
   static constexpr int kPlane = kRows * kX3Stride;  // a part's plane in LDS
   static constexpr int kLds = 2 * 3 * kPlane;       // uint16_t
   static constexpr int kWords = WF32 ? 128 : 192;   // 16-byte words of a weight tile's chunk
+  // units of rows in flight (eight tiles: one, their sums take the registers)
+  static constexpr int kAhead = MT * NT >= 8 ? 1 : 2;
 
   // x: the tile's first row, channel 0 (row stride ld); rmax: its last row that
   // exists; t: the thread among the WN waves; u0 .. u1 - 1: the units; nu: the
@@ -133,8 +142,9 @@ struct X3Walk {
       const int f = t + kThreads * i;
       xo[i] = min(f >> 3, rmax) * ld + 4 * (f & 7);
     }
-    float4 xr[2][kXF4];
+    float4 xr[kAhead][kXF4];
     x3_u4 w[2][NT][WF32 ? 2 : 3];
+    x3_v4f low[NT][MT];  // the sums of the products with a lower part
     auto load_x = [&](int u, int s) {
       const float *p = x + 32 * min(u, u1 - 1);
 #pragma unroll
@@ -151,18 +161,14 @@ struct X3Walk {
 #pragma unroll
       for (int i = 0; i < kXF4; i++) {
         const int f = t + kThreads * i;
-        uint32_t h[4], m[4], l[4];
-        split3(xr[s][i].x, h[0], m[0], l[0]);
-        split3(xr[s][i].y, h[1], m[1], l[1]);
-        split3(xr[s][i].z, h[2], m[2], l[2]);
-        split3(xr[s][i].w, h[3], m[3], l[3]);
+        uint2 h, m, l;
+        split3_rn(xr[s][i].x, xr[s][i].y, h.x, m.x, l.x);
+        split3_rn(xr[s][i].z, xr[s][i].w, h.y, m.y, l.y);
         if (kRows * 8 % kThreads == 0 || f < kRows * 8) {
           uint16_t *d = xs + b * 3 * kPlane + (f >> 3) * kX3Stride + 4 * (f & 7);
-          *reinterpret_cast<uint2 *>(d) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-          *reinterpret_cast<uint2 *>(d + kPlane) =
-              make_uint2(m[0] | (m[1] << 16), m[2] | (m[3] << 16));
-          *reinterpret_cast<uint2 *>(d + 2 * kPlane) =
-              make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+          *reinterpret_cast<uint2 *>(d) = h;
+          *reinterpret_cast<uint2 *>(d + kPlane) = m;
+          *reinterpret_cast<uint2 *>(d + 2 * kPlane) = l;
         }
       }
     };
@@ -186,12 +192,12 @@ struct X3Walk {
             x3_u4 part[3];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-              uint32_t h0, m0, l0, h1, m1, l1;
-              split3(__uint_as_float(w[wb][j][e >> 1][2 * (e & 1)]), h0, m0, l0);
-              split3(__uint_as_float(w[wb][j][e >> 1][2 * (e & 1) + 1]), h1, m1, l1);
-              part[0][e] = h0 | (h1 << 16);
-              part[1][e] = m0 | (m1 << 16);
-              part[2][e] = l0 | (l1 << 16);
+              uint32_t h, m, l;
+              split3_rn(__uint_as_float(w[wb][j][e >> 1][2 * (e & 1)]),
+                        __uint_as_float(w[wb][j][e >> 1][2 * (e & 1) + 1]), h, m, l);
+              part[0][e] = h;
+              part[1][e] = m;
+              part[2][e] = l;
             }
 #pragma unroll
             for (int c = 0; c < kParts; c++) bw[j][c] = __builtin_bit_cast(x3_bf8, part[c]);
@@ -200,17 +206,18 @@ struct X3Walk {
             for (int c = 0; c < kParts; c++) bw[j][c] = __builtin_bit_cast(x3_bf8, w[wb][j][c]);
           }
         }
-        // the small part products first; a part of every tile before the next
-        // part (independent sums back to back)
+        // a part product of every tile before the next (independent sums back to
+        // back), the small ones first
         constexpr int pa[6] = {1, 2, 0, 1, 0, 0}, pb[6] = {1, 0, 2, 0, 1, 0};
 #pragma unroll
         for (int c = 0; c < 6; c++)
 #pragma unroll
           for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int j = 0; j < NT; j++)
-              acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][pa[c]], bw[j][pb[c]],
-                                                                  acc[j][i], 0, 0, 0);
+            for (int j = 0; j < NT; j++) {
+              x3_v4f &o = c < 5 ? low[j][i] : acc[j][i];
+              o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][pa[c]], bw[j][pb[c]], o, 0, 0, 0);
+            }
         load_w(u * TAPS + k + 2, wb);
       }
       if (SUM && (u + 1 - u0) % su == 0) {
@@ -218,36 +225,42 @@ struct X3Walk {
         for (int j = 0; j < NT; j++)
 #pragma unroll
           for (int i = 0; i < MT; i++) {
+            acc[j][i] = acc[j][i] + low[j][i];
             tot[j][i] = u + 1 - u0 == su ? acc[j][i] : tot[j][i] + acc[j][i];
-            acc[j][i] = x3_v4f{0.f, 0.f, 0.f, 0.f};
+            acc[j][i] = low[j][i] = x3_v4f{0.f, 0.f, 0.f, 0.f};
           }
       }
     };
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
-      for (int i = 0; i < MT; i++) acc[j][i] = x3_v4f{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < MT; i++) acc[j][i] = low[j][i] = x3_v4f{0.f, 0.f, 0.f, 0.f};
+    constexpr int kOdd = kAhead - 1;  // slot of the odd units
     load_x(u0, 0);
     load_w(u0 * TAPS, 0);
-    load_x(u0 + 1, 1);
+    if (kOdd) load_x(u0 + 1, kOdd);
     load_w(u0 * TAPS + 1, 1);
     stage(0, 0);
-    load_x(u0 + 2, 0);
+    load_x(u0 + kAhead, 0);
     __syncthreads();
     // unit u: its products from buffer u & 1, unit u + 1 staged in the other
     for (int i = 0; i < nu; i += 2) {
       const int u = u0 + i;
       if (u < u1) unit(u, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-      stage(1, 1);
-      load_x(u + 3, 1);
+      stage(1, kOdd);
+      load_x(u + 1 + kAhead, kOdd);
       __syncthreads();
       if (i + 1 >= nu) break;
       if (u + 1 < u1)
         unit(u + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, TAPS & 1>{});
       stage(0, 0);
-      load_x(u + 4, 0);
+      load_x(u + 2 + kAhead, 0);
       __syncthreads();
     }
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int i = 0; i < MT; i++) acc[j][i] = acc[j][i] + low[j][i];
     if (SUM) {
       const int n = u1 - u0, last = n % su;
 #pragma unroll
@@ -297,21 +310,18 @@ struct X3Short {
 #pragma unroll
     for (int i = 0; i < kXF4; i++) {
       const int f = t + kThreads * i, u = f / kUnitF4, e = f - u * kUnitF4;
-      uint32_t h[4], m[4], l[4];
-      split3(xr[i].x, h[0], m[0], l[0]);
-      split3(xr[i].y, h[1], m[1], l[1]);
-      split3(xr[i].z, h[2], m[2], l[2]);
-      split3(xr[i].w, h[3], m[3], l[3]);
+      uint2 h, m, l;
+      split3_rn(xr[i].x, xr[i].y, h.x, m.x, l.x);
+      split3_rn(xr[i].z, xr[i].w, h.y, m.y, l.y);
       if (SU * kUnitF4 % kThreads == 0 || f < SU * kUnitF4) {
         uint16_t *d = xs + u * 3 * kPlane + (e >> 3) * kX3Stride + 4 * (e & 7);
-        *reinterpret_cast<uint2 *>(d) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-        *reinterpret_cast<uint2 *>(d + kPlane) = make_uint2(m[0] | (m[1] << 16), m[2] | (m[3] << 16));
-        *reinterpret_cast<uint2 *>(d + 2 * kPlane) =
-            make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+        *reinterpret_cast<uint2 *>(d) = h;
+        *reinterpret_cast<uint2 *>(d + kPlane) = m;
+        *reinterpret_cast<uint2 *>(d + 2 * kPlane) = l;
       }
     }
     __syncthreads();
-    x3_v4f acc = x3_v4f{0.f, 0.f, 0.f, 0.f};
+    x3_v4f acc = x3_v4f{0.f, 0.f, 0.f, 0.f}, low = acc;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       constexpr int pa[6] = {1, 2, 0, 1, 0, 0}, pb[6] = {1, 0, 2, 0, 1, 0};
@@ -326,12 +336,12 @@ struct X3Short {
         x3_u4 part[3];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          uint32_t h0, m0, l0, h1, m1, l1;
-          split3(__uint_as_float(w[c % D][e >> 1][2 * (e & 1)]), h0, m0, l0);
-          split3(__uint_as_float(w[c % D][e >> 1][2 * (e & 1) + 1]), h1, m1, l1);
-          part[0][e] = h0 | (h1 << 16);
-          part[1][e] = m0 | (m1 << 16);
-          part[2][e] = l0 | (l1 << 16);
+          uint32_t h, m, l;
+          split3_rn(__uint_as_float(w[c % D][e >> 1][2 * (e & 1)]),
+                    __uint_as_float(w[c % D][e >> 1][2 * (e & 1) + 1]), h, m, l);
+          part[0][e] = h;
+          part[1][e] = m;
+          part[2][e] = l;
         }
 #pragma unroll
         for (int e = 0; e < 3; e++) bw[e] = __builtin_bit_cast(x3_bf8, part[e]);
@@ -340,13 +350,15 @@ struct X3Short {
         for (int e = 0; e < 3; e++) bw[e] = __builtin_bit_cast(x3_bf8, w[c % D][e]);
       }
       if (c + D < NC) load_w(c + D);
-      x3_v4f n = acc;
+      x3_v4f n = low;
 #pragma unroll
-      for (int e = 0; e < 6; e++)
+      for (int e = 0; e < 5; e++)
         n = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa[e]], bw[pb[e]], n, 0, 0, 0);
-      acc = u0 + u < u1 ? n : acc;
+      const x3_v4f hi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bw[0], acc, 0, 0, 0);
+      low = u0 + u < u1 ? n : low;
+      acc = u0 + u < u1 ? hi : acc;
     }
-    return acc;
+    return acc + low;
   }
 };
 

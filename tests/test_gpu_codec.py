@@ -7,6 +7,7 @@ giving the same samples, bit for bit."""
 import numpy as np
 import pytest
 
+import codec_torch
 import q3h
 import q3o
 import synth
@@ -68,6 +69,62 @@ def test_codec_kernel_choice_keeps_the_samples(device, weights, chunks, max_fram
 def test_codec_many_frames_in_one_pass(device, weights):
     x = synth.prompt(7, 64)
     assert np.array_equal(_gpu(device, weights, x, [64], 64), _gpu(device, weights, x, [64], 7))
+
+
+def _one_term_weights(rng):
+    """The decoder with one weight per output of every product of the main
+    branch, near 1, the residual units and ConvNeXt's branch zero and SnakeBeta's
+    term below the last bit (e^80): a sample is seven one-term products."""
+    w = synth.codec_weights(1)
+
+    def near_one(n):
+        return rng.uniform(0.97, 1.03, n).astype(np.float32)
+
+    def tconv(a, stride):  # [in][out][K]: one input channel per output and phase
+        o = np.zeros_like(a)
+        cin, out, _ = a.shape
+        for j in range(stride):
+            o[rng.integers(0, cin, out), np.arange(out), j] = near_one(out)
+        return o
+
+    for i in range(2):
+        w["up_w"][i] = tconv(w["up_w"][i], 2)
+        w["up_b"][i] = np.zeros_like(w["up_b"][i])
+        w["gamma"][i] = np.zeros_like(w["gamma"][i])
+    D, L, _ = w["conv0_w"].shape
+    w["conv0_w"] = np.zeros_like(w["conv0_w"])
+    w["conv0_w"][np.arange(D), rng.integers(0, L, D), 6] = near_one(D)
+    w["conv0_b"] = np.zeros_like(w["conv0_b"])
+    for b, rate in zip(w["block"], synth.CODEC_RATES):
+        b["up_w"], b["up_b"] = tconv(b["up_w"], rate), np.zeros_like(b["up_b"])
+        b["act_beta"] = np.full_like(b["act_beta"], 80)
+        for r in b["res"]:
+            for k in ("c1_w", "c1_b", "c2_w", "c2_b"):
+                r[k] = np.zeros_like(r[k])
+            for k in ("a1_beta", "a2_beta"):
+                r[k] = np.full_like(r[k], 80)
+    w["out_beta"] = np.full_like(w["out_beta"], 80)
+    w["out_w"], w["out_b"] = np.zeros_like(w["out_w"]), np.zeros_like(w["out_b"])
+    w["out_w"][0, 3, 6] = 1
+    return w
+
+
+@pytest.mark.parametrize("frames", [1, 16])
+def test_codec_one_term_products(device, frames):
+    """Seven products of one term each against float64, in the kernels of short
+    and of long calls: at most 2 x 2^-24 each (rounding; the part products left
+    out), 6.6e-8 together (RMS, seven roundings of 2.5e-8) with a mean of 0; 1e-7
+    and 5e-8 leave the dropped parts theirs (parts cut off instead of rounded:
+    4.3e-7, mean -4e-7)."""
+    rng = np.random.default_rng(3)
+    w = _one_term_weights(rng)
+    x = rng.uniform(0.3, 0.7, (frames, 1024)).astype(np.float32)
+    y = _gpu(device, w, x, [frames])
+    ref = codec_torch.back(w, x)
+    e = (y - ref) / ref
+    mean, rms, top = abs(e.mean()), np.sqrt((e ** 2).mean()), abs(e).max()
+    print(f"mean {mean:.2e} rms {rms:.2e} max {top:.2e}", flush=True)
+    assert top <= 14 * 2.0 ** -24 and rms < 1e-7 and mean < 5e-8, (mean, rms, top)
 
 
 def test_codec_reset_and_errors(device, weights):

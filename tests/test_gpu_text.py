@@ -67,6 +67,56 @@ def test_text_project_other_widths(device, hidden):
         p.destroy()
 
 
+@pytest.mark.parametrize("n", [5, 64])
+def test_text_project_one_term(device, n):
+    """One weight a row, so nothing averages the products' errors: y = w2 (w1 e)
+    (SiLU(v) = v for v >= 30), two products against float64. The part products
+    left out of one weigh at most 2^-24 of it, and its sum and the SiLU's
+    division are rounded to fp32: 5 x 2^-24 at most. Two roundings of a uniform
+    significand are 3.5e-8 (RMS) with a mean of 0; 6e-8 and a mean of 3e-8 leave
+    the dropped parts theirs (parts cut off instead of rounded: 9.2e-8, mean
+    6.8e-8)."""
+    TH, H = 2048, 1024
+    rng = np.random.default_rng(5)
+    emb = rng.uniform(5, 8, (n, TH)).astype(np.float32)
+    c1, c2 = rng.integers(0, TH, TH), rng.integers(0, TH, H)
+    w1, w2 = np.zeros((TH, TH), np.float32), np.zeros((H, TH), np.float32)
+    w1[np.arange(TH), c1] = rng.uniform(6, 8, TH)
+    w2[np.arange(H), c2] = rng.uniform(0.5, 2, H)
+    p = q3h.TextProj(device, emb, w1, np.zeros(TH, np.float32), w2, np.zeros(H, np.float32))
+    try:
+        y = p.project(np.arange(n))
+    finally:
+        p.destroy()
+    f = np.float64
+    h = emb.astype(f)[:, c1] * w1[np.arange(TH), c1].astype(f)
+    ref = h[:, c2] * w2[np.arange(H), c2].astype(f)
+    e = (y - ref) / ref
+    mean, rms, top = abs(e.mean()), np.sqrt((e ** 2).mean()), abs(e).max()
+    print(f"mean {mean:.2e} rms {rms:.2e} max {top:.2e}", flush=True)
+    assert top <= 5 * 2.0 ** -24 and rms < 6e-8 and mean < 3e-8, (mean, rms, top)
+
+
+def test_text_project_largest_values(device):
+    """Values within half a bf16 step of the largest float are split without
+    becoming infinite: against float64, 2e-5 as the other widths."""
+    rng = np.random.default_rng(6)
+    emb = rng.standard_normal((3, 1024)).astype(np.float32)
+    emb[:, 3] = (3.4e38, -3.3961e38, 3.4028235e38)
+    w1 = (rng.standard_normal((1024, 1024)) * 0.02).astype(np.float32)
+    w1[:, 3] *= np.float32(1e-30)
+    w2 = (rng.standard_normal((64, 1024)) * 0.02).astype(np.float32)
+    b1, b2 = np.zeros(1024, np.float32), np.zeros(64, np.float32)
+    p = q3h.TextProj(device, emb, w1, b1, w2, b2)
+    try:
+        y = p.project([0, 1, 2])
+    finally:
+        p.destroy()
+    v = emb.astype(np.float64) @ w1.T.astype(np.float64)
+    h = np.where(v < -80, 0.0, v / (1 + np.exp(-np.maximum(v, -80))))
+    assert rel(y, h @ w2.T.astype(np.float64)) < 2e-5
+
+
 def test_text_project_f32_table(device, tables):
     emb = (tables[0][:300].astype(np.uint32) << 16).view(np.float32)
     p = q3h.TextProj(device, emb, *tables[1:])
