@@ -46,31 +46,52 @@ __host__ __device__ inline size_t x3_offset(int m, int k, int K) {
 }
 constexpr int kX3Part = 512;  // elements from a part of a tile to the next
 
+// An infinity among the N values of v: its parts become (+-1, 0, +-inf). The
+// lowest part meets only the other operand's high part, whose sign is the
+// operand's and which is 0 for 0 alone, so the product is the infinity (or the
+// NaN) that the operands' product is; in the high part it would also meet the
+// other's lower parts, which are 0 or of the other sign for ordinary values.
+// h, m, l: the parts in pairs (split3_rn).
+template <int N>
+__device__ __forceinline__ void x3_infinite(const float (&v)[N], uint32_t (&h)[N / 2],
+                                            uint32_t (&m)[N / 2], uint32_t (&l)[N / 2]) {
+  float top = fabsf(v[0]);
+#pragma unroll
+  for (int e = 1; e < N; e++) top = fmaxf(top, fabsf(v[e]));
+  if (__builtin_expect(top != __builtin_inff(), 1)) return;
+#pragma unroll
+  for (int e = 0; e < N; e++) {
+    if (fabsf(v[e]) != __builtin_inff()) continue;
+    const int sh = 16 * (e & 1);
+    const uint32_t keep = ~(0xffffu << sh), sign = (__float_as_uint(v[e]) >> 31) << 15;
+    h[e / 2] = (h[e / 2] & keep) | ((0x3f80u | sign) << sh);
+    m[e / 2] &= keep;
+    l[e / 2] = (l[e / 2] & keep) | ((0x7f80u | sign) << sh);
+  }
+}
+
 // 4 columns from k (a multiple of 4) of row m, split into the tiles at o
 __device__ __forceinline__ void x3_store4(uint16_t *o, int m, int k, int K, const float (&v)[4]) {
-  uint2 h, md, l;
-  split3_rn(v[0], v[1], h.x, md.x, l.x);
-  split3_rn(v[2], v[3], h.y, md.y, l.y);
+  uint32_t h[2], md[2], l[2];
+#pragma unroll
+  for (int e = 0; e < 2; e++) split3_rn(v[2 * e], v[2 * e + 1], h[e], md[e], l[e]);
+  x3_infinite(v, h, md, l);
   uint16_t *d = o + x3_offset(m, k, K);
-  *reinterpret_cast<uint2 *>(d) = h;
-  *reinterpret_cast<uint2 *>(d + kX3Part) = md;
-  *reinterpret_cast<uint2 *>(d + 2 * kX3Part) = l;
+  *reinterpret_cast<uint2 *>(d) = make_uint2(h[0], h[1]);
+  *reinterpret_cast<uint2 *>(d + kX3Part) = make_uint2(md[0], md[1]);
+  *reinterpret_cast<uint2 *>(d + 2 * kX3Part) = make_uint2(l[0], l[1]);
 }
 
 // 8 columns from k (a multiple of 8)
 __device__ __forceinline__ void x3_store8(uint16_t *o, int m, int k, int K, const float (&v)[8]) {
-  x3_u4 part[3];
+  uint32_t h[4], md[4], l[4];
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    uint32_t h, md, l;
-    split3_rn(v[2 * e], v[2 * e + 1], h, md, l);
-    part[0][e] = h;
-    part[1][e] = md;
-    part[2][e] = l;
-  }
-  uint16_t *d = o + x3_offset(m, k, K);
-#pragma unroll
-  for (int c = 0; c < 3; c++) *reinterpret_cast<x3_u4 *>(d + c * kX3Part) = part[c];
+  for (int e = 0; e < 4; e++) split3_rn(v[2 * e], v[2 * e + 1], h[e], md[e], l[e]);
+  x3_infinite(v, h, md, l);
+  x3_u4 *d = reinterpret_cast<x3_u4 *>(o + x3_offset(m, k, K));
+  d[0] = x3_u4{h[0], h[1], h[2], h[3]};
+  d[kX3Part / 8] = x3_u4{md[0], md[1], md[2], md[3]};
+  d[2 * kX3Part / 8] = x3_u4{l[0], l[1], l[2], l[3]};
 }
 
 // weights f [N][K] row-major into the operand tiles x3 (3 N K bf16; N % 16 ==
@@ -91,15 +112,10 @@ __device__ inline void x3_tile_lane(const float *f, int N, int K, size_t i, uint
   const int lane = i & 63, nq = K >> 5;
   const size_t tq = i >> 6;  // tile * nq + chunk
   const int q = (int)(tq % nq), n = (int)(tq / nq) * 16 + (lane & 15);
-  const float *s = f + (size_t)n * K + 32 * q + 8 * (lane >> 4);
-  uint16_t *d = x3 + tq * 3 * 512 + lane * 8;
-  for (int e = 0; e < 8; e += 2) {
-    uint32_t h, m, l;
-    split3_rn(s[e], s[e + 1], h, m, l);
-    *reinterpret_cast<uint32_t *>(d + e) = h;
-    *reinterpret_cast<uint32_t *>(d + 512 + e) = m;
-    *reinterpret_cast<uint32_t *>(d + 1024 + e) = l;
-  }
+  const int k = 32 * q + 8 * (lane >> 4);
+  const float *s = f + (size_t)n * K + k;
+  const float v[8] = {s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]};
+  x3_store8(x3, n, k, K, v);
 }
 
 // The walk of WN waves over a product's columns: wave w owns NT 16-row weight

@@ -117,6 +117,44 @@ def test_text_project_largest_values(device):
     assert rel(y, h @ w2.T.astype(np.float64)) < 2e-5
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+def test_text_project_infinite_values(device, bf16):
+    """Infinities and NaN in the embedding and the weights give those of the fp32
+    formula (-inf ends in the SiLU's 0): rows 1 to 3 hold one of them each, then
+    infinite weights of fc1 meet 0 (NaN) and 1, and fc2 has one.
+    The finite results within 2e-5."""
+    rng = np.random.default_rng(9)
+    emb = rng.standard_normal((5, 1024)).astype(np.float32)
+    emb[:, 8] = 0
+    emb[1, 5], emb[2, 5], emb[3, 9], emb[4, 8] = np.inf, -np.inf, np.nan, 1
+    w1 = (rng.standard_normal((1024, 1024)) * 0.02).astype(np.float32)
+    w1[:, 5] = abs(w1[:, 5])
+    w2 = abs(rng.standard_normal((64, 1024)) * 0.02).astype(np.float32)
+    b1, b2 = np.zeros(1024, np.float32), rng.standard_normal(64).astype(np.float32)
+    bits = (emb.view(np.uint32) >> 16).astype(np.uint16)
+    if bf16:
+        emb = (bits.astype(np.uint32) << 16).view(np.float32)
+    for inf1, inf2 in (((), ()), ((7, 11), ()), ((), (3,))):
+        a, b = w1.copy(), w2.copy()
+        a[inf1, 8] = np.inf
+        b[inf2, 2] = -np.inf
+        p = q3h.TextProj(device, bits if bf16 else emb, a, b1, b, b2)
+        try:
+            y = p.project(np.arange(5))
+        finally:
+            p.destroy()
+        with np.errstate(all="ignore"):
+            v = emb.astype(np.float64) @ a.T.astype(np.float64)
+            h = np.where(v < -80, 0.0, v / (1 + np.exp(-v)))
+            ref = h @ b.T.astype(np.float64) + b2
+        assert np.array_equal(np.isnan(y), np.isnan(ref)), (inf1, inf2)
+        inf = np.isinf(ref)
+        assert np.array_equal(y[inf], ref[inf].astype(np.float32)), (inf1, inf2)
+        fin = np.isfinite(ref)
+        assert inf1 or (fin[0].any() and fin[2].any())
+        assert not fin.any() or rel(y[fin], ref[fin]) < 2e-5
+
+
 def test_text_project_f32_table(device, tables):
     emb = (tables[0][:300].astype(np.uint32) << 16).view(np.float32)
     p = q3h.TextProj(device, emb, *tables[1:])
