@@ -42,22 +42,26 @@ __device__ __forceinline__ float silu_clamp_f(float v) {
 }
 
 // sinf, kept out of line
-__device__ __attribute__((noinline)) inline float sin_far(float x) { return sinf(x); }
+__host__ __device__ __attribute__((noinline)) inline float sin_far(float x) { return sinf(x); }
 
 // sin(x)^2, the SnakeBeta term: of period pi and even, so x is reduced by the
-// nearest multiple of pi (pi as the sum of two floats, both products fused: the
-// reduction is exact to the last bit of r while k < 2^17) and the sign of the
-// result does not matter; sin r, |r| <= pi / 2, by its Taylor series to r^13
-// (truncation < 7e-10) in Horner form. Within 2 units of 2^-24 of sin x,
-// relative; beyond 4e5 by sinf. 16 instructions without a branch taken, where
-// sinf's general reduction, inlined per output, made a decoder epilogue of 32
-// values 9000 lines long.
-__device__ __forceinline__ float sin_squared(float x) {
+// nearest multiple of pi and the sign of the result does not matter. pi is the
+// sum of three floats: the first product is exact below 4e5 (k < 2^17; x and k
+// p1 are multiples of 2^-23 and their difference is below 2), the second is
+// rounded once in the result's own last place, and the third's (k 3.4e-15, which
+// two floats left out) keeps that so where x is next to a multiple of pi. sin r,
+// |r| <= pi / 2, by its Taylor series to r^13 (truncation < 7e-10) in Horner
+// form. sin x within 3 units of 2^-24, relative (two roundings of r, one of the
+// last step); beyond 4e5 by sinf. 17
+// instructions without a branch taken, where sinf's general reduction, inlined
+// per output, made a decoder epilogue of 32 values 9000 lines long.
+__host__ __device__ __forceinline__ float sin_squared(float x) {
   float s;
   if (fabsf(x) < 4e5f) {
     const float k = rintf(x * 0x1.45f306p-2f);
     float r = fmaf(-k, 0x1.921fb6p+1f, x);
     r = fmaf(k, 0x1.777a5cp-24f, r);
+    r = fmaf(k, 0x1.ee59dap-49f, r);
     const float r2 = r * r;
     float p = 0x1.612462p-33f;       // 1/13!
     p = fmaf(p, r2, -0x1.ae6456p-26f);  // -1/11!
