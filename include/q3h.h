@@ -147,10 +147,10 @@ int q3h_context_time_attention(q3h_context *c, int iters, float *us_per_launch,
    are in host memory. rows <= 0 does nothing (lm.pas:394-395). One row
    replays a HIP graph the context captures per (head, position cover)
    (covers of 64 positions up to 256, of 256 beyond; at most 32 graphs per
-   context, dropped when its work buffers grow) and copies its row, logits
-   and state through a pinned host buffer of the context (several rows: the
-   logits and state); the results are those of the same launches made
-   directly (q3h_forward_embeds_noalloc). ---- */
+   context, the one unused longest gives way, all dropped when its work buffers
+   grow) and copies its row, logits and state through a pinned host buffer of
+   the context (several rows: the logits and state); the results are those of
+   the same launches made directly (q3h_forward_embeds_noalloc). ---- */
 int q3h_forward_embeds(q3h_context *c, const float *x, int rows, int head,
                        float *logits, float *normed_last);
 
@@ -193,9 +193,10 @@ int q3h_forward_embeds_probe(q3h_context *c, const float *x, int rows, int head,
    context, n contexts of the same stack at their own positions;
    x [n][hidden]; heads [n] (or NULL: no logits); logits [n][head rows of
    heads[0]] (all heads of one call must have the same rows); normed [n][hidden]
-   (nullable). Up to 256 contexts of one max_positions with one head: replayed
-   from a HIP graph that ctxs[0] captures per (n, head, position cover of the
-   longest context), the contexts read on the device, so any contexts of the
+   (nullable). Up to 256 contexts of one max_positions with one head: from the
+   second use of a (n, head, position cover of the longest context) on replayed
+   from a HIP graph that ctxs[0] captures then (at most 64, the one unused
+   longest gives way), the contexts read on the device, so any contexts of the
    same n may follow. */
 int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const float *x,
                              const int *heads, float *logits, float *normed);

@@ -946,8 +946,8 @@ q3h_context *new_context(q3h_stack *s, int max_positions) {
 }
 
 void drop_graphs(q3h_context *ctx) {
-  for (auto &g : ctx->graphs) (void)hipGraphExecDestroy(g.second);
   ctx->graphs.clear();
+  ctx->batch_graphs.clear();
 }
 
 void free_context(q3h_context *ctx) {
@@ -1191,33 +1191,43 @@ void enqueue_forward(q3h_context *c, Work &w, int rows, int positions, int head,
   launch_advance(c->dev_arr, nullptr, 1, rows, st);
 }
 
-// the graph of key among c's captured forwards on its Work buffers, captured
-// from enqueue() at its first use
-template <class F>
-hipGraphExec_t context_graph(q3h_context *c, uint64_t key, F &&enqueue) {
-  constexpr size_t kMaxGraphs = 32;  // per context: a code predictor's heads, a talker's covers
-  if (c->graphs_gen != c->w.gen || c->graphs.size() >= kMaxGraphs) {
-    drop_graphs(c);
-    c->graphs_gen = c->w.gen;
-  }
-  for (auto &g : c->graphs)
-    if (g.first == key) return g.second;
-  hipGraph_t graph = capture_graph(c->stream, enqueue);
-  hipGraphExec_t exec = nullptr;
-  const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-  (void)hipGraphDestroy(graph);
-  check_hip(e, "forward graph instantiate");
-  c->graphs.push_back({key, exec});
-  return exec;
+// c's graphs were captured on its Work buffers: none is left of buffers that
+// have been replaced
+void current_graphs(q3h_context *c) {
+  if (c->graphs_gen == c->w.gen) return;
+  drop_graphs(c);
+  c->graphs_gen = c->w.gen;
 }
 
-// the captured single-row forward of (head, cover) on c's Work buffers
+// the captured single-row forward of (head, cover) on c's Work buffers, captured
+// at its first use
 hipGraphExec_t forward_graph(q3h_context *c, int head, int positions) {
-  return context_graph(c, ((uint64_t)(uint32_t)(head + 1) << 32) | (uint32_t)positions, [&] {
+  current_graphs(c);
+  const uint64_t key = ((uint64_t)(uint32_t)(head + 1) << 32) | (uint32_t)positions;
+  if (hipGraphExec_t exec = c->graphs.find(key)) return exec;
+  return c->graphs.add(key, c->stream, [&] {
     LayerIO io;
     io.single_context = true;
     enqueue_forward(c, c->w, 1, positions, head, io, c->stream);
   });
+}
+
+// The captured batched forward of n rows that c leads, captured from enqueue()
+// at its second use among the last 64 keys, else null: a batch whose size or
+// position cover is met once (contexts that end, a server whose batch moves) is
+// not slower than its launches, and keys that come round more slowly than the
+// cache holds them are never captured only to be thrown away. 15 heads at 4, 8
+// and 16 contexts in turn (5 int8 layers): 187 / 209 / 219 us a call, 243 / 263 /
+// 330 at their first use as launches, 110 more at the second; 320 / 325 / 345 at
+// every use with 32 graphs in all, captured at first use and dropped together.
+template <class F>
+hipGraphExec_t batch_graph(q3h_context *c, int n, int head, int positions, F &&enqueue) {
+  current_graphs(c);
+  const uint64_t key =
+      ((uint64_t)n << 52) | ((uint64_t)(uint32_t)(head + 1) << 32) | (uint32_t)positions;
+  if (hipGraphExec_t exec = c->batch_graphs.find(key)) return exec;
+  if (!c->batch_graphs.seen(key)) return nullptr;
+  return c->batch_graphs.add(key, c->stream, enqueue);
 }
 
 // c's pinned host staging of at least `floats` floats (c's stream idle)
@@ -1365,7 +1375,7 @@ extern "C" int q3h_forward_embeds_noalloc(q3h_context *c, const float *x, int ro
 }
 
 // rows of a replayed batched forward (more run as direct launches; the key of
-// their graphs holds up to 2047 rows and 2^20 heads)
+// their graphs holds up to 4095 rows and 2^20 heads)
 constexpr int kBatchGraphRows = 256;
 
 extern "C" int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const float *x,
@@ -1399,16 +1409,17 @@ extern "C" int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const f
     check_hip(hipSetDevice(s->dev->ordinal), "hipSetDevice");
     for (int i = 1; i < n; i++) check_hip(hipStreamSynchronize(ctxs[i]->stream), "batch sync");
     const int H = cf.hidden;
-    // contexts of one size and one head: the launches replayed from a graph
-    // captured per (rows, head, cover), as the single-row forward's are (the
-    // contexts themselves are read from w.ctx_arr on the device)
-    bool same = true, replay = n <= kBatchGraphRows;
+    // contexts of one size and one head: the launches of the position cover,
+    // replayed from a graph of (rows, head, cover) once it comes again, as the
+    // single-row forward's are (the contexts themselves are read from w.ctx_arr
+    // on the device)
+    bool same = true, cover = n <= kBatchGraphRows;
     for (int i = 1; i < n; i++) {
       same = same && (!heads || heads[i] == heads[0]);
-      replay = replay && ctxs[i]->max_pos == c0->max_pos;
+      cover = cover && ctxs[i]->max_pos == c0->max_pos;
     }
-    replay = replay && same;
-    const int positions = replay ? graph_cover(maxlen, c0->max_pos) : maxlen;
+    cover = cover && same;
+    const int positions = cover ? graph_cover(maxlen, c0->max_pos) : maxlen;
     Work &w = c0->w;
     w.ensure(s, n, attention_splits(s, positions), head_rows);
     hipStream_t st = c0->stream;
@@ -1430,7 +1441,9 @@ extern "C" int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const f
     for (int i = 0; i < n; i++) arr[i] = ctxs[i]->dev;
     const CtxDev *const *src = arr.data();
     float *lg = logits, *nm = normed;
-    if (replay) {  // through pinned host memory: [contexts | x | normed | logits]
+    const hipGraphExec_t exec =
+        cover ? batch_graph(c0, n, heads ? heads[0] : -1, positions, enqueue) : nullptr;
+    if (exec) {  // through pinned host memory: [contexts | x | normed | logits]
       check_hip(hipStreamSynchronize(st), "batch sync");
       float *pin = context_pin(c0, 2 * (size_t)n + 2 * nx + nl);
       std::memcpy(pin, arr.data(), sizeof(CtxDev *) * n);
@@ -1443,14 +1456,10 @@ extern "C" int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const f
     check_hip(hipMemcpyAsync(w.ctx_arr, src, sizeof(CtxDev *) * n, hipMemcpyHostToDevice, st),
               "upload contexts");
     check_hip(hipMemcpyAsync(w.h, x, sizeof(float) * nx, hipMemcpyHostToDevice, st), "upload x");
-    if (replay) {
-      const int head = heads ? heads[0] : -1;
-      const uint64_t key = (1ull << 63) | ((uint64_t)n << 52) |
-                           ((uint64_t)(uint32_t)(head + 1) << 32) | (uint32_t)positions;
-      check_hip(hipGraphLaunch(context_graph(c0, key, enqueue), st), "batch graph launch");
-    } else {
+    if (exec)
+      check_hip(hipGraphLaunch(exec, st), "batch graph launch");
+    else
       enqueue();
-    }
     check_hip(hipGetLastError(), "batch kernels");
     if (normed)
       check_hip(hipMemcpyAsync(nm, w.normed, sizeof(float) * nx, hipMemcpyDeviceToHost, st),
@@ -1459,8 +1468,8 @@ extern "C" int q3h_forward_embeds_batch(q3h_context *const *ctxs, int n, const f
       check_hip(hipMemcpyAsync(lg, w.logits, sizeof(float) * nl, hipMemcpyDeviceToHost, st),
                 "download logits");
     check_hip(hipStreamSynchronize(st), "batch sync");
-    if (replay && normed) std::memcpy(normed, nm, sizeof(float) * nx);
-    if (replay && logits && heads) std::memcpy(logits, lg, sizeof(float) * nl);
+    if (exec && normed) std::memcpy(normed, nm, sizeof(float) * nx);
+    if (exec && logits && heads) std::memcpy(logits, lg, sizeof(float) * nl);
     for (int i = 0; i < n; i++) ctxs[i]->len += 1;
   });
 }

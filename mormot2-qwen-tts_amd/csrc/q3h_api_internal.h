@@ -3,9 +3,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "q3h.h"
@@ -86,6 +88,61 @@ hipGraph_t capture_graph(hipStream_t st, F &&enqueue) {
   check_hip(hipStreamEndCapture(st, &g), "hipStreamEndCapture");
   return g;
 }
+
+// Captured graphs by key, at most `limit` of them, the one used last at the
+// back: a new one takes the place of the one unused longest. What replays them
+// is idle whenever one is taken out (every call ends with its stream idle).
+struct GraphCache {
+  explicit GraphCache(size_t limit) : limit(limit) {}
+  ~GraphCache() { clear(); }
+  GraphCache(const GraphCache &) = delete;
+  GraphCache &operator=(const GraphCache &) = delete;
+  // the graph of key, null when it has none
+  hipGraphExec_t find(uint64_t key) {
+    for (size_t i = graphs.size(); i-- > 0;)
+      if (graphs[i].first == key) {
+        std::rotate(graphs.begin() + i, graphs.begin() + i + 1, graphs.end());
+        return graphs.back().second;
+      }
+    return nullptr;
+  }
+  // whether key was asked for before among the last `limit` other keys that have
+  // no graph; remembers it
+  bool seen(uint64_t key) {
+    const auto it = std::find(once.begin(), once.end(), key);
+    if (it != once.end()) {
+      once.erase(it);
+      return true;
+    }
+    if (once.size() >= limit) once.erase(once.begin());
+    once.push_back(key);
+    return false;
+  }
+  // the graph of key, which has none, captured from enqueue() on st
+  template <class F>
+  hipGraphExec_t add(uint64_t key, hipStream_t st, F &&enqueue) {
+    hipGraph_t graph = capture_graph(st, enqueue);
+    hipGraphExec_t exec = nullptr;
+    const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    check_hip(e, "forward graph instantiate");
+    if (graphs.size() >= limit) {
+      (void)hipGraphExecDestroy(graphs.front().second);
+      graphs.erase(graphs.begin());
+    }
+    graphs.push_back({key, exec});
+    return exec;
+  }
+  void clear() {
+    for (auto &g : graphs) (void)hipGraphExecDestroy(g.second);
+    graphs.clear();
+  }
+
+ private:
+  const size_t limit;
+  std::vector<std::pair<uint64_t, hipGraphExec_t>> graphs;
+  std::vector<uint64_t> once;
+};
 
 struct Layer {
   Mat qkv;   // [q; k; v] rows
@@ -216,9 +273,11 @@ struct q3h_context {
   float *probe = nullptr;  // the layer outputs of q3h_forward_embeds_probe
   size_t probe_bytes = 0;
   // the captured single-row forwards, keyed by (head + 1) << 32 | cover, and
-  // the batched forwards this context leads (bit 63 and the rows besides),
-  // valid for the Work buffers of generation graphs_gen
-  std::vector<std::pair<uint64_t, hipGraphExec_t>> graphs;
+  // the batched forwards this context leads (the rows besides: << 52), valid for
+  // the Work buffers of generation graphs_gen
+  // (32: a code predictor's heads, a talker's covers; 64: its heads at four
+  // batch sizes, or covers at as many sizes as a server's batch moves through)
+  q3h::GraphCache graphs{32}, batch_graphs{64};
   unsigned graphs_gen = 0;
   // pinned host staging of a forward: the input row, the normed state, the
   // logits (a batched one: contexts, rows, states, logits); hipHostMalloc'ed on

@@ -7,6 +7,7 @@ bar, tests/test.tts.qwen.vulkan.pas:226-231); Q8_0 logits 1e-3 with identical
 greedy codes.
 """
 import os
+import time
 
 import numpy as np
 import pytest
@@ -175,6 +176,58 @@ def test_batch_replays_follow_the_contexts(q8model, q3h, synth):
     finally:
         for c in a + b + [odd, odd_b]:
             c.destroy()
+
+
+def test_batch_graph_keys(device, q3h, q3o, synth):
+    """Batched forwards of 15 heads at 3 sizes in turn (45 graphs of the leading
+    context, a code predictor's use): the first use of a key is launched, the
+    second captured, all later ones replayed, none captured twice, so a third
+    round costs what one key repeated does (1.5 times allowed; a capture costs
+    several calls). Then 90 keys used twice each, more than are kept, between
+    single-row forwards of the leading context: the same results bit for bit as
+    at their first use."""
+    dims = dict(synth.TALKER, layers=2)
+    layers, final = synth.stack_weights(53, "s.", dims, norm_std=0.1, quantize=q3o.quantize_q8_0)
+    st = q3h.Stack(device, dict(dims, dtype=q3h.Q8_0, kv_f16=0, act_q8=0, max_positions=32),
+                   layers, final, q3h.Q8_0)
+    for g in range(15):
+        st.add_head(q3o.quantize_q8_0(synth.cp_head(53, g)), q3h.Q8_0)
+    ctxs = [q3h.Context(st, 32) for _ in range(12)]
+    x = synth.prompt(160, 12)
+
+    def call(n, head):
+        for c in ctxs[:n]:
+            c.reset()
+        t = time.perf_counter()
+        lg, normed = q3h.forward_batch(ctxs[:n], x[:n], heads=[head] * n)
+        return time.perf_counter() - t, lg, normed
+
+    try:
+        call(12, 0)  # the work buffers of all sizes
+        keys = [(n, g) for n in (6, 9, 12) for g in range(15)]
+        first = {k: call(*k)[1:] for k in keys}
+        for _ in range(2):
+            rounds = [call(*k) for k in keys]
+        for k, r in zip(keys, rounds):
+            assert np.array_equal(r[1], first[k][0]) and np.array_equal(r[2], first[k][1]), k
+        turn = np.median([r[0] for r in rounds])
+        one = np.median([call(n, 3)[0] for n in (6, 9, 12) for _ in range(15)])
+        print(f"45 keys in turn {turn * 1e6:.0f} us a call, one key {one * 1e6:.0f} us")
+        assert turn < 1.5 * one
+        ctxs[0].reset()
+        single = ctxs[0].forward(x[0], head=0)[0]
+        for n in (2, 3, 4, 5, 7, 8):
+            for g in range(15):
+                a, b = call(n, g), call(n, g)
+                assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2]), (n, g)
+            ctxs[0].reset()
+            assert np.array_equal(ctxs[0].forward(x[0], head=0)[0], single), n
+        for k in keys:
+            assert np.array_equal(call(*k)[1], first[k][0]), k
+    finally:
+        for c in ctxs:
+            c.destroy()
+        st.destroy()
 
 
 def test_graph_forward_equals_direct(q8model, q3h, synth):
