@@ -49,8 +49,14 @@ void work_fields(const q3h_stack *s, size_t R, int splits, int head_rows, Work &
   const size_t NKV = (size_t)c.kv_heads * c.head_dim, I = c.intermediate;
   each((void **)&w.h, sizeof(float) * R * H);
   each((void **)&w.qkv, sizeof(float) * R * (NQ + 2 * NKV));
-  each((void **)&w.att, sizeof(float) * R * NQ);
-  each((void **)&w.act, sizeof(float) * R * I);
+  // over more than kManyRows rows of f32 activations, also the operand tiles: the
+  // normed rows in att, the attention and SwiGLU outputs in act (run_layers_x3)
+  const bool tiles = !c.act_q8 && R > (size_t)kManyRows;
+  each((void **)&w.att, std::max(sizeof(float) * R * NQ, tiles ? x3_bytes(R, H) : 0));
+  each((void **)&w.act,
+       std::max(sizeof(float) * R * I, tiles ? x3_bytes(R, std::max(NQ, I)) : 0));
+  w.x3n = tiles ? reinterpret_cast<uint16_t *>(w.att) : nullptr;
+  w.x3a = tiles ? reinterpret_cast<uint16_t *>(w.act) : nullptr;
   each((void **)&w.normed, sizeof(float) * R * H);
   each((void **)&w.logits, sizeof(float) * R * (head_rows > 0 ? head_rows : 1));
   each((void **)&w.rd, sizeof(RowDesc) * R);
@@ -78,20 +84,20 @@ void work_fields(const q3h_stack *s, size_t R, int splits, int head_rows, Work &
     pn = std::max(pn, sr * (H / 256) * ldq);
     pn = std::max(pn, sr * std::min<size_t>(kMaxPartSlices, std::max(NQ, I) / 256) * H);
     each((void **)&w.gpart, sizeof(float) * pn);
-    const bool many = R > (size_t)kManyRows;
-    each((void **)&w.x3n, many ? x3_bytes(R, H) : 0);
-    each((void **)&w.x3a, many ? x3_bytes(R, std::max(NQ, I)) : 0);
   }
 }
 
 void Work::ensure(const q3h_stack *s, int rows, int splits, int head_rows) {
   if (rows <= rows_cap && splits <= splits_cap && head_rows <= head_cap) return;
+  rows = std::max(rows, rows_cap);
+  splits = std::max(splits, splits_cap);
+  head_rows = std::max(head_rows, head_cap);
   release();
-  rows_cap = rows > rows_cap ? rows : rows_cap;
-  splits_cap = splits > splits_cap ? splits : splits_cap;
-  head_cap = head_rows > head_cap ? head_rows : head_cap;
-  work_fields(s, rows_cap, splits_cap, head_cap, *this,
+  work_fields(s, rows, splits, head_rows, *this,
               [](void **slot, size_t bytes) { *slot = dev_alloc(bytes); });
+  rows_cap = rows;  // (only now: after a failed allocation the next call starts anew)
+  splits_cap = splits;
+  head_cap = head_rows;
   gen++;
 }
 
@@ -124,8 +130,6 @@ void Work::release() {
   dev_free(xa.q);
   dev_free(xb.q);
   dev_free(gpart);
-  dev_free(x3n);
-  dev_free(x3a);
   x3n = x3a = nullptr;
   xa = QAct{};
   xb = QAct{};
@@ -133,6 +137,7 @@ void Work::release() {
   h = qkv = att = act = normed = logits = part = nullptr;
   rd = nullptr;
   ctx_arr = nullptr;
+  rows_cap = splits_cap = head_cap = 0;
 }
 
 int attention_splits(const q3h_stack *s, int positions) {
@@ -1243,6 +1248,11 @@ float *context_pin(q3h_context *c, size_t floats) {
   return c->pin;
 }
 
+// the pinned floats of a forward: input row, state, logits
+size_t pin_need(const q3h_stack *s, int head) {
+  return (size_t)2 * s->cfg.hidden + (head >= 0 ? s->heads[head].N : 0);
+}
+
 // TQwenLm.Forward on the work buffers w (sized for rows, the attention splits
 // of forward_positions and the head's rows), replayed from a captured graph
 // when graph: blocks until the outputs are in host memory
@@ -1261,7 +1271,7 @@ void forward_rows(q3h_context *c, Work &w, const float *x, int rows, int head, f
   float *pin_lg = nullptr, *pin_n = nullptr;
   pinned = pinned || graph;
   if (pinned) {
-    float *pin = context_pin(c, (size_t)2 * H + head_rows);
+    float *pin = context_pin(c, pin_need(s, head));
     pin_n = pin + H;
     pin_lg = pin + 2 * H;
     if (rows == 1) {
@@ -1331,8 +1341,12 @@ extern "C" int q3h_forward_embeds(q3h_context *c, const float *x, int rows, int 
     check_hip(hipSetDevice(s->dev->ordinal), "hipSetDevice");
     const int head_rows = head >= 0 ? s->heads[head].N : 0;
     c->w.ensure(s, rows, forward_splits(c, rows), head_rows);
-    // one row (a decode step): the forward replayed from a captured graph
-    forward_rows(c, c->w, x, rows, head, logits, normed_last, nullptr, rows == 1, nullptr, true);
+    // one row (a decode step): the forward replayed from a captured graph; a
+    // prompt's results through pinned memory where the context has it, or from
+    // its second prompt on (the first does not pay for the allocation)
+    const bool pinned = c->pin_floats >= pin_need(s, head) || c->prompted;
+    c->prompted = c->prompted || rows > 1;
+    forward_rows(c, c->w, x, rows, head, logits, normed_last, nullptr, rows == 1, nullptr, pinned);
   });
 }
 

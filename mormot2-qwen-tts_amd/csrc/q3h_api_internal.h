@@ -170,7 +170,8 @@ struct Work {
   QAct xa, xb;              // quantized activations (act_q8 stacks)
   float *gpart = nullptr;   // chunk partials of the int8 products (act_q8)
   // operand tiles of the products over more than kManyRows rows (f32
-  // activations): the normed rows, and the attention / SwiGLU outputs
+  // activations): the normed rows, and the attention / SwiGLU outputs; the
+  // memory of att and act, which that path needs at other times only
   uint16_t *x3n = nullptr, *x3a = nullptr;
   void ensure(const struct ::q3h_stack *s, int rows, int splits, int head_rows);
   void release();
@@ -284,6 +285,7 @@ struct q3h_context {
   // first use, pin_floats floats, at most those of kBatchGraphRows rows
   float *pin = nullptr;
   size_t pin_floats = 0;
+  bool prompted = false;  // a forward of several rows has run
 };
 
 // the text projection (q3h_text.hip)
