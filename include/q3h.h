@@ -232,7 +232,8 @@ int q3h_frame_start(q3h_frame *f, int stream, const float *prefill, int rows,
 /* no reference counterpart (batched serving; the reference starts one
    sentence at a time): q3h_frame_start for n distinct streams at once. The
    prompts of an int8 stack, and those over 64 rows of the others, run as the
-   rows of one pass (of at most 8192 rows; further passes follow); the rest
+   rows of one pass (of at most 8192 rows, each taking the prompts left that
+   still fit; its work buffers, at most 0.54 GB, stay with the frame); the rest
    each on its stream's own talker context and HIP stream, so that they overlap
    on the device; blocks until all are done. streams [n];
    prefill[i] [rows[i]][hidden]; trailing (nullable) and trailing_rows

@@ -20,6 +20,7 @@
 
 #include "q3h.h"
 #include "q3h_api_internal.h"
+#include "q3h_passes.h"
 #include "q3h_quant.h"
 #include "q3h_sample.h"
 
@@ -1172,8 +1173,9 @@ struct StartArg {
   uint64_t seed;
 };
 
-// Rows of one pass of a batched start (a prompt longer than this, which no
-// configuration reaches, goes alone): about 51 KB of work buffers a row.
+// Rows of one pass of a batched start (a longer prompt goes alone): 51 KB of
+// work buffers a row on int8 stacks, 66 KB on others, at most 0.42 and 0.54 GB
+// in all, kept with the frame for its next start.
 constexpr int kStartRows = 8192;
 // Whether a prompt joins a pass: on the int8 path any does; with f32
 // activations those whose products sum a row in one order whatever the row
@@ -1359,38 +1361,46 @@ extern "C" int q3h_frame_start_batch(q3h_frame *f, int n, const int *streams,
     std::stable_partition(args.begin(), args.end(), [&](const StartArg &a) {
       return start_joins(f->talker, a.rows);
     });
+    const int joined = (int)(std::partition_point(args.begin(), args.end(),
+                                                  [&](const StartArg &a) {
+                                                    return start_joins(f->talker, a.rows);
+                                                  }) -
+                             args.begin());
     std::vector<StartVals> sv(n);
+    std::vector<std::vector<StartArg>> passes;
     std::vector<std::vector<StartPrompt>> prompts;
     std::vector<std::vector<int2>> tiles;
+    auto alone = [&](int i) {
+      const StartArg &a = args[i];
+      start_enqueue(f, a.stream, a.rows, a.trailing_rows, a.seed, sv[i],
+                    [&](float *pre, float *trail, hipStream_t st) {
+                      check_hip(hipMemcpyAsync(pre, a.prefill, sizeof(float) * a.rows * H,
+                                               hipMemcpyHostToDevice, st),
+                                "upload prefill");
+                      if (a.trailing_rows > 0)
+                        check_hip(hipMemcpyAsync(trail, a.trailing,
+                                                 sizeof(float) * a.trailing_rows * H,
+                                                 hipMemcpyHostToDevice, st),
+                                  "upload trailing");
+                    });
+    };
     try {
-      int i = 0, before = -1;  // the first prompt of the pass before
-      while (i < n && start_joins(f->talker, args[i].rows)) {
-        int j = i, M = 0;
-        while (j < n && start_joins(f->talker, args[j].rows) && M + args[j].rows <= kStartRows)
-          M += args[j++].rows;
-        if (j - i == 1) break;  // alone (what is left joins nothing: its own stream)
-        if (before >= 0)  // the pass before still uses the work buffers
-          check_hip(hipStreamSynchronize(f->tctx[args[before].stream]->stream), "start sync");
-        before = i;
+      std::vector<int> counts(joined);
+      for (int i = 0; i < joined; i++) counts[i] = args[i].rows;
+      for (const std::vector<int> &pass : start_passes(counts.data(), joined, kStartRows)) {
+        if (pass.size() == 1) {
+          alone(pass[0]);
+          continue;
+        }
+        if (!passes.empty())  // the pass before still uses the work buffers
+          check_hip(hipStreamSynchronize(f->tctx[passes.back()[0].stream]->stream), "start sync");
+        passes.emplace_back();
         prompts.emplace_back();
         tiles.emplace_back();
-        start_group(f, &args[i], j - i, prompts.back(), tiles.back());
-        i = j;
+        for (int i : pass) passes.back().push_back(args[i]);
+        start_group(f, passes.back().data(), (int)pass.size(), prompts.back(), tiles.back());
       }
-      for (; i < n; i++) {
-        const StartArg &a = args[i];
-        start_enqueue(f, a.stream, a.rows, a.trailing_rows, a.seed, sv[i],
-                      [&](float *pre, float *trail, hipStream_t st) {
-                        check_hip(hipMemcpyAsync(pre, a.prefill, sizeof(float) * a.rows * H,
-                                                 hipMemcpyHostToDevice, st),
-                                  "upload prefill");
-                        if (a.trailing_rows > 0)
-                          check_hip(hipMemcpyAsync(trail, a.trailing,
-                                                   sizeof(float) * a.trailing_rows * H,
-                                                   hipMemcpyHostToDevice, st),
-                                    "upload trailing");
-                      });
-      }
+      for (int i = joined; i < n; i++) alone(i);
     } catch (...) {
       // what is enqueued still reads the host values: let it end before they go
       for (const StartArg &a : args) (void)hipStreamSynchronize(f->tctx[a.stream]->stream);

@@ -192,6 +192,7 @@ def test_frame_start_batch_equals_starts(small, synth, q3h):
 @pytest.mark.parametrize("act_q8, lens, dtype", [
     (0, [70, 16, 130, 65, 64, 1], q3h.Q8_0),         # prompts of 65 rows or more join one pass
     (0, [70, 40, 600, 465], q3h.F32),                # (32-query attention tiles)
+    (0, [5000, 4000, 70, 40, 90], q3h.Q8_0),         # one alone, the shorter ones with the first
     (1, [70, 16, 130, 65, 64, 1], q3h.Q8_0),         # the int8 path: all of them
     (1, [1900, 2001, 1999, 2000, 1500], q3h.Q8_0)])  # more rows than one pass takes
 def test_frame_start_batch_joined_prompts(device, synth, act_q8, lens, dtype):
