@@ -295,8 +295,10 @@ struct q3h_text_proj {
   void *emb = nullptr;  // [text_vocab][text_hidden], BF16 or f32
   q3h::Mat fc1, fc2;    // f32; as split operand tiles only (x3) when split
   // both products over split operands, K in kTextSlices slices (widths that are
-  // multiples of 64 and 512): e and h hold operand tiles, part the slices' sums
-  bool split = false;
+  // multiples of 64 and 512), at most `rows` rows in a pass: e and h hold
+  // operand tiles of that many rows, part the slices' sums
+  bool split = false, beyond = false;  // beyond: a call has had more rows
+  int rows = 0;
   float *part = nullptr;
   float *b1 = nullptr, *b2 = nullptr;
   int cap = 0;               // rows of the work buffers
@@ -310,10 +312,10 @@ struct q3h_text_proj {
 };
 
 namespace q3h {
-// the work buffers of t for n rows (grows, synchronizing t->stream first)
+// the work buffers of t for a call of n rows (grows, synchronizing t->stream first)
 void text_ensure(q3h_text_proj *t, int n);
 // y [n][ldy] = the projection of the n ids at ids_dev (device, each in
-// [0, text_vocab): the caller checks), on stream st; uses t->e and t->h
+// [0, text_vocab): the caller checks), on stream st; uses t's work buffers
 // (text_ensure(t, n) first)
 void text_project_dev(q3h_text_proj *t, const int32_t *ids_dev, int n, float *y, int ldy,
                       hipStream_t st);

@@ -61,7 +61,15 @@ __global__ __launch_bounds__(256) void k_text_rows(const void *__restrict__ emb,
   for (int i = t; i < H; i += 256) yr[i] = b2[i];
 }
 
+// K slices of both products, at every row count: 48 ids 58 us a call (81 as full
+// K on the f32 matrix cores), 520 ids 246 (339), 1100 ids 440 (552), 4000 ids
+// 1490 (1520-1610). Their sums are 64 KB a row of work area, 50 us of allocation: so
+// the area holds 64 rows from the start, a call beyond it runs in passes the
+// first time (520 ids: 0.6 ms, 1.5-2.0 with the allocation) and the area grows at
+// the second such call, up to kTextRows (2100 ids: 891 us in passes of 512 rows,
+// 989 of 256, 807 in one).
 constexpr int kTextSlices = 8;
+constexpr int kTextRows = 1024;
 
 // one workgroup per row: emb[ids[r]] split into operand tiles (TH % 32 == 0)
 template <bool BF16>
@@ -162,31 +170,63 @@ T *upload(const T *src, size_t n, const char *what) {
 }  // namespace
 
 void text_ensure(q3h_text_proj *t, int n) {
-  if (n <= t->cap) return;
-  const int cap = std::max(n, std::max(64, 2 * t->cap));
+  const size_t TH = t->cfg.text_hidden, H = t->cfg.hidden;
+  if (n > t->cap) {
+    const int cap = std::max(n, std::max(64, 2 * t->cap));
+    check_hip(hipStreamSynchronize(t->stream), "text sync");
+    dev_free(t->ids);
+    dev_free(t->y);
+    t->ids = nullptr;
+    t->y = nullptr;
+    if (!t->split) {
+      dev_free(t->e);
+      dev_free(t->h);
+      t->e = t->h = nullptr;
+    }
+    t->cap = 0;
+    t->ids = (int32_t *)dev_alloc(sizeof(int32_t) * cap);
+    t->y = (float *)dev_alloc(sizeof(float) * cap * H);
+    if (!t->split) {
+      t->e = (float *)dev_alloc(sizeof(float) * cap * TH);
+      t->h = (float *)dev_alloc(sizeof(float) * cap * TH);
+    }
+    t->cap = cap;
+  }
+  if (!t->split || n <= t->rows || t->rows == kTextRows) return;
+  if (t->rows > 0 && !t->beyond) {  // in passes of the rows there are, this once
+    t->beyond = true;
+    return;
+  }
+  const int rows = std::min(kTextRows, std::max(n, std::max(64, 2 * t->rows)));
   check_hip(hipStreamSynchronize(t->stream), "text sync");
-  dev_free(t->ids);
   dev_free(t->e);
   dev_free(t->h);
-  dev_free(t->y);
   dev_free(t->part);
-  t->ids = nullptr;
-  t->e = t->h = t->y = t->part = nullptr;
-  t->cap = 0;
-  const size_t TH = t->cfg.text_hidden, H = t->cfg.hidden;
-  t->ids = (int32_t *)dev_alloc(sizeof(int32_t) * cap);
-  t->e = (float *)dev_alloc(t->split ? x3_bytes(cap, TH) : sizeof(float) * cap * TH);
-  t->h = (float *)dev_alloc(t->split ? x3_bytes(cap, TH) : sizeof(float) * cap * TH);
-  if (t->split) t->part = (float *)dev_alloc(sizeof(float) * kTextSlices * cap * std::max(TH, H));
-  t->y = (float *)dev_alloc(sizeof(float) * cap * H);
-  t->cap = cap;
+  t->e = t->h = t->part = nullptr;
+  t->rows = 0;
+  t->e = (float *)dev_alloc(x3_bytes(rows, TH));
+  t->h = (float *)dev_alloc(x3_bytes(rows, TH));
+  t->part = (float *)dev_alloc(sizeof(float) * kTextSlices * rows * std::max(TH, H));
+  t->rows = rows;
+  t->beyond = false;
 }
 
 void text_project_dev(q3h_text_proj *t, const int32_t *ids_dev, int n, float *y, int ldy,
                       hipStream_t st) {
   const q3h_text_config &c = t->cfg;
   const int TH = c.text_hidden, H = c.hidden;
+  if (t->split && n > t->rows) {  // equal passes (a row's result is that of any other row count)
+    const int passes = (n + t->rows - 1) / t->rows;
+    for (int p = 0, r = 0; p < passes; p++) {
+      const int rows = (n - r) / (passes - p);
+      text_project_dev(t, ids_dev + r, rows, y + (size_t)r * ldy, ldy, st);
+      r += rows;
+    }
+    return;
+  }
   if (t->split) {
+    // (the hidden rows in the memory of the embedding rows: 58.7 against 57.6 us at
+    // 48 ids)
     uint16_t *e = reinterpret_cast<uint16_t *>(t->e), *h = reinterpret_cast<uint16_t *>(t->h);
     if (c.emb_dtype == Q3H_BF16)
       hipLaunchKernelGGL(k_text_rows_x3<true>, dim3(n), dim3(256), 0, st, t->emb, ids_dev, TH, e);
@@ -253,7 +293,7 @@ extern "C" int q3h_text_create(q3h_device *dev, const q3h_text_config *cfg, cons
       split_weights(t->fc1, t->stream);
       split_weights(t->fc2, t->stream);
     }
-    text_ensure(t, 1);  // the first call's workspace: 0.3 ms of allocations
+    text_ensure(t, 1);  // the work area of the first calls: 0.3 ms of allocations
     t->bytes = (int64_t)(es * c.text_vocab * TH + (t->split ? 6 : 4) * (TH * TH + H * TH) +
                          4 * (TH + H));
     dev->bytes += t->bytes;

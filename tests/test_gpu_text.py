@@ -48,6 +48,24 @@ def test_text_project_parity(proj, tables, n):
     assert rel(y[n // 2], ref[0]) < 1e-4
 
 
+def test_text_project_passes(device, tables):
+    """Calls beyond the work area run in passes the first time and in one, or in
+    passes of its largest size, once it has grown: the same bits, a row's result
+    being that of any row count."""
+    p = q3h.TextProj(device, *tables)
+    rng = np.random.default_rng(8)
+    try:
+        for n in (65, 200, 1030, 2100):
+            ids = rng.integers(0, TV, n).astype(np.int32)
+            first = p.project(ids)
+            assert np.array_equal(first, p.project(ids)), n
+            assert np.array_equal(first[n // 2:], p.project(ids[n // 2:])), n
+        ref = _oracle(tables, ids[-70:])
+        assert rel(first[-70:], ref) < 2e-5
+    finally:
+        p.destroy()
+
+
 @pytest.mark.parametrize("hidden", [32, 192], ids=["f32_products", "split_products"])
 def test_text_project_other_widths(device, hidden):
     """Widths on both sides of the split products' rule (hidden a multiple of
