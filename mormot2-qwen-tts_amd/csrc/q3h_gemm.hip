@@ -14,7 +14,7 @@
 // Operand layouts (v_mfma_i32_16x16x32_i8, wave64): lane l holds 8 int8 of
 // row l % 16 of A and of column l % 16 of B, k = 8 * (l / 16) .. + 7; the
 // result C[4 * (l / 16) + r][l % 16], r < 4, lands in lane l. A is 16 weight
-// rows, B 16 activation rows, both stored in operand order (wtile_offset: the
+// rows, B 16 activation rows, both stored in operand order (launch_tile_q8: the
 // matrices of an act_q8 stack are rewritten so at load; qtile_offset: written
 // so by the quantizers), so one coalesced 1 KB load gives the operands of two
 // blocks.
@@ -604,7 +604,7 @@ void gemm_by_k(const Mat &W, const QAct &xa, int M, int epi, float *y, int ldy, 
     gemm_launch<TM, 2>(W, xa, M, epi, y, ldy, st);
 }
 
-// Q8_0 quants [N][K] row-major to operand order (wtile_offset), 16 bytes (a
+// Q8_0 quants [N][K] row-major to operand order (launch_tile_q8), 16 bytes (a
 // lane's operands of a pair of blocks) per thread
 __global__ __launch_bounds__(256) void k_tile_q8(const int8_t *__restrict__ src, int N, int K,
                                                  int8_t *__restrict__ dst) {

@@ -12,7 +12,7 @@ namespace q3h {
 // same allocation, by the fp16 scales [N][K/32] (d == q + N*K; structure of
 // arrays, so a wave reads 1 KB of quants per instruction), or f32 [N][K]. The
 // quants of act_q8 stacks are in the operand order of the int8 products
-// instead (wtile_offset).
+// instead (launch_tile_q8).
 struct Mat {
   int N = 0, K = 0;
   int8_t *q = nullptr;
@@ -108,15 +108,10 @@ __host__ __device__ inline size_t qscale_offset(int m, int b, int nb) {
   return ((size_t)(m >> 4) * (nb >> 2) + (b >> 2)) * 64 + (m & 15) * 4 + (b & 3);
 }
 size_t qact_bytes(int M, int K);
-// The quants of a matrix of an act_q8 stack, in the same operand order: the
-// tile of rows 16 i .. + 15 and block pair p is the 1 KB at (i K / 64 + p) KB,
-// lane g * 16 + n % 16 its bytes 8g .. + 7 of both blocks (K % 64 == 0,
-// N % 16 == 0; the scales stay row-major at q + N K)
-__host__ __device__ inline size_t wtile_offset(int n, int k, int K) {
-  return (((size_t)(n >> 4) * (K >> 6) + (k >> 6)) * 64 + ((k & 31) >> 3) * 16 + (n & 15)) * 16 +
-         ((k >> 5) & 1) * 8 + (k & 7);
-}
-// row-major quants [N][K] at src to that order at dst
+// The quants of a matrix of an act_q8 stack, in the same operand order: row-major
+// quants [N][K] at src to dst, where the tile of rows 16 i .. + 15 and block pair
+// p is the 1 KB at (i K / 64 + p) KB, lane g * 16 + n % 16 its bytes 8g .. + 7 of
+// both blocks (K % 64 == 0, N % 16 == 0; the scales stay row-major at q + N K)
 void launch_tile_q8(const int8_t *src, int N, int K, int8_t *dst, hipStream_t st);
 
 void launch_gemv(const GemvArgs &a, int epi, bool q8, hipStream_t st);
