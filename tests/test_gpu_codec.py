@@ -127,6 +127,40 @@ def test_codec_one_term_products(device, frames):
     assert top <= 14 * 2.0 ** -24 and rms < 1e-7 and mean < 5e-8, (mean, rms, top)
 
 
+def test_codec_large_snake_arguments(device):
+    """SnakeBeta of arguments up to 1e6, on both sides of the change to sinf
+    (4e5) and next to multiples of pi: the second SnakeBeta of block 0's first
+    residual unit sees a bias V alone, z = V + ib sin(V)^2 with ib = 3.3e8, and
+    its product takes 1e-9 z of one channel on, which reaches the samples through
+    products by 1. The samples 1e-9 V + 0.33 sin(V)^2 within 1e-6 (about 12
+    roundings of 2^-24 each)."""
+    rng = np.random.default_rng(4)
+    w = _one_term_weights(rng)
+    for i, b in enumerate(w["block"]):
+        b["up_w"] = np.zeros_like(b["up_w"])
+        if i == 0:
+            continue
+        cin, out, k = b["up_w"].shape  # output channel o, phase j: input channel k o / 2 + j
+        for j in range(k // 2):
+            b["up_w"][(np.arange(out) * (k // 2) + j) % cin, np.arange(out), j] = 1
+    r = w["block"][0]["res"][0]
+    C = r["c1_b"].size
+    v = np.exp(rng.uniform(0, np.log(1e6), C))
+    v[::3] = np.arange(1, v[::3].size + 1) * 313 * np.pi  # to 2.5e5
+    v = np.where(rng.random(C) < 0.5, -v, v).astype(np.float32)
+    r["c1_b"] = v
+    r["a2_alpha"], r["a2_beta"] = np.zeros_like(r["a2_alpha"]), np.full_like(r["a2_beta"], -20)
+    r["c2_w"] = np.zeros_like(r["c2_w"])
+    r["c2_w"][np.arange(C), np.arange(C), 0] = 1e-9
+    y = _gpu(device, w, np.zeros((1, 1024), np.float32), [1])
+    ref = codec_torch.back(w, np.zeros((1, 1024), np.float32))
+    ib = 1 / (np.exp(-20) + 1e-9)
+    seen = np.unique(ref.round(9)).size
+    print(f"{seen} values, peak {ref.max():.3f}, max error {abs(y - ref).max():.2e}")
+    assert seen >= 50 and 0.1 < ref.max() <= 1.1e-9 * ib
+    assert abs(y - ref).max() <= 1e-6 * ref.max()
+
+
 def test_codec_reset_and_errors(device, weights):
     x = synth.prompt(5, 2)
     c = q3h.Codec(device, weights, max_frames=4)

@@ -242,6 +242,27 @@ def test_int8_prompt_attention_tiles(device, q3h, q3o, synth, heads, kvh, kv16):
         o.destroy()
 
 
+def test_int8_many_contexts_head(small8, q3h, q3o, synth):
+    """250 contexts, one row each, with the 3072-row head: 16 activation tiles,
+    from which the head's product takes a wave per 64 weight rows over the whole K
+    (k_gemm_i8r), the last tile 10 rows."""
+    m, n = small8, 250
+    ctxs = [q3h.Context(m.ts, 4) for _ in range(n)]
+    octx = q3o.Ctx(m.ot, 4)
+    try:
+        x = synth.prompt(230, n)
+        lg, normed = q3h.forward_batch(ctxs, x, heads=[0] * n)
+        for i in range(n):
+            octx.reset()
+            ost = octx.forward(x[i:i + 1])
+            assert np.array_equal(normed[i], ost), i
+            assert np.array_equal(lg[i], m.ot.head(m.th, ost)), i
+    finally:
+        for c in ctxs:
+            c.destroy()
+        octx.destroy()
+
+
 @pytest.fixture(scope="module")
 def small8h(device):
     """The int8 path with half-float K/V caches (the reference's KvF16,

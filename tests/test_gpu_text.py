@@ -69,7 +69,10 @@ def test_text_project_passes(device, tables):
 @pytest.mark.parametrize("hidden", [32, 192], ids=["f32_products", "split_products"])
 def test_text_project_other_widths(device, hidden):
     """Widths on both sides of the split products' rule (hidden a multiple of
-    64): 1024 text columns, 7 and 70 rows."""
+    64): 1024 text columns, 7 and 70 rows. Two products of 1024 terms, whose sums
+    are rounded at every step on the oracle's side and at every chunk of 32 (4 on
+    the f32 matrix cores) here: 2.3e-7 to 5.7e-7 of the largest result measured,
+    1e-6 allowed; a lost part product is 7.6e-6."""
     rng = np.random.default_rng(hidden)
     emb = (rng.standard_normal((64, 1024)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
     tables = (emb, rng.standard_normal((1024, 1024), np.float32) * np.float32(0.02),
@@ -80,7 +83,9 @@ def test_text_project_other_widths(device, hidden):
     try:
         for n in (7, 70):
             ids = rng.integers(0, 64, n).astype(np.int32)
-            assert rel(p.project(ids), _oracle(tables, ids)) < 2e-5, n
+            worst = rel(p.project(ids), _oracle(tables, ids))
+            print(f"{n} rows: relative error {worst:.2e}", flush=True)
+            assert worst < 1e-6, n
     finally:
         p.destroy()
 
