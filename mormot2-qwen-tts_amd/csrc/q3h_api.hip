@@ -167,7 +167,7 @@ void linear(const q3h_stack *s, Work &w, const Mat &W, const float *x, int ldx, 
       ldx = W.K;
     }
     if (M > kManyRows && epi == EPI_STORE && W.K == c.hidden && gemm_x3_supported(W, 1)) {
-      launch_x3_rows(x, ldx, M, W.K, w.x3n, st);
+      launch_x3_rows(x, ldx, M, W.K, w.x3n, W.q != nullptr, st);
       launch_gemm_x3(W, w.x3n, M, y, ldy, st);
       return;
     }
@@ -290,8 +290,9 @@ static void run_layers_x3(const q3h_stack *s, Work &w, int M, int positions, boo
   const int H = c.hidden, hd = c.head_dim, NQ = c.heads * hd, NKV = c.kv_heads * hd;
   const int ldq = NQ + 2 * NKV;
   const bool kv16 = c.kv_f16 != 0;
+  const bool cut = c.dtype == Q3H_Q8_0;
   const float eps = c.rms_eps;
-  launch_resid_norm(w.h, nullptr, M, H, s->layers[0].in_norm, eps, nullptr, 0, st, w.x3n);
+  launch_resid_norm(w.h, nullptr, M, H, s->layers[0].in_norm, eps, nullptr, 0, st, w.x3n, cut);
   for (int l = 0; l < c.layers; l++) {
     const Layer &L = s->layers[l];
     launch_gemm_x3(L.qkv, w.x3n, M, w.qkv, ldq, st);
@@ -314,17 +315,18 @@ static void run_layers_x3(const q3h_stack *s, Work &w, int M, int positions, boo
     at.tile_rows = io.tile_rows;
     if (!fused && (io.tiles || io.single_context)) {
       at.out3 = w.x3a;
+      at.cut3 = cut;
       launch_attn_prefill(at, M, kv16, st);
     } else {
       launch_attn(at, M, positions, fused, kv16, st);
-      launch_x3_rows(w.att, NQ, M, NQ, w.x3a, st);
+      launch_x3_rows(w.att, NQ, M, NQ, w.x3a, cut, st);
     }
     const int so = launch_gemm_x3_part(L.o, w.x3a, M, w.gpart, st);
-    launch_resid_norm(w.h, w.gpart, M, H, L.post_norm, eps, nullptr, so, st, w.x3n);
+    launch_resid_norm(w.h, w.gpart, M, H, L.post_norm, eps, nullptr, so, st, w.x3n, cut);
     launch_gemm_x3_swiglu(L.gu, w.x3n, M, w.x3a, st);
     const int sd = launch_gemm_x3_part(L.down, w.x3a, M, w.gpart, st);
     const float *next = l + 1 < c.layers ? s->layers[l + 1].in_norm : nullptr;
-    launch_resid_norm(w.h, w.gpart, M, H, next, eps, nullptr, sd, st, w.x3n);
+    launch_resid_norm(w.h, w.gpart, M, H, next, eps, nullptr, sd, st, w.x3n, cut);
     probe_layer(io, w, l, M, H, st);
   }
 }

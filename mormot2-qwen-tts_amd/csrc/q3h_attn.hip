@@ -989,7 +989,8 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_x3(const RowDesc *__res
                                                             int layer, int kvh, int M,
                                                             float *__restrict__ outp,
                                                             const int2 *__restrict__ tiles,
-                                                            uint16_t *__restrict__ out3) {
+                                                            uint16_t *__restrict__ out3,
+                                                            bool cut3) {
   __shared__ float ms[QT][4][16], ls[QT][4][16];
   __shared__ float os[4][8][4][64];
   __shared__ u32x4 qs[QT][4][3][64];
@@ -1168,7 +1169,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_x3(const RowDesc *__res
         v[e] = den > 0.f ? num / den : 0.f;
       }
       if (out3) {
-        x3_store8(out3, q0 + row, h * HD + k0, heads * HD, v);
+        x3_store8(out3, q0 + row, h * HD + k0, heads * HD, v, cut3);
       } else {
         float *op = outp + (size_t)(q0 + row) * (heads * HD) + h * HD + k0;
         *reinterpret_cast<float4 *>(op) = make_float4(v[0], v[1], v[2], v[3]);
@@ -1370,10 +1371,10 @@ void launch_attn_prefill(const AttnArgs &a, int M, bool kv16, hipStream_t st) {
   do {                                                                                          \
     if (rows == 32)                                                                             \
       hipLaunchKernelGGL((k_attn_prefill_x3<KV, G, 2>), grid, block, 0, st, a.rd, a.qkv, a.ldq, \
-                         a.layer, a.kvh, M, a.out, a.tiles, a.out3);                            \
+                         a.layer, a.kvh, M, a.out, a.tiles, a.out3, a.cut3);                    \
     else                                                                                        \
       hipLaunchKernelGGL((k_attn_prefill_x3<KV, G, 1>), grid, block, 0, st, a.rd, a.qkv, a.ldq, \
-                         a.layer, a.kvh, M, a.out, a.tiles, a.out3);                            \
+                         a.layer, a.kvh, M, a.out, a.tiles, a.out3, a.cut3);                    \
   } while (0)
   if (kv16) {
     if (grp == 1) Q3H_P(_Float16, 1);

@@ -591,7 +591,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_x3(const void *__restrict__ wp,
       const float4 p0 = *reinterpret_cast<const float4 *>(&o[row * G::kOutLd + 8 * j]);
       const float4 p1 = *reinterpret_cast<const float4 *>(&o[row * G::kOutLd + 8 * j + 4]);
       const float v[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-      if (m < M) x3_store8(y3, m, n0 / 2 + 8 * j, N / 2, v);
+      if (m < M) x3_store8(y3, m, n0 / 2 + 8 * j, N / 2, v, Q8);
     }
   } else {
     float *yo = y + (EPI == EPI_PART ? (size_t)blockIdx.z * M * ldy : 0) + n0 + r;
@@ -609,12 +609,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_x3(const void *__restrict__ wp,
 
 // rows x [M][ldx] split into operand tiles, a thread per 4 columns
 __global__ __launch_bounds__(256) void k_x3_rows(const float *__restrict__ x, int ldx, int M, int K,
-                                                 uint16_t *__restrict__ o) {
+                                                 uint16_t *__restrict__ o, bool cut) {
   const int i = blockIdx.x * 256 + threadIdx.x, m = i / (K / 4), k = 4 * (i - m * (K / 4));
   if (m >= M) return;
   const float4 v = ld4(x + (size_t)m * ldx + k);
   const float v4[4] = {v.x, v.y, v.z, v.w};
-  x3_store4(o, m, k, K, v4);
+  x3_store4(o, m, k, K, v4, cut);
 }
 
 // h[m] += slices 0 .. S-1 of part [S][M][K], added in slice order (S == 0: h
@@ -631,7 +631,7 @@ __global__ __launch_bounds__(256) void k_resid_norm(float *__restrict__ h,
                                                     const float *__restrict__ part, int M,
                                                     int K, const float *__restrict__ w,
                                                     float eps, float *__restrict__ xn,
-                                                    uint16_t *__restrict__ x3) {
+                                                    uint16_t *__restrict__ x3, bool cut) {
   constexpr int NR = kResidNormRounds;
   __shared__ double red[4];
   // operand tiles: the 16 rows of a tile on one XCD (workgroups go to the XCDs
@@ -676,7 +676,7 @@ __global__ __launch_bounds__(256) void k_resid_norm(float *__restrict__ h,
     const float o[4] = {wv[r].x * (hv[r].x * inv), wv[r].y * (hv[r].y * inv),
                         wv[r].z * (hv[r].z * inv), wv[r].w * (hv[r].w * inv)};
     if (x3)
-      x3_store4(x3, m, k, K, o);
+      x3_store4(x3, m, k, K, o, cut);
     else
       *reinterpret_cast<float4 *>(xn + (size_t)m * K + k) = make_float4(o[0], o[1], o[2], o[3]);
   }
@@ -882,10 +882,11 @@ int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hi
   return ks;
 }
 
-void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, hipStream_t st) {
+void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, bool cut,
+                    hipStream_t st) {
   const size_t n = (size_t)M * (K / 4);
   hipLaunchKernelGGL(k_x3_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, ldx, M, K,
-                     o);
+                     o, cut);
 }
 
 bool gemm_f32_supported(int N, int K) {
@@ -930,11 +931,12 @@ int launch_gemm_f32_part(const Mat &W, const float *x, int ldx, int M, float *pa
 }
 
 void launch_resid_norm(float *h, const float *part, int M, int K, const float *norm_w,
-                       float eps, float *xn, int slices, hipStream_t st, uint16_t *x3) {
+                       float eps, float *xn, int slices, hipStream_t st, uint16_t *x3,
+                       bool cut) {
   require(K <= 1024 * kResidNormRounds && K % 4 == 0, Q3H_E_ARG, "launch_resid_norm: K above 4096");
 #define Q3H_RN(S)                                                                               \
   hipLaunchKernelGGL(k_resid_norm<S>, dim3(x3 ? (M + 127) / 128 * 128 : M), dim3(256), 0, st, h, \
-                     part, M, K, norm_w, eps, xn, x3)
+                     part, M, K, norm_w, eps, xn, x3, cut)
   switch (slices) {
     case 0: Q3H_RN(0); break;
     case 1: Q3H_RN(1); break;

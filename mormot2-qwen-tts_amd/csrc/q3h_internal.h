@@ -155,7 +155,8 @@ void launch_gemm_x3_swiglu(const Mat &W, const uint16_t *x3, int M, uint16_t *y3
 int launch_gemm_x3_part(const Mat &W, const uint16_t *x3, int M, float *part, hipStream_t st,
                         int ks = kF32Slices);
 // rows x [M][ldx] split into operand tiles
-void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, hipStream_t st);
+// (cut: for Q8_0 weights, x3_split)
+void launch_x3_rows(const float *x, int ldx, int M, int K, uint16_t *o, bool cut, hipStream_t st);
 constexpr int kGemvRows = 4;
 void launch_gemm_f32(const Mat &W, const float *x, int ldx, int M, int epi, float *y, int ldy,
                      hipStream_t st);
@@ -176,9 +177,10 @@ int launch_gemm_f32_part(const Mat &W, const float *x, int ldx, int M, float *pa
 int q8x_slices(const Mat &W, int M);
 // h [M][K] += the `slices` slices of part (0-4, 6, 8 or 12), in slice order; then,
 // when norm_w != nullptr, RMSNorm(h) with norm_w (double sum of squares) to xn
-// [M][K], or to the operand tiles x3 when that is non-null
+// [M][K], or to the operand tiles x3 when that is non-null (cut: x3_split)
 void launch_resid_norm(float *h, const float *part, int M, int K, const float *norm_w,
-                       float eps, float *xn, int slices, hipStream_t st, uint16_t *x3 = nullptr);
+                       float eps, float *xn, int slices, hipStream_t st, uint16_t *x3 = nullptr,
+                       bool cut = false);
 // the int8 path (q3h_gemm.hip): shapes it takes (N % 16 == 0, K % 256 == 0,
 // K <= 3072)
 bool gemm_i8_supported(int N, int K);
@@ -243,7 +245,8 @@ struct AttnArgs {
   const float *qkn;  // [q_norm | k_norm | eps] of the layer
   const float2 *rope_cs;
   float *out;    // [M][heads * head_dim]
-  uint16_t *out3;  // launch_attn_prefill: the outputs as operand tiles instead, when non-null
+  uint16_t *out3;  // launch_attn_prefill: the outputs as operand tiles instead, when non-null,
+  bool cut3;       // their parts cut off (x3_split)
   float *part;   // [M][heads][attn_splits slots][head_dim + 2]
   int layers;    // > layer + 1: a decode launch also loads layer + 1's cache rows ahead
   // launch_attn_prefill and launch_attn_x_prompt over several contexts' rows:

@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256) void k_text_rows_x3(const void *__restrict__ e
       const float4 a = s[0], b = s[1];
       v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
     }
-    x3_store8(e, r, k, TH, v);
+    x3_store8(e, r, k, TH, v, false);
   }
 }
 
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void k_text_mid(const float *__restrict__ part
   text_sum4(part, b1, M, TH, m, k, v);
 #pragma unroll
   for (int e = 0; e < 4; e++) v[e] = silu_clamp_f(v[e]);
-  x3_store4(h, m, k, TH, v);
+  x3_store4(h, m, k, TH, v, false);
 }
 
 // y = b2 + sum
