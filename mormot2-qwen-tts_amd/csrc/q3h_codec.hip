@@ -569,7 +569,7 @@ void conv_launch(q3h_codec *c, const DConv &d, const ConvArgs &a, int T, int epi
 // or 32-row tiles walked whole where they fill the chip, a workgroup per slice
 // otherwise.
 // (The kernels are built for the decoder's layers only: the front layers, f32
-// tiles, have 4 slices at one tap, more than 4 otherwise; the blocks' transposed
+// tiles, have 4 and 16 slices at one tap, 6 to 16 otherwise; the blocks' transposed
 // convolutions of two taps have 4, 2 and 1, their dilated convolutions 12, 6, 3
 // and 3, and their pointwise ones 3, 2, 1 and 1.)
 template <int WN, int TAPS, bool WF32, int SU>
