@@ -105,10 +105,11 @@ __device__ __forceinline__ void split3(float x, uint32_t &h, uint32_t &m, uint32
 // so the part products below hi lo that a six-part product leaves out (mid lo,
 // lo mid, lo lo) weigh at most 2^-24 of it and cancel on average. Cut off
 // instead of rounded (split3) they reach 2^-21 and all have the product's sign:
-// a product of one term 9.2e-8 off (RMS) instead of 3.6e-8. As many
+// a result of two one-term products 9.2e-8 off (RMS) instead of 3.6e-8. As many
 // instructions (the pair conversion of gfx950 packs as it rounds) and one more
 // per value: hi of a value within half a bf16 step of the largest float would
-// round to infinity, so it is taken of the value limited to the largest bf16.
+// be infinite, so it is taken of the value limited to the largest bf16. (Parts
+// below the smallest normal number, of values under 2^-102, may be lost.)
 __device__ __forceinline__ void split3_rn(float a, float b, uint32_t &h, uint32_t &m,
                                           uint32_t &l) {
   typedef float f2 __attribute__((ext_vector_type(2)));

@@ -181,8 +181,8 @@ def test_batch_replays_follow_the_contexts(q8model, q3h, synth):
 def test_batch_graph_keys(device, q3h, q3o, synth):
     """Batched forwards of 15 heads at 3 sizes in turn (45 graphs of the leading
     context, a code predictor's use): the first use of a key is launched, the
-    second captured, all later ones replayed, none captured twice, so a third
-    round costs what one key repeated does (1.5 times allowed; a capture costs
+    second captured, all later ones replayed, none captured twice, so the third
+    turn costs what one key repeated does (1.5 times allowed; a capture costs
     several calls). Then 90 keys used twice each, more than are kept, between
     single-row forwards of the leading context: the same results bit for bit as
     at their first use."""
