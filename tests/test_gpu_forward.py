@@ -182,8 +182,8 @@ def test_batch_graph_keys(device, q3h, q3o, synth):
     """Batched forwards of 15 heads at 3 sizes in turn (45 graphs of the leading
     context, a code predictor's use): the first use of a key is launched, the
     second captured, all later ones replayed, none captured twice, so the third
-    turn costs what one key repeated does (1.5 times allowed; a capture costs
-    several calls). Then 90 keys used twice each, more than are kept, between
+    turn costs what one key repeated does (144 against 139 us, 1.3 times allowed;
+    a capture at every call makes 220 us of it). Then 90 keys used twice each, more than are kept, between
     single-row forwards of the leading context: the same results bit for bit as
     at their first use."""
     dims = dict(synth.TALKER, layers=2)
@@ -213,7 +213,7 @@ def test_batch_graph_keys(device, q3h, q3o, synth):
         turn = np.median([r[0] for r in rounds])
         one = np.median([call(n, 3)[0] for n in (6, 9, 12) for _ in range(15)])
         print(f"45 keys in turn {turn * 1e6:.0f} us a call, one key {one * 1e6:.0f} us")
-        assert turn < 1.5 * one
+        assert turn < 1.3 * one
         ctxs[0].reset()
         single = ctxs[0].forward(x[0], head=0)[0]
         for n in (2, 3, 4, 5, 7, 8):
