@@ -52,9 +52,9 @@ __host__ __device__ __attribute__((noinline)) inline float sin_far(float x) { re
 // two floats left out) keeps that so where x is next to a multiple of pi. sin r,
 // |r| <= pi / 2, by its Taylor series to r^13 (truncation < 7e-10) in Horner
 // form. sin x within 3 units of 2^-24, relative (two roundings of r, one of the
-// last step); beyond 4e5 by sinf. 17
-// instructions without a branch taken, where sinf's general reduction, inlined
-// per output, made a decoder epilogue of 32 values 9000 lines long.
+// last step); beyond 4e5 by sinf. 17 instructions without a branch taken, where
+// sinf's general reduction, inlined per output, made a decoder epilogue of 32
+// values 9000 lines long.
 __host__ __device__ __forceinline__ float sin_squared(float x) {
   float s;
   if (fabsf(x) < 4e5f) {
